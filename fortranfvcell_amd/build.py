@@ -39,7 +39,7 @@ def _run(cmd, cwd=None):
 
 # translation units: the host code and small kernels, then one per family of
 # solver kernels (explicitly instantiated there, see csrc/fvc_instances.h)
-HIP_UNITS = ("fvcell", "k_cg", "k_bicg", "k_gmres", "k_mixed", "k_batch")
+HIP_UNITS = ("fvcell", "k_cg", "k_bicg", "k_gmres", "k_mixed", "k_batch", "k_resident")
 
 
 def build_hip() -> str:

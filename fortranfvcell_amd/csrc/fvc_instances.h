@@ -9,12 +9,16 @@
 #include "fvc_mixed_krylov.h"
 #include "fvc_batch.h"
 #include "fvc_gmres_lag.h"
+#include "fvc_resident.h"
 
 // Device formats (Fmt): every format for the FP64 solvers, ELLPACK and CSRD
 // for mixed precision and for batches.
 #define FVCI_FORMATS_ALL(X, P) X(P, 0) X(P, 1) X(P, 2) X(P, 3) X(P, 4) X(P, 5) X(P, 6)
 #define FVCI_FORMATS_MIXED(X, P) X(P, 0) X(P, 1) X(P, 2) X(P, 3)
 #define FVCI_FORMATS_BATCH(X, P) X(P, 0) X(P, 1) X(P, 2) X(P, 3)
+
+// On-chip solves: ELLPACK widths 4 and 3, CSRD.
+#define FVCI_FORMATS_RES(X, P) X(P, 0) X(P, 1) X(P, 3)
 
 #define FVCI_CG(P, F)                                      \
   P __global__ void fvc::cg1_persistent<F>(fvc::Cg1Args); \
@@ -48,6 +52,12 @@
   P __global__ void fvc::pcg_batch_persistent<F>(fvc::BatchArgs);   \
   P __global__ void fvc::mixed_batch_persistent<F>(fvc::BatchArgs); \
   P __global__ void fvc::batch_scale_kernel<F>(fvc::BatchArgs, int, const int *, const int *);
+#define FVCI_RES_R(P, F, R)                                      \
+  P __global__ void fvc::resident_kernel<F, R, 1>(fvc::ResArgs); \
+  P __global__ void fvc::resident_kernel<F, R, 2>(fvc::ResArgs);
+#define FVCI_RES(P, F)                                            \
+  P __global__ void fvc::resident_prep_kernel<F>(fvc::ResPrepArgs); \
+  FVCI_RES_R(P, F, 1) FVCI_RES_R(P, F, 2) FVCI_RES_R(P, F, 4) FVCI_RES_R(P, F, 8)
 #define FVCI_COLOFF(P, W) P __global__ void fvc::col_offsets_kernel<W>(int, const int *, const float *, short *, int *);
 
 // In the host translation unit: declarations only.
@@ -57,6 +67,7 @@ FVCI_FORMATS_ALL(FVCI_BICG, extern template)
 FVCI_FORMATS_ALL(FVCI_GMRES, extern template)
 FVCI_FORMATS_MIXED(FVCI_MIXED, extern template)
 FVCI_FORMATS_BATCH(FVCI_BATCH, extern template)
+FVCI_FORMATS_RES(FVCI_RES, extern template)
 FVCI_COLOFF(extern template, 3)
 FVCI_COLOFF(extern template, 4)
 #endif

@@ -1,0 +1,719 @@
+// fvc_resident.h -- PCG and BiCGSTAB with the whole system held on chip.
+//
+// One launch solves the system: every block loads its rows' matrix entries
+// once into registers and keeps its rows of every Krylov vector there too
+// (256 CUs hold 128 MB of registers; a row of a 4-neighbour system with its
+// six vectors takes about 100 bytes), so that an iteration reads nothing from
+// HBM.  What an iteration waits for is the exchange between blocks, once per
+// grid reduction:
+//   * the SpMV reads its operand from an LDS window of the block's own rows
+//     and of the halo rows its columns reach.  A halo row's operand is not
+//     sent: its r, s, p ... follow the same recurrences as the owner's, on
+//     the same values, so only the result of the previous SpMV at that row
+//     has to arrive, and it travels together with the reduction;
+//   * a block's partial sums go to all blocks, and every block adds all of
+//     them in the same order and runs the scalar recurrence itself.
+// Both travel as 8-byte words that carry half a double and the number of the
+// exchange, stored and loaded at agent scope (past the caches that are not
+// coherent between XCDs): a reader polls the data itself, so an exchange is
+// one store and one load away, with no fence, no flag and no cache
+// write-back.  Two buffers alternate; a block can run at most one exchange
+// ahead of any other (it needs every block's partial sums), so a word is
+// never overwritten before it was read.
+//
+// Measured on MI355X (us per exchange, 512 threads a block, three sums):
+// 3.3 at 8 blocks with 64 halo rows each side, 3.7 at 64 blocks, 4.3 at 256
+// with 64..256 halo rows a side, 8.0 at 256 with 1,024; a launch per phase
+// costs 9 us at 4,096 rows and 26-30 us at a million.  The halo volume is
+// what makes the difference at 256 blocks, so rows are dealt in tiles of the
+// mesh where the columns show one (ResPlan), else in contiguous strips.
+#pragma once
+#include <limits.h>
+#include <stddef.h>
+
+#include "fvc_krylov.h"
+#include "fvc_resplan.h"
+
+namespace fvc {
+
+constexpr unsigned kResSpin = 1u << 20;   // polls of a bounded wait (about two seconds)
+
+typedef unsigned long long res_word;
+
+// KState::pad6 after a launch: solved, or the system does not fit this scheme
+// (solve it another way).  Anything else, or KState::next set: a wait expired.
+constexpr int kResSolved = 1, kResDeclined = 2;
+
+// ------------------------------------------------------------------- prep --
+
+struct ResPrepArgs {
+  Mat A;
+  ResPlan *plan;      // zeroed
+  res_word *part, *rows;   // cleared here: kResPartWords and 4 neq words
+  int rmax, bmax, hmax;   // rows per block, blocks and halo entries at most
+};
+
+// The columns of row i that count: off-diagonal entries other than
+// ELLPACK's padding (column 1 with value 0).
+template <int F, class Fn>
+__device__ __forceinline__ void res_columns(const Mat &A, int i, Fn &&fn) {
+  if constexpr (F == F_CSRD) {
+    for (int k = A.ia[i] - 1; k < A.ia[i + 1] - 1; ++k) fn(A.ja[k] - 1);
+  } else {
+    constexpr int w = F == F_ELL3 ? 3 : 4;
+#pragma unroll
+    for (int k = 0; k < w; ++k) {
+      const int j = A.ja[(size_t)w * i + k] - 1;
+      if (j != 0 || A.av[(size_t)w * i + k] != 0.0) fn(j);
+    }
+  }
+}
+
+// Clears the exchange words, finds the largest |column - row|, and (its last
+// block) decides how the rows are dealt.  One pass over the columns.
+template <int F>
+__global__ __launch_bounds__(256) void resident_prep_kernel(ResPrepArgs a) {
+  __shared__ int s_h, s_last, s_best, s_hx[2];
+  const int n = a.A.neq, step = (int)(gridDim.x * blockDim.x);
+  if (threadIdx.x == 0) s_h = 0;
+  __syncthreads();
+  const int first = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  for (size_t k = first; k < (size_t)4 * n; k += (size_t)step) a.rows[k] = 0ull;
+  for (int k = first; k < kResPartWords; k += step) a.part[k] = 0ull;
+  int h = 0;
+  for (long i = first; i < n; i += step) {
+    res_columns<F>(a.A, (int)i, [&](int j) { h = max(h, abs(j - (int)i)); });
+    if (F == F_CSRD && a.A.ia[i + 1] - a.A.ia[i] > 4) h = n;   // longer rows do not fit the registers
+  }
+  atomicMax(&s_h, h);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    atomicMax(&a.plan->H, s_h);
+    fence_release();
+    s_last = __hip_atomic_fetch_add(&a.plan->ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 ==
+             (int)gridDim.x;
+    fence_acquire();
+    s_hx[0] = s_hx[1] = 0;
+    s_best = INT_MAX;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  const int H = __hip_atomic_load(&a.plan->H, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (H >= n) return;   // a row too long, or nothing to gain: nb stays 0
+  // A structured numbering shows a row length S of H (quads: the north and
+  // south neighbours) or H + 1 (triangles split from quads): every offset is
+  // then a row up or down and a few columns aside, and none wraps around an
+  // end of the row.  Looked for on 1,024 rows spread over the system; the
+  // solve checks every column against its window and declines otherwise.
+  const int ns = min(n, 1024);
+  int worst[2] = {0, 0};
+  for (int q = threadIdx.x; q < ns; q += blockDim.x) {
+    const int i = (int)((long)q * n / ns);
+    res_columns<F>(a.A, i, [&](int j) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int S = max(H + s, 1);
+        const int yi = i / S, yj = j / S;
+        const int dy = yj - yi, dx = abs((j - yj * S) - (i - yi * S));
+        worst[s] = max(worst[s], abs(dy) > 1 ? n : dx);
+      }
+    });
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    if (worst[s] > 0) atomicMax(&s_hx[s], worst[s]);
+  __syncthreads();
+  // thread t tries t / 2 + 1 columns of tiles over the row lengths H and
+  // H + 1 in turn; the fewest halo entries win
+  auto tiles = [&](int q, ResPlan &p) {
+    return res_tiles(n, H + (q & 1), max(s_hx[q & 1], 1), (q >> 1) + 1, a.rmax, a.bmax, a.hmax, p);
+  };
+  for (int q = threadIdx.x; q < 2 * min(a.bmax, kResMaxBlocks); q += blockDim.x) {
+    ResPlan p{};
+    if (tiles(q, p)) atomicMin(&s_best, (p.nh << 10) | q);
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  ResPlan p{};
+  const bool strips = res_strips(n, H, a.rmax, a.bmax, a.hmax, p);
+  if (s_best < INT_MAX && !(strips && 2 * H <= (s_best >> 10))) tiles(s_best & 1023, p);
+  p.H = H;
+  p.ticket = (int)gridDim.x;
+  *a.plan = p;
+}
+
+// --------------------------------------------------------------- exchange --
+
+__device__ __forceinline__ res_word res_load(const res_word *p) {
+  return __hip_atomic_load(const_cast<res_word *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void res_store(res_word *p, res_word v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A double as two words: the exchange's number in the low half, half of the
+// double in the high one.
+__device__ __forceinline__ void res_put(res_word *p, double v, unsigned ep) {
+  const res_word u = __builtin_bit_cast(res_word, v);
+  res_store(p, (u << 32) | ep);
+  res_store(p + 1, (u & 0xffffffff00000000ull) | ep);
+}
+__device__ __forceinline__ double res_get(res_word lo, res_word hi) {
+  return __builtin_bit_cast(double, (hi & 0xffffffff00000000ull) | (lo >> 32));
+}
+
+// The sum over a wavefront, in its last lane: row shifts and row broadcasts
+// in the ALU's data path (DPP) instead of the shuffles' trips through LDS,
+// which an iteration would wait for twice.
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ double res_dpp_add(double v) {
+  const res_word u = __builtin_bit_cast(res_word, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, Ctrl, RowMask, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), Ctrl, RowMask, 0xF, false);
+  return v + __builtin_bit_cast(double, ((res_word)(unsigned)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double res_row_sum(double v) {   // of each 16 lanes, in the last
+  v = res_dpp_add<0x111, 0xF>(v);   // row_shr:1
+  v = res_dpp_add<0x112, 0xF>(v);   // row_shr:2
+  v = res_dpp_add<0x114, 0xF>(v);   // row_shr:4
+  return res_dpp_add<0x118, 0xF>(v);   // row_shr:8
+}
+__device__ __forceinline__ double res_wave_sum(double v) {
+  v = res_row_sum(v);
+  v = res_dpp_add<0x142, 0xA>(v);   // row_bcast:15 into rows 1 and 3
+  v = res_dpp_add<0x143, 0xC>(v);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+__device__ __forceinline__ double res_lane(double v, int lane) {
+  const res_word u = __builtin_bit_cast(res_word, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(u >> 32), lane);
+  return __builtin_bit_cast(double, ((res_word)hi << 32) | lo);
+}
+
+// Waits for up to E doubles, at(q) being the address of the q-th or null;
+// all loads of a poll are issued together.  False if the wait expired.
+template <int E, class At>
+__device__ __forceinline__ bool res_wait(unsigned ep, double *v, At &&at) {
+  res_word lo[E], hi[E];
+  for (unsigned spins = 0;;) {
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const res_word *p = at(q);
+      lo[q] = hi[q] = ep;
+      if (p) {
+        lo[q] = res_load(p);
+        hi[q] = res_load(p + 1);
+      }
+    }
+    bool ok = true;
+#pragma unroll
+    for (int q = 0; q < E; ++q) ok = ok && (unsigned)lo[q] == ep && (unsigned)hi[q] == ep;
+    if (ok) break;
+    if (++spins > kResSpin) return false;
+  }
+#pragma unroll
+  for (int q = 0; q < E; ++q) v[q] = res_get(lo[q], hi[q]);
+  return true;
+}
+
+struct ResArgs {
+  Mat A;
+  const ResPlan *plan;     // null: one block holds the system
+  KState *st;              // written by block 0 at the end: pad6 is a kRes* outcome
+  const double *m;         // Jacobi diagonal
+  double *x;
+  const double *b;
+  res_word *rows;          // 2 buffers of 2 neq words
+  res_word *part;          // kResPartWords
+  double tol;
+  int maxit, x0_zero, stop_rule;
+};
+
+template <int F, int RPT>
+struct Resident {
+  static constexpr int NT = kResThreads, NW = F == F_ELL3 ? 3 : 4, RB = NT * RPT;
+  static constexpr int HE = 3;   // halo entries a thread waits for at once
+
+  const ResArgs &a;
+  ResMap map;
+  double *win;             // LDS: RB + nh
+  double *own;             // LDS: x, then the shadow residual (RB each)
+  double *hs;              // LDS: the halo rows' vectors, nh each
+  int *row;                // LDS: global row of each own row, or -1
+  int *hrow;               // LDS: global row of each halo entry, or -1
+  double *red;             // LDS: kMaxK * kMaxWaves
+  KState *S;               // LDS
+  int *bad;                // LDS
+  int nh, nb;
+  unsigned ep = 0;
+  double av[RPT][NW], dm[RPT];
+  unsigned idx[RPT][2];
+  unsigned pub = 0;        // bit k: another block reads row k
+
+  __device__ __forceinline__ Resident(const ResArgs &args) : a(args) {}
+
+  __device__ __forceinline__ double *state(int q) const { return hs + (size_t)q * nh; }
+
+  // Loads the matrix rows.  False where a column is outside the window.
+  __device__ __forceinline__ bool load_rows() {
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int l = (int)threadIdx.x + k * NT;
+      const int i = map.own(l);
+      row[l] = i;
+      dm[k] = 1.0;
+      int s[4] = {l, l, l, l};
+#pragma unroll
+      for (int e = 0; e < NW; ++e) av[k][e] = 0.0;
+      if (i >= 0) {
+        if (nb > 1 && map.edge(l)) pub |= 1u << k;
+        dm[k] = a.A.ad[i];
+        if constexpr (F == F_CSRD) {
+          const int k1 = a.A.ia[i] - 1, cnt = a.A.ia[i + 1] - 1 - k1;
+          if (cnt > NW) ok = false;
+#pragma unroll
+          for (int e = 0; e < NW; ++e)
+            if (e < cnt) {
+              av[k][e] = a.A.av[k1 + e];
+              s[e] = map.slot(a.A.ja[k1 + e] - 1, RB);
+            }
+        } else {
+#pragma unroll
+          for (int e = 0; e < NW; ++e) {
+            av[k][e] = a.A.av[(size_t)NW * i + e];
+            // padding multiplies the row's own operand by its zero
+            if (av[k][e] != 0.0) s[e] = map.slot(a.A.ja[(size_t)NW * i + e] - 1, RB);
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (s[e] < 0) {
+          ok = false;
+          s[e] = l;
+        }
+      }
+      idx[k][0] = (unsigned)s[0] | ((unsigned)s[1] << 16);
+      idx[k][1] = (unsigned)s[2] | ((unsigned)s[3] << 16);
+    }
+    return ok;
+  }
+
+  // (A u)_k from the window; own = the row's own operand.  The reference's
+  // order of the products, as RowRegs / row_apply.
+  __device__ __forceinline__ double apply(int k, double own) const {
+    const double x0 = win[idx[k][0] & 0xffffu], x1 = win[idx[k][0] >> 16], x2 = win[idx[k][1] & 0xffffu];
+    const double t5 = dm[k] * own;
+    if constexpr (F == F_ELL3) {
+      return ((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + t5;
+    } else {
+      const double x3 = win[idx[k][1] >> 16];
+      if constexpr (F == F_CSRD) return (((t5 + av[k][0] * x0) + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3;
+      else return (((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3) + t5;
+    }
+  }
+
+  __device__ __forceinline__ void publish(int k, double v) const {
+    if (pub >> k & 1u) res_put(a.rows + 2 * ((size_t)((ep + 1) & 1) * a.A.neq + row[threadIdx.x + k * NT]), v, ep + 1);
+  }
+
+  // One exchange: the block's K sums to every block and theirs here, added in
+  // the order of the blocks; the published rows of the halo into hdst (LDS,
+  // nh entries; null: none); then epi(totals) on thread 0.  publish() goes
+  // before.  Some waves wait for the sums and the others for the halo.
+  // False if a wait expired.
+  template <int K, class Epi>
+  __device__ __forceinline__ bool exchange(const double *v, double *hdst, Epi &&epi) {
+    ++ep;
+    const int t = (int)threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const double s = res_wave_sum(v[k]);
+      if (lane == kWave - 1) red[k * kMaxWaves + wid] = s;
+    }
+    lds_barrier();
+    static_assert(K <= 4, "16 lanes per value");
+    res_word *part = a.part + (size_t)(ep & 1) * (kResPartWords / 2);
+    // Up to 64 blocks a lane per block adds all sums.  Beyond, so many
+    // readers of so many words hold each other up (256 blocks: 7 us), and
+    // the sums go in two steps: the first block of 16 adds its group's and
+    // passes the totals to every group, 16 lanes to a value in both steps.
+    const bool wide = nb > kWave, leads = wide && (map.c & 15) == 0;
+    const int waiting = leads ? 2 : 1;   // waves that wait for sums
+    if (wid == 0) {
+      double own = 0.0;
+      if (lane < K) {
+        double q[NT / kWave];
+#pragma unroll
+        for (int w = 0; w < NT / kWave; ++w) q[w] = red[lane * kMaxWaves + w];
+        own = q[0];
+#pragma unroll
+        for (int w = 1; w < NT / kWave; ++w) own += q[w];
+        const int to = wide ? (map.c >> 4) * kWave + lane * 16 + (map.c & 15) : lane * kResMaxBlocks + map.c;
+        if (nb > 1) res_put(part + 2 * (size_t)to, own, ep);
+      }
+      double tot[K];
+      if (nb == 1) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) tot[k] = res_lane(own, k);
+      } else if (!wide) {
+        double pv[K];
+        if (!res_wait<K>(ep, pv, [&](int q) -> const res_word * {
+              return lane < nb ? part + 2 * ((size_t)q * kResMaxBlocks + lane) : nullptr;
+            }))
+          *bad = 1;
+#pragma unroll
+        for (int k = 0; k < K; ++k) tot[k] = res_lane(res_wave_sum(lane < nb ? pv[k] : 0.0), kWave - 1);
+      } else {
+        double g[1];
+        const bool mine = lane < 16 * K && (lane & 15) < (nb + 15) / 16;
+        const res_word *from = part + 2 * (size_t)(kResGroups * kWave + (map.c >> 4) * kWave + lane);
+        if (!res_wait<1>(ep, g, [&](int) { return mine ? from : nullptr; })) *bad = 1;
+        const double s = res_row_sum(mine ? g[0] : 0.0);
+#pragma unroll
+        for (int k = 0; k < K; ++k) tot[k] = res_lane(s, 16 * k + 15);
+      }
+      if (lane == 0) epi(tot);
+    } else if (leads && wid == 1) {
+      double g[1];
+      const int grp = map.c >> 4;
+      const bool mine = lane < 16 * K && (lane & 15) < nb - 16 * grp;
+      const res_word *from = part + 2 * (size_t)(grp * kWave + lane);
+      if (!res_wait<1>(ep, g, [&](int) { return mine ? from : nullptr; })) *bad = 1;
+      const double s = res_row_sum(mine ? g[0] : 0.0);
+      double tot = 0.0;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const double sk = res_lane(s, 16 * k + 15);
+        if (lane >> 4 == k) tot = sk;
+      }
+      // lane (value, group): that group's copy
+      if (lane < 16 * K && (lane & 15) < (nb + 15) / 16)
+        res_put(part + 2 * (size_t)(kResGroups * kWave + (lane & 15) * kWave + (lane & 48) + grp), tot, ep);
+    } else if (nb > 1 && hdst && wid >= waiting) {
+      const res_word *rows = a.rows + (size_t)(ep & 1) * 2 * a.A.neq;
+      const int ht = NT - waiting * kWave, h0 = t - waiting * kWave;
+      auto from = [&](int h) -> const res_word * {
+        const int j = h < nh ? hrow[h] : -1;
+        return j >= 0 ? rows + 2 * (size_t)j : nullptr;
+      };
+      for (int base = 0; base < nh; base += ht * HE) {
+        double hv[HE];
+        const bool few = nh - base <= ht;
+        const bool ok = few ? res_wait<1>(ep, hv, [&](int) { return from(base + h0); })
+                            : res_wait<HE>(ep, hv, [&](int q) { return from(base + h0 + q * ht); });
+        if (!ok) {
+          *bad = 1;
+          break;
+        }
+#pragma unroll
+        for (int q = 0; q < HE; ++q) {
+          const int h = base + h0 + q * ht;
+          if ((q == 0 || !few) && h < nh && hrow[h] >= 0) hdst[h] = hv[q];
+        }
+      }
+    }
+    lds_barrier();
+    if (nb == 1) return true;
+    if (*bad) {
+      if (t == 0) st_relaxed(reinterpret_cast<unsigned *>(&a.st->next), 1u);
+      return false;
+    }
+    return true;
+  }
+
+  // r = b - A x0 on the block's rows, x0 read from memory.
+  __device__ __forceinline__ void residual(double *r, double *bb) {
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int l = (int)threadIdx.x + k * NT, i = row[l];
+      double xi = 0.0, ax = 0.0;
+      bb[k] = 0.0;
+      if (i >= 0) {
+        bb[k] = a.b[i];
+        if (!a.x0_zero) {
+          xi = a.x[i];
+          ax = row_apply<F>(a.A, i, XVec{a.x});
+        }
+      }
+      own[l] = xi;
+      r[k] = bb[k] - ax;
+    }
+  }
+
+  // Energy x.Ax and ||b - Ax||^2 (src/Iterativos.f:82-83,204-205), then x and
+  // the state are written.
+  // A breakdown or an overflow depends on the roundings on the way there, so
+  // such a solve is declined, with x as it came: it is solved again in the
+  // other engine's order of sums, whose outcome the caller gets.
+  __device__ __forceinline__ void finish() {
+    if (S->status == S_BREAKDOWN || S->status == S_NONFINITE) return outcome(kResDeclined);
+    const int t = (int)threadIdx.x;
+    const double *x = own + t;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      win[t + k * NT] = x[k * NT];
+      publish(k, x[k * NT]);
+    }
+    double none[1] = {0.0};
+    // the halo's x must be here before the product: an exchange of its own
+    if (!exchange<1>(none, win + RB, [](const double *) {})) return;
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const double xi = x[k * NT], ax = apply(k, xi);
+      const int i = row[t + k * NT];
+      const double bi = i >= 0 ? a.b[i] : 0.0;
+      const double ri = bi - ax;
+      v[0] += xi * ax;
+      v[1] += ri * ri;
+    }
+    KState *s = S;
+    if (!exchange<2>(v, nullptr, [s](const double *tot) {
+          s->energy = tot[0];
+          s->res2 = tot[1];
+        }))
+      return;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+      if (row[t + k * NT] >= 0) a.x[row[t + k * NT]] = x[k * NT];
+    outcome(kResSolved);
+  }
+
+  // Block 0 writes the state, all of it but `next`, which any block sets when
+  // a wait expires (cleared before the launch; one block alone never waits).
+  __device__ __forceinline__ void outcome(int how) {
+    if (map.c != 0) return;
+    if (threadIdx.x == 0) S->pad6 = how;
+    lds_barrier();
+    constexpr int skip = offsetof(KState, next) / sizeof(unsigned);
+    for (int q = (int)threadIdx.x; q < (int)(sizeof(KState) / sizeof(unsigned)); q += NT)
+      if (q != skip || nb == 1)
+        reinterpret_cast<unsigned *>(a.st)[q] = reinterpret_cast<const unsigned *>(S)[q];
+  }
+
+  __device__ __forceinline__ void pcg();
+  __device__ __forceinline__ void bicgstab();
+};
+
+// The fused PCG (cg1_*, fvc_krylov.h), one exchange per iteration.
+template <int F, int RPT>
+__device__ __forceinline__ void Resident<F, RPT>::pcg() {
+  const int t = (int)threadIdx.x;
+  Cg1Args e{};
+  e.tol = a.tol;
+  e.maxit = a.maxit;
+  e.stop_rule = a.stop_rule;
+  KState *s_ = S;
+  double r[RPT], w[RPT], s[RPT], p[RPT];
+  double *x = own + t;
+  double *hr = state(0), *hw = state(1), *hsv = state(2), *hm = state(3);
+  const bool ok = load_rows();
+  residual(r, w);   // w = b for the moment
+  for (int h = t; h < nh; h += NT) {
+    const int j = hrow[h];
+    hm[h] = j >= 0 ? a.m[j] : 1.0;
+    hr[h] = hw[h] = hsv[h] = 0.0;
+    win[RB + h] = 0.0;
+  }
+  double v[4] = {0.0, 0.0, 0.0, ok ? 0.0 : 1.0};
+#pragma unroll
+  for (int k = 0; k < RPT; ++k) {
+    s[k] = p[k] = 0.0;
+    publish(k, r[k]);
+    v[0] += r[k] * (r[k] / dm[k]);
+    v[1] += w[k] * w[k];
+    v[2] += r[k] * r[k];
+  }
+  if (!exchange<4>(v, hr, [&](const double *tot) {
+        cg1_epi(e, CG1_SETUP, s_, tot);
+        if (tot[3] != 0.0) s_->pend = 1;
+      }))
+    return;
+  if (S->pend) return outcome(kResDeclined);   // a block's columns do not fit its window
+  // round 0 is W0 (w = A u), the following ones CG1_ITER
+  for (int it = 0; !S->done; ++it) {
+    if (it > 0) {
+      const double al = S->alpha, be = S->beta;
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        const double u = win[t + k * NT];   // r / m, of the previous iteration
+        p[k] = it == 1 ? u : u + be * p[k];
+        s[k] = it == 1 ? w[k] : w[k] + be * s[k];
+        x[k * NT] = x[k * NT] + al * p[k];
+        r[k] = r[k] - al * s[k];
+      }
+      for (int h = t; h < nh; h += NT) {
+        const double sj = it == 1 ? hw[h] : hw[h] + be * hsv[h];
+        hsv[h] = sj;
+        hr[h] = hr[h] - al * sj;
+      }
+    }
+    double u[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      u[k] = r[k] / dm[k];
+      win[t + k * NT] = u[k];
+    }
+    for (int h = t; h < nh; h += NT) win[RB + h] = hr[h] / hm[h];
+    lds_barrier();
+    double v3[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      w[k] = apply(k, u[k]);
+      publish(k, w[k]);
+      v3[0] += r[k] * u[k];
+      v3[1] += w[k] * u[k];
+      v3[2] += r[k] * r[k];
+    }
+    if (!exchange<3>(v3, hw, [&](const double *tot) {
+          if (it == 0) cg1_epi(e, CG1_W0, s_, tot + 1);
+          else cg1_epi(e, CG1_ITER, s_, tot);
+        }))
+      return;
+  }
+  finish();
+}
+
+// The two-phase BiCGSTAB (bicg2_*, fvc_krylov.h), one exchange per phase.
+template <int F, int RPT>
+__device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
+  const int t = (int)threadIdx.x;
+  Bicg2Args e{};
+  e.tol = a.tol;
+  e.maxit = a.maxit;
+  e.stop_rule = a.stop_rule;
+  KState *s_ = S;
+  double s[RPT], q_[RPT], p[RPT], v[RPT];   // s holds b between P and Q; q_ is t
+  double *x = own + t, *rh = own + RB + t;
+  double *hsb = state(0), *ht = state(1), *hp = state(2), *hv = state(3), *hm = state(4);
+  const bool ok = load_rows();
+  residual(s, q_);
+  for (int h = t; h < nh; h += NT) {
+    const int j = hrow[h];
+    hm[h] = j >= 0 ? a.m[j] : 1.0;
+    hsb[h] = ht[h] = hp[h] = hv[h] = 0.0;
+    win[RB + h] = 0.0;
+  }
+  double v0[4] = {0.0, 0.0, 0.0, ok ? 0.0 : 1.0};
+#pragma unroll
+  for (int k = 0; k < RPT; ++k) {
+    const double ri = s[k];
+    rh[k * NT] = p[k] = ri;
+    v[k] = 0.0;
+    publish(k, ri);
+    v0[0] += ri * (ri / dm[k]);
+    v0[1] += ri * ri;
+    v0[2] += q_[k] * q_[k];
+    q_[k] = 0.0;
+  }
+  if (!exchange<4>(v0, hp, [&](const double *tot) {
+        bicg2_epi(e, B2_SETUP, s_, tot);
+        if (tot[3] != 0.0) s_->pend = 1;
+      }))
+    return;
+  if (S->pend) return outcome(kResDeclined);
+  for (int h = t; h < nh; h += NT) hsb[h] = hp[h];
+  for (int it = 1; !S->done; ++it) {
+    // P: completes iteration it - 1, p, v = A (p/m)
+    double v3[3] = {0.0, 0.0, 0.0};
+    if (it > 1) {
+      const double al = S->alpha, be = S->beta, om = S->omega;
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        const double z2 = s[k] / dm[k];
+        const double bi = s[k] - om * q_[k];
+        x[k * NT] = (x[k * NT] + al * (p[k] / dm[k])) + om * z2;
+        s[k] = bi;
+        p[k] = bi + be * (p[k] - om * v[k]);
+        v3[1] += bi * z2;
+        v3[2] += bi * bi;
+      }
+      for (int h = t; h < nh; h += NT) {
+        const double bi = hsb[h] - om * ht[h];
+        hsb[h] = bi;
+        hp[h] = bi + be * (hp[h] - om * hv[h]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) win[t + k * NT] = p[k] / dm[k];
+    for (int h = t; h < nh; h += NT) win[RB + h] = hp[h] / hm[h];
+    lds_barrier();
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      v[k] = apply(k, win[t + k * NT]);
+      publish(k, v[k]);
+      v3[0] += v[k] * rh[k * NT];
+    }
+    if (!exchange<3>(v3, hv, [&](const double *tot) { bicg2_epi(e, B2_P, s_, tot); })) return;
+    if (S->done) break;
+    // Q: s = b - alpha v, t = A (s/m)
+    const double al = S->alpha;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      s[k] = s[k] - al * v[k];
+      win[t + k * NT] = s[k] / dm[k];
+    }
+    for (int h = t; h < nh; h += NT) {
+      hsb[h] = hsb[h] - al * hv[h];
+      win[RB + h] = hsb[h] / hm[h];
+    }
+    lds_barrier();
+    double v4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      q_[k] = apply(k, win[t + k * NT]);
+      publish(k, q_[k]);
+      v4[0] += q_[k] * s[k];
+      v4[1] += q_[k] * q_[k];
+      v4[2] += rh[k * NT] * s[k];
+      v4[3] += rh[k * NT] * q_[k];
+    }
+    if (!exchange<4>(v4, ht, [&](const double *tot) { bicg2_epi(e, B2_Q, s_, tot); })) return;
+  }
+  finish();
+}
+
+// One block per CU, all co-resident (the host checks that the grid fits).
+template <int F, int RPT, int Code>
+__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ double red[2 * kMaxK * kMaxWaves];
+  __shared__ KState S;
+  __shared__ int bad;
+  ResPlan p{};
+  if (a.plan) {
+    p = *a.plan;
+  } else {
+    p.nb = 1;
+    p.R = a.A.neq;
+  }
+  const int g = (int)gridDim.x, b = (int)blockIdx.x;
+  // consecutive parts of the system on one XCD (blocks b = x mod 8)
+  const int c = (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
+  if (p.nb == 0 && b == 0 && threadIdx.x == 0) a.st->pad6 = kResDeclined;
+  if (c >= p.nb || p.nb > kResMaxBlocks || p.nh > res_max_halo(Code, RPT) || p.R > kResThreads * RPT) return;
+  const int t = (int)threadIdx.x;
+  for (int k = t; k < (int)(sizeof(KState) / sizeof(unsigned)); k += kResThreads)
+    reinterpret_cast<unsigned *>(&S)[k] = 0u;
+  if (t == 0) bad = 0;
+  Resident<F, RPT> w(a);
+  w.map.init(p, a.A.neq, c);
+  w.nh = p.nb > 1 ? p.nh : 0;
+  w.nb = p.nb;
+  w.win = dyn;
+  w.own = dyn + kResThreads * RPT + w.nh;
+  w.hs = w.own + (size_t)res_own_vecs(Code) * kResThreads * RPT;
+  w.row = reinterpret_cast<int *>(w.hs + (size_t)res_halo_vecs(Code) * w.nh);
+  w.hrow = w.row + kResThreads * RPT;
+  w.red = red;
+  w.S = &S;
+  w.bad = &bad;
+  for (int h = t; h < w.nh; h += kResThreads) w.hrow[h] = w.map.halo(h);
+  __syncthreads();
+  if constexpr (Code == 1) w.pcg();
+  else w.bicgstab();
+}
+
+}  // namespace fvc

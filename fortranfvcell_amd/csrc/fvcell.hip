@@ -313,6 +313,7 @@ int read_state(DevState &d, KState *st, hipStream_t s) {
 
 void fill_stats(fvc_stats *stats, const KState &hs, int code, bool persistent, float ms, int G, int bs,
                 int flags);
+int status_of(const KState &hs);
 int finish(const KState &hs, unsigned *ctr);
 
 // The size of the next batch: doubling up to kMaxBatch, capped near the end
@@ -378,11 +379,82 @@ int drive_batches(DevState &d, hipStream_t s, int maxit, Iter &&iteration, State
   return FVC_OK;
 }
 
+// The on-chip PCG / BiCGSTAB (fvc_resident.h).  Measured on MI355X against one
+// kernel per phase, whole solves to a true residual of 1e-10: PCG 4,096 rows
+// 3.93 -> 1.27 ms, 429,713 rows 77.8 -> 22.8; BiCGSTAB 12,707 rows 0.92 ->
+// 0.37, 1,048,576 rows 2.61 -> 0.77.
+constexpr bool resident_format(int F) { return F == F_ELL4 || F == F_ELL3 || F == F_CSRD; }
+
+template <int F>
+const void *resident_fn(int code, int rpt) {
+  if constexpr (resident_format(F)) {
+    switch (rpt) {
+      case 1: return code == FVC_PCG ? (const void *)&resident_kernel<F, 1, 1> : (const void *)&resident_kernel<F, 1, 2>;
+      case 2: return code == FVC_PCG ? (const void *)&resident_kernel<F, 2, 1> : (const void *)&resident_kernel<F, 2, 2>;
+      case 4: return code == FVC_PCG ? (const void *)&resident_kernel<F, 4, 1> : (const void *)&resident_kernel<F, 4, 2>;
+      case 8: return code == FVC_PCG ? (const void *)&resident_kernel<F, 8, 1> : (const void *)&resident_kernel<F, 8, 2>;
+    }
+  }
+  return nullptr;
+}
+
+// Solves on chip if the system fits; *done says whether it did (else the
+// caller solves it one kernel per phase).  part: kResPartWords words; rows:
+// at least 4 neq words (vectors that the caller does not need yet).
+template <int F>
+int run_resident(DevState &d, const SolveIn &in, KState *st, unsigned *ctr, res_word *part, res_word *rows,
+                 fvc_stats *stats, hipStream_t s, bool *done) {
+  *done = false;
+  if constexpr (!resident_format(F)) {
+    return FVC_OK;
+  } else {
+    const int neq = in.A.neq;
+    const ResShape sh = resident_shape(neq, d.cus);
+    if (sh.rpt == 0) return FVC_OK;
+    ResArgs a{};
+    a.A = in.A; a.st = st; a.m = in.m; a.x = in.x; a.b = in.b;
+    a.tol = in.tol; a.maxit = in.maxit; a.x0_zero = in.x0_zero; a.stop_rule = in.stop_rule;
+    const void *fn = resident_fn<F>(in.code, sh.rpt);
+    const int hmax = sh.blocks > 1 ? res_max_halo(in.code, sh.rpt) : 0;
+    const size_t lds = res_lds_bytes(in.code, sh.rpt, hmax);
+    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int occ = 0;
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, kResThreads, lds));
+    if ((long)occ * d.cus < sh.blocks) return FVC_OK;
+    HIPCHK(hipEventRecord(d.ev0, s));
+    if (sh.blocks > 1) {
+      // the plan sits among the counters, which the reset clears
+      ResPlan *plan = reinterpret_cast<ResPlan *>(ctr + 8);
+      static_assert(8 * sizeof(unsigned) + sizeof(ResPlan) <= kCtrStride * sizeof(unsigned), "plan outgrows its gap");
+      a.plan = plan;
+      a.rows = rows;
+      a.part = part;
+      hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, (int)kCtrWords, st, 1);
+      ResPrepArgs pa{in.A, plan, part, rows, kResThreads * sh.rpt, sh.blocks, hmax};
+      hipLaunchKernelGGL(resident_prep_kernel<F>, dim3(std::min((neq + 255) / 256, 4 * d.cus)), dim3(256), 0, s, pa);
+    }
+    HIPCHK(hipGetLastError());
+    void *params[] = {&a};
+    HIPCHK(hipLaunchKernel(fn, dim3(sh.blocks), dim3(kResThreads), params, lds, s));
+    HIPCHK(hipEventRecord(d.ev1, s));
+    const int rc = read_state(d, st, s);
+    if (rc) return rc;
+    const KState &hs = *d.host_st;
+    if (hs.pad6 != kResSolved || hs.next != 0) return FVC_OK;   // does not fit, or a wait expired
+    *done = true;
+    float ms = 0.f;
+    HIPCHK(hipEventElapsedTime(&ms, d.ev0, d.ev1));
+    fill_stats(stats, hs, in.code, true, ms, sh.blocks, kResThreads, 0);
+    return status_of(hs);
+  }
+}
+
 template <int F>
 int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   const int neq = in.A.neq;
   const bool fused = in.recurrence == FVC_REC_FUSED;
-  // AUTO: PCG and BiCGSTAB run one kernel per phase (with kernel boundaries
+  // AUTO: PCG and BiCGSTAB that do not fit the chip (run_resident below) run
+  // one kernel per phase (with kernel boundaries
   // for ordering, a phase needs no fence and no atomic; measured faster on
   // MI355X than the grid barrier of one persistent launch); GMRES, whose
   // Arnoldi step is a chain of short phases, runs persistent.
@@ -469,12 +541,18 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
                  align_up((size_t)(k + 2) * (k + 2) * sizeof(double)) * 2 + align_up(n * sizeof(double)) +
                  align_up(2 * sizeof(KState)) + align_up(2 * kMaxK * (size_t)G * sizeof(double)) +
                  align_up(lag_small * sizeof(double)) + align_up(lag_parts * sizeof(double)) + 4096;
+  // the on-chip solver's words for partial sums, where the fixed workspace
+  // has room for them (its limit stays that of the engines below)
+  size_t res_part = align_up(kResPartWords * sizeof(res_word));
+  if (d.noalloc && bytes + res_part > kScratchBytes) res_part = 0;
+  bytes += res_part;
   char *ws = nullptr;
   if ((rc = workspace(d, bytes, &ws))) return rc;
   Carve cv{ws, bytes};
   unsigned *ctr = cv.take<unsigned>(kCtrWords + (size_t)G);
   KState *st = cv.take<KState>(1);
   double *partials = cv.take<double>(npart);
+  res_word *part = cv.take<res_word>(res_part / sizeof(res_word));
   // deferred reductions (kernel-per-phase engine of the fused methods)
   Defer dfr{cv.take<KState>(2), cv.take<double>(2 * kMaxK * (size_t)G), 0};
   double *vec[kMaxGmresK + 1];
@@ -484,6 +562,14 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   double *lagsmall = cv.take<double>(lag_small);
   double *lagpart = cv.take<double>(lag_parts);
   if (!cv.fits()) return carve_overflow(cv);
+  // On chip where the launch is the library's choice; options that shape it
+  // keep the engines they were written for.
+  if (in.engine == FVC_ENGINE_AUTO && in.code != FVC_GMRES && fused && in.bs == 0 && in.G_req == 0 &&
+      in.barrier == 0 && in.row_order == 0 && !in.lanex && res_part) {
+    bool done = false;
+    rc = run_resident<F>(d, in, st, ctr, part, reinterpret_cast<res_word *>(vec[0]), stats, s, &done);
+    if (rc || done) return rc;
+  }
   const bool may_fall_back = persistent && in.engine == FVC_ENGINE_AUTO;
   if (may_fall_back && !in.x0_zero)
     HIPCHK(hipMemcpyAsync(xbackup, in.x, n * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -756,6 +842,10 @@ int finish(const KState &hs, unsigned *ctr) {
   unsigned err = 0;
   HIPCHK(hipMemcpy(&err, ctr + kCtrErr, sizeof err, hipMemcpyDeviceToHost));
   if (err) return fail(FVC_DEVICE_ERROR, "persistent solve: a grid barrier wait expired");
+  return status_of(hs);
+}
+
+int status_of(const KState &hs) {
   if (hs.status != S_OK) {
     static const char *names[] = {"converged", "maximum iterations reached", "breakdown", "non-finite value"};
     return fail(hs.status, "%s after %d iterations", names[std::min(std::max(hs.status, 0), 3)], hs.iter);

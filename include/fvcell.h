@@ -73,7 +73,12 @@ extern "C" {
                                    cycles                                                    */
 
 /* Engines. */
-#define FVC_ENGINE_AUTO 0        /* KERNELS for PCG and BiCGSTAB, PERSISTENT for GMRES   */
+#define FVC_ENGINE_AUTO 0        /* PCG and BiCGSTAB (fused, FP64, ELLPACK of width 3 or 4
+                                    or CSRD rows of at most four off-diagonals, none of
+                                    the options that shape a launch set): on chip in one
+                                    launch where the system fits (up to 1,048,576 rows on
+                                    256 CUs; stats.engine then says PERSISTENT), else
+                                    KERNELS.  GMRES: PERSISTENT                          */
 #define FVC_ENGINE_KERNELS 1     /* one kernel per phase; fused recurrences sum the block
                                     partials at the next launch, the others in the last
                                     block of the launch                                 */

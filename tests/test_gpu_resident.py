@@ -1,0 +1,120 @@
+"""PCG and BiCGSTAB held on chip (fvc_resident.h), which AUTO takes where the
+system fits: against the engine that runs one kernel per phase, at the edges
+of what a block, a launch and a tile hold, for every layout that takes this
+path, both starting points and a capped iteration count.
+
+Bars: after three iterations only the order of the sums differs, so x agrees
+to 1e-12 (a few hundred roundings of sums of up to 300,000 terms); solved to a
+true residual of 1e-10, ||x - x'|| <= 1e-8 ||x'||, the library's bar for
+solutions."""
+import numpy as np
+import pytest
+
+from fortranfvcell_amd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+def _mesh(kind, nx, ny):
+    return P.quad_mesh(nx, ny, jitter=0.1, seed=nx) if kind == "quad" else P.tri_mesh(nx, jitter=0.1, seed=nx)
+
+
+# one row; one thread's, two's, four's rows of one block and just beyond (2,048
+# rows); up to 64 blocks and just beyond; rows per thread 2 -> 4 (249k rows) and
+# 4 -> 8; long, thin meshes (strips, wide and narrow tiles)
+SHAPES = [("quad", 1, 1), ("quad", 3, 2), ("quad", 32, 16), ("quad", 27, 19), ("quad", 32, 32), ("quad", 64, 32),
+          ("quad", 41, 50), ("tri", 37, 0), ("quad", 13, 2041), ("quad", 2041, 13), ("quad", 163, 163),
+          ("quad", 231, 230), ("tri", 170, 0), ("quad", 499, 498), ("quad", 499, 501), ("tri", 500, 0)]
+
+
+@pytest.mark.parametrize("kind,nx,ny", SHAPES)
+@pytest.mark.parametrize("code", [1, 2], ids=["pcg", "bicgstab"])
+def test_resident_matches_kernels(fvc, kind, nx, ny, code):
+    m = _mesh(kind, nx, ny)
+    s = P.pressure_system(m, k=P.lognormal_k(3, m.neq), pin="penalty") if code == 1 else \
+        P.advdiff_system(m, dt=0.005, under_relax=0.8) if m.neq > 1 else P.pressure_system(m, pin="identity")
+    if code == 1 and m.neq == 1:
+        s = P.pressure_system(m, pin="identity")
+        s.b[:] = 2.0
+    x0 = np.random.default_rng(nx).normal(size=m.neq)
+    for lay in (P.to_ell, P.to_csrd):
+        f = lay(s)
+        for opt in (dict(x0_rule=fvc.X0_ZERO, maxit=3), dict(x0_rule=fvc.X0_GIVEN, maxit=3),
+                    dict(x0_rule=fvc.X0_ZERO), dict(x0_rule=fvc.X0_GIVEN)):
+            if "maxit" not in opt and code == 1 and m.neq > 60000:
+                continue
+            print(f"resident {kind} {nx}x{ny} neq={m.neq} code={code} {lay.__name__} {opt}", flush=True)
+            kw = dict(tol=1e-10, stop_rule=fvc.STOP_RELRES, **opt)
+            xa, sa = fvc.solve(f, code, x0=x0, **kw)
+            xk, sk = fvc.solve(f, code, x0=x0, engine=fvc.ENGINE_KERNELS, **kw)
+            assert sa["status"] == sk["status"] and sk["engine"] == fvc.ENGINE_KERNELS
+            # a breakdown (BiCGSTAB on one row) is left to the other engine
+            assert sa["engine"] == (fvc.ENGINE_PERSISTENT if sa["status"] <= 1 else fvc.ENGINE_KERNELS)
+            capped = "maxit" in opt
+            assert _rel(xa, xk) <= (1e-12 if capped else 1e-8), (opt, sa, sk)
+            if capped:
+                assert sa["iterations"] == sk["iterations"]
+                assert abs(sa["energy"] - sk["energy"]) <= 1e-10 * abs(sk["energy"])
+            elif sa["status"] == 0:
+                assert sa["true_relres"] <= 1e-10
+
+
+@pytest.mark.parametrize("n", [(24, 23), (113, 90), (400, 380)], ids=["one_block", "few_blocks", "many_blocks"])
+def test_resident_repeats_bit_for_bit(fvc, n):
+    s = P.advdiff_system(_mesh("quad", *n), dt=0.005, under_relax=0.8)
+    ds = fvc.DeviceSystem(P.to_ell(s))
+    xs = []
+    for _ in range(3):
+        ds.solve(fvc.BICGSTAB, tol=1e-11, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_ZERO)
+        xs.append(ds.x.get())
+    assert np.array_equal(xs[0], xs[1]) and np.array_equal(xs[0], xs[2])
+
+
+def test_resident_declines_what_does_not_fit(fvc):
+    """Columns far apart (a random numbering), and rows of more than four
+    off-diagonals: solved one kernel per phase, the same answer."""
+    s = P.config_pressure_lognormal(100)
+    p = np.random.default_rng(5).permutation(s.neq)
+    q = np.empty(s.neq, np.int64)
+    q[p] = np.arange(s.neq)
+    nbr = np.where(s.nbr[p] >= 0, q[np.maximum(s.nbr[p], 0)], -1)
+    renum = P.System(s.neq, s.w, s.ad[p], s.off[p], nbr, s.b[p])
+    x, st = fvc.solve(P.to_ell(renum), fvc.PCG, tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_ZERO)
+    assert st["engine"] == fvc.ENGINE_KERNELS and st["status"] == 0 and st["true_relres"] <= 1e-10
+    # a 9-point operator in CSRD: eight off-diagonals a row, in one block and in several
+    import scipy.sparse as sp
+    for n in (16, 70):
+        t = sp.diags([-1.0, 2.5, -1.0], [-1, 0, 1], shape=(n, n))
+        A = sp.kron(t, t).tocsr()
+        A.sort_indices()
+        d = A.diagonal()
+        off = (A - sp.diags(d)).tocsr()
+        off.eliminate_zeros()
+        off.sort_indices()
+        b = np.random.default_rng(n).normal(size=n * n)
+        f = dict(matriz=1, neq=n * n, nad=off.nnz, iax=(off.indptr + 1).astype(np.int32),
+                 ja=(off.indices + 1).astype(np.int32), ad=d, al=off.data.copy(), au=None, b=b, sym=False)
+        x, st = fvc.solve(f, fvc.PCG, tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_ZERO, maxit=20000)
+        assert st["engine"] == fvc.ENGINE_KERNELS and st["status"] == 0
+        assert np.linalg.norm(b - A @ x) <= 1.01e-10 * np.linalg.norm(b)
+
+
+def test_resident_reports_breakdown_and_nonfinite(fvc):
+    """Left to one kernel per phase, whose status the caller gets, in one block
+    and in several; x0 is what that engine starts from."""
+    for n in (16, 70):
+        s = P.config_advdiff(n, peclet_max=10.0)
+        f = P.to_ell(s)
+        for b in (np.zeros(s.neq), np.where(np.arange(s.neq) == 3, np.nan, 1.0)):
+            for code in (1, 2):
+                for stop in (fvc.STOP_RELRES, fvc.STOP_REFERENCE):
+                    kw = dict(b=b, tol=1e-10, stop_rule=stop, x0_rule=fvc.X0_ZERO, maxit=50)
+                    _, sa = fvc.solve(f, code, **kw)
+                    _, sk = fvc.solve(f, code, engine=fvc.ENGINE_KERNELS, **kw)
+                    assert (sa["status"], sa["iterations"]) == (sk["status"], sk["iterations"]), (n, code, stop)
+                    if sa["status"] > 1:
+                        assert sa["engine"] == fvc.ENGINE_KERNELS
