@@ -24,7 +24,9 @@ from . import GMRES, DeviceSystem, device_info
 CACHE_PATH = os.environ.get("FVC_TUNE_CACHE", os.path.join(os.path.expanduser("~"), ".cache",
                                                             "fvcell_tune.json"))
 
-BLOCK_SIZES = (256, 512, 1024)
+# 0: the library's own choice, which holds a system (or a batch) that fits on
+# the chip; the others shape the engines that stream it from memory
+BLOCK_SIZES = (0, 256, 512, 1024)
 BARRIERS = (0, 1)
 
 
@@ -33,7 +35,9 @@ def _bucket(neq: int) -> int:
 
 
 def _key(method: int, fmt_family: str, neq: int) -> str:
-    return f"{device_info()['name']}|m{method}|{fmt_family}|2^{_bucket(neq)}"
+    # "c": the candidates include the library's own choice (entries without it
+    # were chosen among the other shapes and are not read)
+    return f"c|{device_info()['name']}|m{method}|{fmt_family}|2^{_bucket(neq)}"
 
 
 def load_cache() -> dict:
@@ -53,10 +57,10 @@ def save_cache(cache: dict) -> None:
 
 
 def candidates(cus: int, neq: int):
-    """Launch shapes worth timing: blocks from half the CUs to four per CU,
-    never fewer than 64 rows per block."""
-    out = []
-    for bs in BLOCK_SIZES:
+    """Launch shapes worth timing: the library's own choice, and blocks from
+    half the CUs to four per CU, never fewer than 64 rows per block."""
+    out = [dict(block_size=0, grid_blocks=0, barrier=0)]
+    for bs in BLOCK_SIZES[1:]:
         for per_cu in (0.5, 1, 2, 4):
             G = int(cus * per_cu)
             if G < 8 or neq // G < 64:

@@ -31,6 +31,7 @@
 #include <limits.h>
 #include <stddef.h>
 
+#include "fvc_batch.h"
 #include "fvc_krylov.h"
 #include "fvc_resplan.h"
 
@@ -41,16 +42,17 @@ constexpr unsigned kResSpin = 1u << 20;   // polls of a bounded wait (about two 
 typedef unsigned long long res_word;
 
 // KState::pad6 after a launch: solved, or the system does not fit this scheme
-// (solve it another way).  Anything else, or KState::next set: a wait expired.
+// (solve it another way).  Anything else, or the err word set: a wait expired.
 constexpr int kResSolved = 1, kResDeclined = 2;
 
 // ------------------------------------------------------------------- prep --
 
 struct ResPrepArgs {
   Mat A;
-  ResPlan *plan;      // zeroed
-  res_word *part, *rows;   // cleared here: kResPartWords and 4 neq words
-  int rmax, bmax, hmax;   // rows per block, blocks and halo entries at most
+  ResPlan *plan;           // zeroed
+  res_word *part, *rows;   // cleared here: nparts and 4 neq words
+  int nparts;
+  int rmax, bmax, hmax;    // rows per block, blocks and halo entries at most
 };
 
 // The columns of row i that count: off-diagonal entries other than
@@ -70,16 +72,17 @@ __device__ __forceinline__ void res_columns(const Mat &A, int i, Fn &&fn) {
 }
 
 // Clears the exchange words, finds the largest |column - row|, and (its last
-// block) decides how the rows are dealt.  One pass over the columns.
+// block) decides how the rows are dealt.  One pass over the columns by
+// gridDim.x blocks.
 template <int F>
-__global__ __launch_bounds__(256) void resident_prep_kernel(ResPrepArgs a) {
+__device__ __forceinline__ void resident_prep(const ResPrepArgs &a) {
   __shared__ int s_h, s_last, s_best, s_hx[2];
   const int n = a.A.neq, step = (int)(gridDim.x * blockDim.x);
   if (threadIdx.x == 0) s_h = 0;
   __syncthreads();
   const int first = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   for (size_t k = first; k < (size_t)4 * n; k += (size_t)step) a.rows[k] = 0ull;
-  for (int k = first; k < kResPartWords; k += step) a.part[k] = 0ull;
+  for (int k = first; k < a.nparts; k += step) a.part[k] = 0ull;
   int h = 0;
   for (long i = first; i < n; i += step) {
     res_columns<F>(a.A, (int)i, [&](int j) { h = max(h, abs(j - (int)i)); });
@@ -142,6 +145,11 @@ __global__ __launch_bounds__(256) void resident_prep_kernel(ResPrepArgs a) {
   *a.plan = p;
 }
 
+template <int F>
+__global__ __launch_bounds__(256) void resident_prep_kernel(ResPrepArgs a) {
+  resident_prep<F>(a);
+}
+
 // --------------------------------------------------------------- exchange --
 
 __device__ __forceinline__ res_word res_load(const res_word *p) {
@@ -191,9 +199,10 @@ __device__ __forceinline__ double res_lane(double v, int lane) {
 }
 
 // Waits for up to E doubles, at(q) being the address of the q-th or null;
-// all loads of a poll are issued together.  False if the wait expired.
+// all loads of a poll are issued together.  False if the wait expired, after
+// `limit` polls or when another wait did (*err).
 template <int E, class At>
-__device__ __forceinline__ bool res_wait(unsigned ep, double *v, At &&at) {
+__device__ __forceinline__ bool res_wait(unsigned ep, double *v, unsigned limit, const unsigned *err, At &&at) {
   res_word lo[E], hi[E];
   for (unsigned spins = 0;;) {
 #pragma unroll
@@ -209,7 +218,11 @@ __device__ __forceinline__ bool res_wait(unsigned ep, double *v, At &&at) {
 #pragma unroll
     for (int q = 0; q < E; ++q) ok = ok && (unsigned)lo[q] == ep && (unsigned)hi[q] == ep;
     if (ok) break;
-    if (++spins > kResSpin) return false;
+    if (++spins > limit) return false;
+    if (spins >= 1024u) {   // somebody is late: leave the memory to them
+      __builtin_amdgcn_s_sleep(8);
+      if ((spins & 1023u) == 0u && ld_relaxed(const_cast<unsigned *>(err)) != 0u) return false;
+    }
   }
 #pragma unroll
   for (int q = 0; q < E; ++q) v[q] = res_get(lo[q], hi[q]);
@@ -224,7 +237,10 @@ struct ResArgs {
   double *x;
   const double *b;
   res_word *rows;          // 2 buffers of 2 neq words
-  res_word *part;          // kResPartWords
+  res_word *part;          // two buffers of part_half words
+  unsigned *err;           // set when a wait expired; the waits of others end too
+  int part_half;
+  int gang;                // how many times longer the first exchange may take
   double tol;
   int maxit, x0_zero, stop_rule;
 };
@@ -334,7 +350,9 @@ struct Resident {
     }
     lds_barrier();
     static_assert(K <= 4, "16 lanes per value");
-    res_word *part = a.part + (size_t)(ep & 1) * (kResPartWords / 2);
+    res_word *part = a.part + (size_t)(ep & 1) * (size_t)a.part_half;
+    // a block may come to its first exchange long before the others
+    const unsigned limit = ep == 1 ? kResSpin * (unsigned)a.gang : kResSpin;
     // Up to 64 blocks a lane per block adds all sums.  Beyond, so many
     // readers of so many words hold each other up (256 blocks: 7 us), and
     // the sums go in two steps: the first block of 16 adds its group's and
@@ -350,7 +368,7 @@ struct Resident {
         own = q[0];
 #pragma unroll
         for (int w = 1; w < NT / kWave; ++w) own += q[w];
-        const int to = wide ? (map.c >> 4) * kWave + lane * 16 + (map.c & 15) : lane * kResMaxBlocks + map.c;
+        const int to = wide ? (map.c >> 4) * kWave + lane * 16 + (map.c & 15) : lane * kWave + map.c;
         if (nb > 1) res_put(part + 2 * (size_t)to, own, ep);
       }
       double tot[K];
@@ -359,8 +377,8 @@ struct Resident {
         for (int k = 0; k < K; ++k) tot[k] = res_lane(own, k);
       } else if (!wide) {
         double pv[K];
-        if (!res_wait<K>(ep, pv, [&](int q) -> const res_word * {
-              return lane < nb ? part + 2 * ((size_t)q * kResMaxBlocks + lane) : nullptr;
+        if (!res_wait<K>(ep, pv, limit, a.err, [&](int q) -> const res_word * {
+              return lane < nb ? part + 2 * ((size_t)q * kWave + lane) : nullptr;
             }))
           *bad = 1;
 #pragma unroll
@@ -369,7 +387,7 @@ struct Resident {
         double g[1];
         const bool mine = lane < 16 * K && (lane & 15) < (nb + 15) / 16;
         const res_word *from = part + 2 * (size_t)(kResGroups * kWave + (map.c >> 4) * kWave + lane);
-        if (!res_wait<1>(ep, g, [&](int) { return mine ? from : nullptr; })) *bad = 1;
+        if (!res_wait<1>(ep, g, limit, a.err, [&](int) { return mine ? from : nullptr; })) *bad = 1;
         const double s = res_row_sum(mine ? g[0] : 0.0);
 #pragma unroll
         for (int k = 0; k < K; ++k) tot[k] = res_lane(s, 16 * k + 15);
@@ -380,7 +398,7 @@ struct Resident {
       const int grp = map.c >> 4;
       const bool mine = lane < 16 * K && (lane & 15) < nb - 16 * grp;
       const res_word *from = part + 2 * (size_t)(grp * kWave + lane);
-      if (!res_wait<1>(ep, g, [&](int) { return mine ? from : nullptr; })) *bad = 1;
+      if (!res_wait<1>(ep, g, limit, a.err, [&](int) { return mine ? from : nullptr; })) *bad = 1;
       const double s = res_row_sum(mine ? g[0] : 0.0);
       double tot = 0.0;
 #pragma unroll
@@ -401,8 +419,8 @@ struct Resident {
       for (int base = 0; base < nh; base += ht * HE) {
         double hv[HE];
         const bool few = nh - base <= ht;
-        const bool ok = few ? res_wait<1>(ep, hv, [&](int) { return from(base + h0); })
-                            : res_wait<HE>(ep, hv, [&](int q) { return from(base + h0 + q * ht); });
+        const bool ok = few ? res_wait<1>(ep, hv, limit, a.err, [&](int) { return from(base + h0); })
+                            : res_wait<HE>(ep, hv, limit, a.err, [&](int q) { return from(base + h0 + q * ht); });
         if (!ok) {
           *bad = 1;
           break;
@@ -417,7 +435,7 @@ struct Resident {
     lds_barrier();
     if (nb == 1) return true;
     if (*bad) {
-      if (t == 0) st_relaxed(reinterpret_cast<unsigned *>(&a.st->next), 1u);
+      if (t == 0) st_relaxed(a.err, 1u);
       return false;
     }
     return true;
@@ -481,8 +499,8 @@ struct Resident {
     outcome(kResSolved);
   }
 
-  // Block 0 writes the state, all of it but `next`, which any block sets when
-  // a wait expires (cleared before the launch; one block alone never waits).
+  // Block 0 writes the state, all of it but `next`, which is a solve's err
+  // word (cleared before the launch; one block alone never waits).
   __device__ __forceinline__ void outcome(int how) {
     if (map.c != 0) return;
     if (threadIdx.x == 0) S->pad6 = how;
@@ -675,25 +693,13 @@ __device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
   finish();
 }
 
-// One block per CU, all co-resident (the host checks that the grid fits).
+// Sets a block up as part c of a system and solves it.  dyn: the block's
+// dynamic shared memory (res_lds_bytes).
 template <int F, int RPT, int Code>
-__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a) {
-  extern __shared__ double dyn[];
-  __shared__ double red[2 * kMaxK * kMaxWaves];
+__device__ __forceinline__ void resident_solve(const ResArgs &a, const ResPlan &p, int c, double *dyn) {
+  __shared__ double red[kMaxK * kMaxWaves];
   __shared__ KState S;
   __shared__ int bad;
-  ResPlan p{};
-  if (a.plan) {
-    p = *a.plan;
-  } else {
-    p.nb = 1;
-    p.R = a.A.neq;
-  }
-  const int g = (int)gridDim.x, b = (int)blockIdx.x;
-  // consecutive parts of the system on one XCD (blocks b = x mod 8)
-  const int c = (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
-  if (p.nb == 0 && b == 0 && threadIdx.x == 0) a.st->pad6 = kResDeclined;
-  if (c >= p.nb || p.nb > kResMaxBlocks || p.nh > res_max_halo(Code, RPT) || p.R > kResThreads * RPT) return;
   const int t = (int)threadIdx.x;
   for (int k = t; k < (int)(sizeof(KState) / sizeof(unsigned)); k += kResThreads)
     reinterpret_cast<unsigned *>(&S)[k] = 0u;
@@ -714,6 +720,124 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a) {
   __syncthreads();
   if constexpr (Code == 1) w.pcg();
   else w.bicgstab();
+}
+
+// Does block c take part in plan p?
+template <int RPT, int Code>
+__device__ __forceinline__ bool resident_part(const ResPlan &p, int c) {
+  return c < p.nb && p.nb <= kResMaxBlocks && p.nh <= res_max_halo(Code, RPT) && p.R <= kResThreads * RPT;
+}
+
+// One system on the whole grid, one block per CU, all co-resident (the host
+// checks that the grid fits).
+template <int F, int RPT, int Code>
+__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a) {
+  extern __shared__ double dyn[];
+  ResPlan p{};
+  if (a.plan) {
+    p = *a.plan;
+  } else {
+    p.nb = 1;
+    p.R = a.A.neq;
+  }
+  const int g = (int)gridDim.x, b = (int)blockIdx.x;
+  // consecutive parts of the system on one XCD (blocks b = x mod 8)
+  const int c = (g & 7) == 0 ? (b & 7) * (g >> 3) + (b >> 3) : b;
+  if (p.nb == 0 && b == 0 && threadIdx.x == 0) a.st->pad6 = kResDeclined;
+  if (!resident_part<RPT, Code>(p, c)) return;
+  resident_solve<F, RPT, Code>(a, p, c, dyn);
+}
+
+// ---------------------------------------------------------------- batches --
+//
+// Many systems in one launch: a system gets a team of consecutive blocks just
+// large enough to hold it, and a block's systems follow each other in the
+// order of one list, the same for all blocks, so teams never wait in a ring.
+// All blocks are co-resident.
+struct ResBatchArgs {
+  int w;
+  const double *ad, *av, *b;
+  const int *ia, *ja;
+  double *x;
+  const SysDesc *desc;       // g_first, g_count: the team
+  const int *part_off;       // where a system's words for partial sums start
+  const int *block_ptr, *block_list;
+  KState *st;                // per system, cleared
+  ResPlan *plans;            // per system, cleared
+  res_word *rows, *part;
+  unsigned *err;
+  double tol;
+  int maxit, x0_zero, stop_rule, rmax, hmax;
+};
+
+constexpr int kResGang = 32;   // a team's first exchange may wait for its members' earlier systems
+
+template <int F>
+__device__ __forceinline__ void resident_batch_mat(const ResBatchArgs &B, const SysDesc &D, Mat &A) {
+  A.neq = D.neq;
+  A.w = B.w;
+  A.ad = B.ad + D.row_off;
+  A.av = B.av + D.val_off;
+  A.au = nullptr;
+  A.ia = F == F_CSRD ? B.ia + D.ia_off : nullptr;
+  A.ja = B.ja + D.val_off;
+  A.tptr = A.tsrc = A.tpos = nullptr;
+}
+
+// blockIdx.y: the systems of `multi` (those of more than one block)
+template <int F>
+__global__ __launch_bounds__(256) void resident_batch_prep_kernel(ResBatchArgs B, const int *multi) {
+  const int sys = multi[blockIdx.y];
+  const SysDesc D = B.desc[sys];
+  ResPrepArgs a{};
+  resident_batch_mat<F>(B, D, a.A);
+  a.plan = B.plans + sys;
+  a.part = B.part + B.part_off[sys];
+  a.rows = B.rows + (size_t)4 * D.row_off;
+  a.nparts = 2 * res_part_half(D.g_count);
+  a.rmax = B.rmax;
+  a.bmax = D.g_count;
+  a.hmax = B.hmax;
+  resident_prep<F>(a);
+}
+
+template <int F, int RPT>
+__global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArgs B) {
+  extern __shared__ double dyn[];
+  const int g = (int)gridDim.x, b0 = (int)blockIdx.x;
+  const int b = (g & 7) == 0 ? (b0 & 7) * (g >> 3) + (b0 >> 3) : b0;
+  for (int k = B.block_ptr[b]; k < B.block_ptr[b + 1]; ++k) {
+    const int sys = B.block_list[k];
+    const SysDesc D = B.desc[sys];
+    const int c = b - D.g_first;
+    ResPlan p{};
+    if (D.g_count > 1) {
+      p = B.plans[sys];
+    } else {
+      p.nb = 1;
+      p.R = D.neq;
+    }
+    if (p.nb == 0 && c == 0 && threadIdx.x == 0) B.st[sys].pad6 = kResDeclined;
+    if (!resident_part<RPT, 1>(p, c)) continue;
+    ResArgs a{};
+    resident_batch_mat<F>(B, D, a.A);
+    a.st = B.st + sys;
+    a.m = a.A.ad;
+    a.x = B.x + D.row_off;
+    a.b = B.b + D.row_off;
+    a.rows = B.rows + (size_t)4 * D.row_off;
+    a.part = B.part + B.part_off[sys];
+    a.part_half = res_part_half(D.g_count);
+    a.err = B.err;
+    a.gang = kResGang;
+    a.tol = B.tol;
+    a.maxit = B.maxit;
+    a.x0_zero = B.x0_zero;
+    a.stop_rule = B.stop_rule;
+    resident_solve<F, RPT, 1>(a, p, c, dyn);
+    if (ld_relaxed(B.err) != 0u) return;   // (uniform enough: a block that goes on only waits, bounded)
+    __syncthreads();                       // LDS is reused
+  }
 }
 
 }  // namespace fvc

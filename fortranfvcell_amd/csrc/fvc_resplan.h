@@ -5,6 +5,10 @@
 #pragma once
 #include <stddef.h>
 
+#include <algorithm>
+#include <cmath>
+#include <vector>
+
 #if defined(__HIPCC__)
 #define FVC_HD __host__ __device__ __forceinline__
 #else
@@ -17,9 +21,11 @@ constexpr int kResThreads = 512;     // two waves per SIMD: 256 registers a thre
 constexpr int kResMaxBlocks = 256;   // partial sums: up to four blocks per lane of a wave
 constexpr int kResMaxHalo = 2048;    // halo rows of a block
 constexpr int kResGroups = 16;       // groups of 16 blocks whose sums are added first
-// two buffers of either a word pair per (value, block), or one per (group,
-// value, block of the group) and one per (receiving group, value, group)
-constexpr int kResPartWords = 2 * 2 * 2 * kResGroups * 64;
+// The words of one buffer for the partial sums of nb blocks: a pair per
+// (value, block) up to 64 blocks, beyond that one per (group, value, block of
+// the group) and one per (receiving group, value, group).
+constexpr int res_part_half(int nb) { return nb <= 64 ? 2 * 4 * 64 : 2 * 2 * kResGroups * 64; }
+constexpr int kResPartWords = 2 * res_part_half(kResMaxBlocks);
 
 // How rows are dealt to blocks, decided on the device by resident_prep_kernel
 // (the host never sees the columns of a resident system).
@@ -198,6 +204,104 @@ inline ResShape resident_shape(int neq, int cus) {
     if (n <= (rpt < 8 ? room - room / 20 : room)) return {rpt, blocks(rpt)};
   }
   return {0, 0};
+}
+
+// ---------------------------------------------------------------- batches --
+//
+// Teams of blocks for a batch: how many rows a thread holds (one choice for
+// the launch), each system's team, and each block's systems in turn.
+struct ResBatchPlan {
+  int rpt = 0, blocks = 0;             // rpt 0: nothing to gain
+  std::vector<char> on;                // per system: solved by this launch
+  std::vector<int> first, count;       // its team
+  std::vector<int> ptr, list;          // block b runs list[ptr[b]] .. list[ptr[b + 1] - 1] in this order
+  double load = 0.0;                   // the most loaded block, us per unit of iterations
+};
+
+// us per PCG iteration at 1, 2, 4, 8 rows a thread, one block and a team
+// (MI355X, resident_shape's measurements)
+constexpr double kResIterAlone[4] = {1.3, 1.5, 1.9, 2.75}, kResIterTeam[4] = {2.8, 2.95, 3.4, 4.4};
+
+// blocks: co-resident ones.  A system's iterations are taken as
+// neq^(expo - 1) (PCG on these meshes: expo 1.5), its time as iterations
+// times the time of one, which hardly falls with more blocks: so a team is
+// as small as holds the system, and the rows per thread are those whose most
+// loaded block ends first: few systems want few rows a thread (short
+// iterations), many want eight (a third of the block time of one row).
+// Systems go longest first onto the run of blocks that is free first; runs
+// may start anywhere (256 systems of side 32 .. 512: 1.15 times the mean
+// load against 1.41 with runs at multiples of the team).
+inline ResBatchPlan plan_resident_batch(const std::vector<int> &neq, double expo, int blocks) {
+  const int n = (int)neq.size();
+  ResBatchPlan best;
+  blocks = (blocks < kResMaxBlocks ? blocks : kResMaxBlocks) & ~7;
+  if (blocks < 8) return best;
+  std::vector<double> its(n), cost(n), load;
+  std::vector<int> order, count(n), first(n), run;
+  for (int i = 0; i < n; ++i) its[i] = std::pow((double)neq[i], expo - 1.0);
+  for (int q = 0; q < 4; ++q) {
+    double total = 0.0;
+    bool all = true;
+    order.clear();
+    for (int i = 0; i < n; ++i) {
+      const long g = ((long)neq[i] + (kResThreads << q) - 1) / (kResThreads << q);
+      count[i] = g <= blocks ? (int)g : 0;
+      all = all && count[i] > 0;
+      if (!count[i]) continue;
+      cost[i] = its[i] * (g > 1 ? kResIterTeam[q] : kResIterAlone[q]);
+      total += g * cost[i];
+      order.push_back(i);
+    }
+    // (at eight rows a thread, systems that do not fit are left out)
+    if (order.empty() || (!all && q < 3) || (best.rpt && total / blocks >= best.load)) continue;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    load.assign(blocks, 0.0);
+    double longest = 0.0;
+    for (int i : order) {
+      // the run of count[i] blocks whose largest load is least: the largest
+      // load of every run by a queue of candidates
+      const int g = count[i];
+      int at = 0;
+      double when = -1.0;
+      run.clear();
+      size_t head = 0;
+      for (int k = 0; k < blocks; ++k) {
+        while (run.size() > head && load[run.back()] <= load[k]) run.pop_back();
+        run.push_back(k);
+        if (run[head] <= k - g) ++head;
+        if (k + 1 >= g && (when < 0.0 || load[run[head]] < when)) {
+          when = load[run[head]];
+          at = k + 1 - g;
+        }
+      }
+      first[i] = at;
+      for (int k = at; k < at + g; ++k) load[k] = when + cost[i];
+      longest = longest < when + cost[i] ? when + cost[i] : longest;
+    }
+    if (best.rpt && longest >= best.load) continue;
+    best.rpt = 1 << q;
+    best.load = longest;
+    best.first = first;
+    best.count = count;
+    best.list = order;
+  }
+  if (!best.rpt) return best;
+  best.on.assign(n, 0);
+  std::vector<std::vector<int>> lists(blocks);
+  int used = 0;
+  for (int i : best.list) {
+    best.on[i] = 1;
+    used = used < best.first[i] + best.count[i] ? best.first[i] + best.count[i] : used;
+    for (int k = best.first[i]; k < best.first[i] + best.count[i]; ++k) lists[k].push_back(i);
+  }
+  best.blocks = (used + 7) & ~7;
+  best.list.clear();
+  best.ptr.assign(1, 0);
+  for (int k = 0; k < best.blocks; ++k) {
+    best.list.insert(best.list.end(), lists[k].begin(), lists[k].end());
+    best.ptr.push_back((int)best.list.size());
+  }
+  return best;
 }
 
 }  // namespace fvc

@@ -429,8 +429,11 @@ int run_resident(DevState &d, const SolveIn &in, KState *st, unsigned *ctr, res_
       a.plan = plan;
       a.rows = rows;
       a.part = part;
+      a.part_half = kResPartWords / 2;
+      a.err = reinterpret_cast<unsigned *>(&st->next);
+      a.gang = 1;
       hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, (int)kCtrWords, st, 1);
-      ResPrepArgs pa{in.A, plan, part, rows, kResThreads * sh.rpt, sh.blocks, hmax};
+      ResPrepArgs pa{in.A, plan, part, rows, kResPartWords, kResThreads * sh.rpt, sh.blocks, hmax};
       hipLaunchKernelGGL(resident_prep_kernel<F>, dim3(std::min((neq + 255) / 256, 4 * d.cus)), dim3(256), 0, s, pa);
     }
     HIPCHK(hipGetLastError());
@@ -1628,6 +1631,111 @@ int dot_impl(const double *a, const double *b, int n, double *result, bool on_de
 
 // ------------------------------------------------------------- batches --
 
+// Systems lo .. hi - 1 of an FP64 batch on chip (fvc_resident.h): solves what
+// fits, in one launch, and adds to `todo` the systems it did not solve.
+// Measured on MI355X against the streaming kernels below: 48 systems of side
+// 32 .. 160 40.4 -> 4.6 ms; 256 systems of side 32 .. 512 (10.2M rows) 835 ms at
+// the tuned launches -> 115.
+template <int F>
+int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_off, const std::vector<int> &val_off, int w,
+                       const double *ad, const double *av, const int *ia, const int *ja, double *x, const double *b,
+                       double tol, int maxit, const fvc_options &o, std::vector<KState> &host_st,
+                       std::vector<int> &todo, hipStream_t s) {
+  const int nsys = hi - lo;
+  const auto leave = [&] {
+    for (int i = lo; i < hi; ++i) todo.push_back(i);
+    return FVC_OK;
+  };
+  if constexpr (!resident_format(F)) {
+    return leave();
+  } else {
+    static const void *const fns[4] = {(const void *)&resident_batch_kernel<F, 1>, (const void *)&resident_batch_kernel<F, 2>,
+                                       (const void *)&resident_batch_kernel<F, 4>, (const void *)&resident_batch_kernel<F, 8>};
+    std::vector<int> sizes(nsys);
+    for (int i = 0; i < nsys; ++i) sizes[i] = row_off[lo + i + 1] - row_off[lo + i];
+    const ResBatchPlan plan = plan_resident_batch(sizes, o.batch_work_exp10 > 0 ? o.batch_work_exp10 / 10.0 : 1.5, d.cus);
+    if (plan.rpt == 0) return leave();
+    // one block per CU: two (which one row a thread would allow) hold each
+    // other up (48 systems of side 32 .. 160: 9.4 ms on 512 blocks of one row a
+    // thread, 4.3 on 208 of four)
+    const void *fn = fns[plan.rpt == 1 ? 0 : plan.rpt == 2 ? 1 : plan.rpt == 4 ? 2 : 3];
+    const int hmax = res_max_halo(FVC_PCG, plan.rpt);
+    const size_t lds = res_lds_bytes(FVC_PCG, plan.rpt, hmax);
+    HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int occ = 0;
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, kResThreads, lds));
+    if ((long)occ * d.cus < plan.blocks) return leave();
+    // one upload: descriptions, offsets of the partial sums, the systems of
+    // several blocks, the blocks' lists
+    std::vector<int> multi, part_off(nsys, 0);
+    size_t npart = 0;
+    for (int i = 0; i < nsys; ++i) {
+      if (!plan.on[i] || plan.count[i] < 2) continue;
+      multi.push_back(i);
+      part_off[i] = (int)npart;
+      npart += 2 * (size_t)res_part_half(plan.count[i]);
+      if (npart > INT_MAX / 2) return leave();
+    }
+    std::vector<int> up;
+    const auto put = [&](const int *p, size_t m) {
+      const size_t at = up.size();
+      up.insert(up.end(), p, p + m);
+      return at;
+    };
+    for (int i = 0; i < nsys; ++i) {
+      const SysDesc D{row_off[lo + i], sizes[i], plan.first[i], plan.count[i], val_off[lo + i], row_off[lo + i] + lo + i};
+      put(reinterpret_cast<const int *>(&D), sizeof D / sizeof(int));
+    }
+    const size_t at_part = put(part_off.data(), part_off.size()), at_multi = put(multi.data(), multi.size()),
+                 at_ptr = put(plan.ptr.data(), plan.ptr.size()), at_list = put(plan.list.data(), plan.list.size());
+    const size_t n = (size_t)row_off[hi];
+    const size_t nclear = (size_t)nsys * (sizeof(ResPlan) / sizeof(unsigned)) + 1;
+    const size_t bytes = align_up(up.size() * sizeof(int)) + align_up(nsys * sizeof(KState)) +
+                         align_up(nclear * sizeof(unsigned)) + align_up(npart * sizeof(res_word)) +
+                         align_up(4 * n * sizeof(res_word)) + 4096;
+    int rc = ensure_arena(d, bytes);
+    if (rc) return rc;
+    Carve cv{d.arena, bytes};
+    int *dup = cv.take<int>(up.size());
+    KState *st = cv.take<KState>(nsys);
+    unsigned *clear = cv.take<unsigned>(nclear);
+    res_word *part = cv.take<res_word>(npart);
+    res_word *rows = cv.take<res_word>(4 * n);
+    if (!cv.fits()) return carve_overflow(cv);
+    HIPCHK(hipMemcpyAsync(dup, up.data(), up.size() * sizeof(int), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, clear, (int)nclear, st, nsys);
+    ResBatchArgs B{};
+    B.w = w; B.ad = ad; B.av = av; B.b = b; B.ia = ia; B.ja = ja; B.x = x;
+    B.desc = reinterpret_cast<const SysDesc *>(dup);
+    B.part_off = dup + at_part;
+    B.block_ptr = dup + at_ptr;
+    B.block_list = dup + at_list;
+    B.st = st;
+    B.err = clear;
+    B.plans = reinterpret_cast<ResPlan *>(clear + 1);
+    B.rows = rows;
+    B.part = part;
+    B.tol = tol;
+    B.maxit = maxit;
+    B.x0_zero = o.x0_rule == FVC_X0_GIVEN ? 0 : 1;
+    B.stop_rule = o.stop_rule;
+    B.rmax = kResThreads * plan.rpt;
+    B.hmax = hmax;
+    if (!multi.empty())
+      hipLaunchKernelGGL(resident_batch_prep_kernel<F>, dim3(8, (unsigned)multi.size()), dim3(256), 0, s, B, dup + at_multi);
+    HIPCHK(hipGetLastError());
+    void *params[] = {&B};
+    HIPCHK(hipLaunchKernel(fn, dim3(plan.blocks), dim3(kResThreads), params, lds, s));
+    unsigned err = 0;
+    HIPCHK(hipMemcpyAsync(host_st.data() + lo, st, nsys * sizeof(KState), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(&err, B.err, sizeof err, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    for (int i = lo; i < hi; ++i)
+      if (err || host_st[i].pad6 != kResSolved) todo.push_back(i);
+    return FVC_OK;
+  }
+}
+
 template <int F>
 int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std::vector<int> &val_off, int w,
               const double *ad, const double *av, const int *ia, const int *ja, double *x, const double *b,
@@ -1657,6 +1765,39 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
   const double expo = o.batch_work_exp10 > 0 ? o.batch_work_exp10 / 10.0 : 1.5;
   if (o.batch_rows_per_wave < 0) return fail(FVC_BAD_ARGUMENT, "batch_rows_per_wave %d", o.batch_rows_per_wave);
   const int min_rows = o.batch_rows_per_wave > 0 ? o.batch_rows_per_wave * (bs / 64) : 64;
+  std::vector<KState> host_st(nsys);
+  std::vector<int> todo;   // the systems the launches below solve
+  HIPCHK(hipEventRecord(d.ev0, s));
+  // On chip where the launch is the library's choice; options that shape it
+  // keep the kernels they were written for.
+  if (!mixed && o.engine == FVC_ENGINE_AUTO && o.recurrence == FVC_REC_FUSED && o.block_size == 0 &&
+      o.grid_blocks == 0 && o.barrier == 0 && o.batch_rows_per_wave == 0) {
+    const int per = o.batch_launch_systems > 0 ? o.batch_launch_systems : nsys;
+    for (int lo = 0; lo < nsys; lo += std::min(per, nsys - lo))
+      if ((rc = run_resident_batch<F>(d, lo, lo + std::min(per, nsys - lo), row_off, val_off, w, ad, av, ia, ja, x, b, tol,
+                                      maxit, o, host_st, todo, s)))
+        return rc;
+  } else {
+    for (int i = 0; i < nsys; ++i) todo.push_back(i);
+  }
+  auto close = [&](int flags) -> int {   // the time and every system's statistics
+    HIPCHK(hipEventRecord(d.ev1, s));
+    HIPCHK(hipEventSynchronize(d.ev1));
+    float ms = 0.f;
+    HIPCHK(hipEventElapsedTime(&ms, d.ev0, d.ev1));
+    int worst = S_OK;
+    for (int i = 0; i < nsys; ++i) {
+      if (stats) {
+        fill_stats(&stats[i], host_st[i], FVC_PCG, true, ms, 0, bs, flags);
+        if (mixed) stats[i].inner_iterations = host_st[i].cycle;
+      }
+      if (host_st[i].status != S_OK && worst == S_OK) worst = host_st[i].status;
+    }
+    if (worst != S_OK) return fail(worst, "a system of the batch did not converge");
+    return FVC_OK;
+  };
+  const int ntodo = (int)todo.size();
+  if (ntodo == 0) return close(0);
   const size_t n = (size_t)total;
   const size_t nv = (size_t)val_off[nsys];   // stored off-diagonal values
   size_t bytes = align_up(((size_t)wave * kCtrWords + cap) * sizeof(unsigned)) + align_up((size_t)wave * sizeof(KState)) +
@@ -1711,7 +1852,6 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
   B.partials = partials;
   B.desc = ddesc;
   B.block_ptr = dplan;
-  HIPCHK(hipEventRecord(d.ev0, s));
   if (mixed) {
     if (B.jo) hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(64), 0, s, reinterpret_cast<unsigned *>(B.wide), 1, st, 0);
     hipLaunchKernelGGL(batch_scale_kernel<F>, dim3((total + 255) / 256), dim3(256), 0, s, B, nsys, d_row_off,
@@ -1724,16 +1864,17 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
       if (h_wide) B.jo = nullptr;   // keep the int32 columns
     }
   }
-  std::vector<KState> host_st(nsys);
-  for (int s0 = 0; s0 < nsys; s0 += wave) {
-    const int m = std::min(wave, nsys - s0);
+  std::vector<KState> wave_st(wave);
+  for (int s0 = 0; s0 < ntodo; s0 += wave) {
+    const int m = std::min(wave, ntodo - s0);
     std::vector<int> sizes(m);
-    for (int i = 0; i < m; ++i) sizes[i] = row_off[s0 + i + 1] - row_off[s0 + i];
+    for (int i = 0; i < m; ++i) sizes[i] = row_off[todo[s0 + i] + 1] - row_off[todo[s0 + i]];
     const BlockPlan plan = plan_blocks(sizes, cap, expo, min_rows);
     std::vector<SysDesc> desc(m);
-    for (int i = 0; i < m; ++i)
-      desc[i] = SysDesc{row_off[s0 + i], sizes[i], plan.first[i], plan.count[i], val_off[s0 + i],
-                        row_off[s0 + i] + s0 + i};
+    for (int i = 0; i < m; ++i) {
+      const int sys = todo[s0 + i];
+      desc[i] = SysDesc{row_off[sys], sizes[i], plan.first[i], plan.count[i], val_off[sys], row_off[sys] + sys};
+    }
     const int G = plan.blocks;
     // block_ptr (G + 1 entries) then block_list (one per block of a group,
     // one per packed system: at most cap + m)
@@ -1747,28 +1888,16 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
     hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, wave * kCtrWords + cap, st, m);
     HIPCHK(hipGetLastError());
     if ((rc = launch(fn, true, G, bs, B, s))) return rc;
-    HIPCHK(hipMemcpyAsync(host_st.data() + s0, st, m * sizeof(KState), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(wave_st.data(), st, m * sizeof(KState), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));   // desc/hplan host buffers are reused next wave
+    for (int i = 0; i < m; ++i) host_st[todo[s0 + i]] = wave_st[i];
     // every system's barrier words in one copy, then its error word
     std::vector<unsigned> hctr((size_t)m * kCtrWords);
     HIPCHK(hipMemcpy(hctr.data(), ctr, hctr.size() * sizeof(unsigned), hipMemcpyDeviceToHost));
     for (int i = 0; i < m; ++i)
       if (hctr[(size_t)i * kCtrWords + kCtrErr]) return fail(FVC_DEVICE_ERROR, "batched solve: a grid barrier wait expired");
   }
-  HIPCHK(hipEventRecord(d.ev1, s));
-  HIPCHK(hipEventSynchronize(d.ev1));
-  float ms = 0.f;
-  HIPCHK(hipEventElapsedTime(&ms, d.ev0, d.ev1));
-  int worst = S_OK;
-  for (int i = 0; i < nsys; ++i) {
-    if (stats) {
-      fill_stats(&stats[i], host_st[i], FVC_PCG, true, ms, 0, bs, B.jo ? FVC_FLAG_COL16 : 0);
-      if (mixed) stats[i].inner_iterations = host_st[i].cycle;
-    }
-    if (host_st[i].status != S_OK && worst == S_OK) worst = host_st[i].status;
-  }
-  if (worst != S_OK) return fail(worst, "a system of the batch did not converge");
-  return FVC_OK;
+  return close(B.jo ? FVC_FLAG_COL16 : 0);
 }
 
 // Batched Jacobi-PCG over ELLPACK (matriz 4, width w) or CSRD (matriz 1,

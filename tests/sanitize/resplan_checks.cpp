@@ -71,8 +71,57 @@ static void check_plan(const ResPlan &p, int n, int rmax, int bmax, int hmax) {
   }
 }
 
+// Every system that takes part has its team of blocks, the blocks' lists hold
+// it once per block of the team, and going through the lists never waits in a
+// ring.
+static void check_batch(const std::vector<int> &neq, int cap) {
+  const ResBatchPlan p = plan_resident_batch(neq, 1.5, cap);
+  if (p.rpt == 0) return;
+  ++plans;
+  const int n = (int)neq.size();
+  CHECK(p.blocks <= cap && p.blocks % 8 == 0 && (int)p.ptr.size() == p.blocks + 1, "%d blocks of %d", p.blocks, cap);
+  std::vector<int> seen(n, 0), at(p.blocks);
+  for (int b = 0; b < p.blocks; ++b) {
+    at[b] = p.ptr[b];
+    for (int k = p.ptr[b]; k < p.ptr[b + 1]; ++k) {
+      const int i = p.list[k];
+      CHECK(p.on[i] && b >= p.first[i] && b < p.first[i] + p.count[i], "block %d runs system %d of others", b, i);
+      ++seen[i];
+    }
+  }
+  int left = 0;
+  for (int i = 0; i < n; ++i) {
+    if (!p.on[i]) { CHECK(seen[i] == 0, "system %d", i); continue; }
+    ++left;
+    CHECK(seen[i] == p.count[i] && p.first[i] + p.count[i] <= p.blocks, "system %d: %d of %d blocks", i, seen[i], p.count[i]);
+    CHECK((long)p.count[i] * p.rpt * kResThreads >= neq[i], "system %d does not fit its team", i);
+  }
+  for (bool moved = true; moved;) {
+    moved = false;
+    for (int b = 0; b < p.blocks; ++b) {
+      if (at[b] >= p.ptr[b + 1]) continue;
+      const int i = p.list[at[b]];
+      if (p.first[i] != b) continue;
+      bool ready = true;
+      for (int k = b; k < b + p.count[i]; ++k) ready = ready && at[k] < p.ptr[k + 1] && p.list[at[k]] == i;
+      if (!ready) continue;
+      for (int k = b; k < b + p.count[i]; ++k) ++at[k];
+      --left;
+      moved = true;
+    }
+  }
+  CHECK(left == 0, "%d systems wait for each other", left);
+}
+
 int main() {
-  const int sizes[] = {9, 64, 513, 1000, 2047, 4096, 5003, 12707, 33333, 65536};
+  unsigned seed = 1;
+  const auto rnd = [&] { return (seed = seed * 1664525u + 1013904223u) >> 8; };
+  for (int t = 0; t < 60; ++t) {
+    std::vector<int> neq(1 + rnd() % (t < 30 ? 40 : 400));
+    for (int &v : neq) v = 1 + (int)std::pow(10.0, (rnd() % 1000) / 1000.0 * (t % 3 == 0 ? 3.0 : 5.7));
+    for (int cap : {256, 304, 64, 8}) check_batch(neq, cap);
+  }
+  const int sizes[] = {9, 64, 513, 2047, 4096, 5003, 12707, 40000};
   for (int n : sizes)
     for (int rmax : {512, 1024, 4096})
       for (int bmax : {8, 40, 256}) {
@@ -81,7 +130,7 @@ int main() {
           ResPlan p{};
           p.H = H;
           if (H < n && res_strips(n, H, rmax, bmax, hmax, p)) check_plan(p, n, rmax, bmax, hmax);
-          for (int ntx = 1; ntx <= 12; ++ntx)
+          for (int ntx = 1; ntx <= 12; ntx += 1 + ntx / 4)
             for (int hx : {1, 3, 4}) {
               ResPlan q{};
               q.H = H;

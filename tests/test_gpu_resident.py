@@ -118,3 +118,45 @@ def test_resident_reports_breakdown_and_nonfinite(fvc):
                     assert (sa["status"], sa["iterations"]) == (sk["status"], sk["iterations"]), (n, code, stop)
                     if sa["status"] > 1:
                         assert sa["engine"] == fvc.ENGINE_KERNELS
+
+
+@pytest.mark.parametrize("given", [False, True], ids=["x0_zero", "x0_given"])
+def test_resident_batch_beside_systems_that_do_not_fit(fvc, given):
+    """One launch takes the systems that fit, whatever their team (one block,
+    a few, many), and the streaming kernels the others (a random numbering)."""
+    sides = [1, 3, 8, 22, 23, 33, 46, 64, 91, 130, 201]
+    systems = [P.pressure_system(P.quad_mesh(n), k=P.lognormal_k(n, n * n), seed=n, pin="penalty" if n > 1 else "identity")
+               for n in sides]
+    s = P.config_pressure_lognormal(60)
+    p = np.random.default_rng(5).permutation(s.neq)
+    q = np.empty(s.neq, np.int64)
+    q[p] = np.arange(s.neq)
+    systems.insert(4, P.System(s.neq, s.w, s.ad[p], s.off[p], np.where(s.nbr[p] >= 0, q[np.maximum(s.nbr[p], 0)], -1), s.b[p]))
+    systems[0].b[:] = 3.0
+    for lay, cat in ((P.to_ell, fvc.concat_ell), (P.to_csrd, fvc.concat_csrd)):
+        batch = cat([lay(t) for t in systems])
+        n = int(batch["row_offsets"][-1])
+        x0 = np.random.default_rng(1).normal(size=n) if given else None
+        if given:
+            # where the 1e60 pin holds it: off it, the pinned row's residual is 1e60
+            # and no recursive residual of the solve knows what rounding left of it
+            x0[batch["ad"] > 1e50] = 0.0
+        kw = dict(tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_GIVEN if given else fvc.X0_ZERO)
+        print(f"resident batch of {len(systems)} systems {lay.__name__} given={given}", flush=True)
+        x, sts = fvc.solve_batch(batch, x0=x0, **kw)
+        xs, ss = fvc.solve_batch(batch, x0=x0, block_size=256, **kw)
+        ro = batch["row_offsets"]
+        for i, t in enumerate(systems):
+            xi, yi = x[ro[i]:ro[i + 1]], xs[ro[i]:ro[i + 1]]
+            assert sts[i]["status"] == ss[i]["status"] == 0, (i, sts[i], ss[i])
+            assert np.linalg.norm(t.b - P.scipy_csr(t) @ xi) <= 1.01e-10 * np.linalg.norm(t.b), i
+            assert np.linalg.norm(xi - yi) <= 1e-8 * np.linalg.norm(yi), i
+
+
+def test_resident_batch_maxit(fvc):
+    systems = [P.pressure_system(P.quad_mesh(n), seed=n) for n in (10, 40, 90)]
+    batch = fvc.concat_ell([P.to_ell(s) for s in systems])
+    x, sts = fvc.solve_batch(batch, tol=1e-10, maxit=5, stop_rule=fvc.STOP_RELRES)
+    xs, ss = fvc.solve_batch(batch, tol=1e-10, maxit=5, stop_rule=fvc.STOP_RELRES, block_size=256)
+    assert [(s["status"], s["iterations"]) for s in sts] == [(s["status"], s["iterations"]) for s in ss] == [(1, 5)] * 3
+    assert np.linalg.norm(x - xs) <= 1e-12 * np.linalg.norm(xs)
