@@ -54,14 +54,15 @@
   P __global__ void fvc::batch_scale_kernel<F>(fvc::BatchArgs, int, const int *, const int *);
 #define FVCI_RES_R(P, F, R)                                      \
   P __global__ void fvc::resident_kernel<F, R, 1>(fvc::ResArgs); \
-  P __global__ void fvc::resident_kernel<F, R, 2>(fvc::ResArgs);
+  P __global__ void fvc::resident_kernel<F, R, 2>(fvc::ResArgs); \
+  P __global__ void fvc::resident_kernel<F, R, 3>(fvc::ResArgs);
+#define FVCI_RES_RB(P, F, R)                                          \
+  P __global__ void fvc::resident_batch_kernel<F, R, 1>(fvc::ResBatchArgs); \
+  P __global__ void fvc::resident_batch_kernel<F, R, 3>(fvc::ResBatchArgs);
 #define FVCI_RES(P, F)                                            \
   P __global__ void fvc::resident_prep_kernel<F>(fvc::ResPrepArgs); \
   P __global__ void fvc::resident_batch_prep_kernel<F>(fvc::ResBatchArgs, const int *); \
-  P __global__ void fvc::resident_batch_kernel<F, 1>(fvc::ResBatchArgs); \
-  P __global__ void fvc::resident_batch_kernel<F, 2>(fvc::ResBatchArgs); \
-  P __global__ void fvc::resident_batch_kernel<F, 4>(fvc::ResBatchArgs); \
-  P __global__ void fvc::resident_batch_kernel<F, 8>(fvc::ResBatchArgs); \
+  FVCI_RES_RB(P, F, 1) FVCI_RES_RB(P, F, 2) FVCI_RES_RB(P, F, 4) FVCI_RES_RB(P, F, 8) \
   FVCI_RES_R(P, F, 1) FVCI_RES_R(P, F, 2) FVCI_RES_R(P, F, 4) FVCI_RES_R(P, F, 8)
 #define FVCI_COLOFF(P, W) P __global__ void fvc::col_offsets_kernel<W>(int, const int *, const float *, short *, int *);
 

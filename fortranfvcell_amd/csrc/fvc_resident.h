@@ -1,4 +1,5 @@
-// fvc_resident.h -- PCG and BiCGSTAB with the whole system held on chip.
+// fvc_resident.h -- PCG, BiCGSTAB and mixed PCG with the whole system held on
+// chip.
 //
 // One launch solves the system: every block loads its rows' matrix entries
 // once into registers and keeps its rows of every Krylov vector there too
@@ -30,6 +31,8 @@
 #pragma once
 #include <limits.h>
 #include <stddef.h>
+
+#include <type_traits>
 
 #include "fvc_batch.h"
 #include "fvc_krylov.h"
@@ -198,11 +201,11 @@ __device__ __forceinline__ double res_lane(double v, int lane) {
   return __builtin_bit_cast(double, ((res_word)hi << 32) | lo);
 }
 
-// Waits for up to E doubles, at(q) being the address of the q-th or null;
+// Waits for up to E doubles (or floats, a word each), at(q) being the address of the q-th or null;
 // all loads of a poll are issued together.  False if the wait expired, after
 // `limit` polls or when another wait did (*err).
-template <int E, class At>
-__device__ __forceinline__ bool res_wait(unsigned ep, double *v, unsigned limit, const unsigned *err, At &&at) {
+template <int E, class T, class At>
+__device__ __forceinline__ bool res_wait(unsigned ep, T *v, unsigned limit, const unsigned *err, At &&at) {
   res_word lo[E], hi[E];
   for (unsigned spins = 0;;) {
 #pragma unroll
@@ -211,7 +214,7 @@ __device__ __forceinline__ bool res_wait(unsigned ep, double *v, unsigned limit,
       lo[q] = hi[q] = ep;
       if (p) {
         lo[q] = res_load(p);
-        hi[q] = res_load(p + 1);
+        if constexpr (sizeof(T) == 8) hi[q] = res_load(p + 1);
       }
     }
     bool ok = true;
@@ -225,7 +228,10 @@ __device__ __forceinline__ bool res_wait(unsigned ep, double *v, unsigned limit,
     }
   }
 #pragma unroll
-  for (int q = 0; q < E; ++q) v[q] = res_get(lo[q], hi[q]);
+  for (int q = 0; q < E; ++q) {
+    if constexpr (sizeof(T) == 8) v[q] = res_get(lo[q], hi[q]);
+    else v[q] = __builtin_bit_cast(float, (unsigned)(lo[q] >> 32));
+  }
   return true;
 }
 
@@ -242,19 +248,18 @@ struct ResArgs {
   int part_half;
   int gang;                // how many times longer the first exchange may take
   double tol;
+  double delta;            // mixed: residual drop that triggers an FP64 update
+  int max_inner;           // mixed: FP32 iterations between updates, at most
   int maxit, x0_zero, stop_rule;
 };
 
-template <int F, int RPT>
-struct Resident {
-  static constexpr int NT = kResThreads, NW = F == F_ELL3 ? 3 : 4, RB = NT * RPT;
+// A block's place among the others and its exchanges with them.
+struct ResNet {
+  static constexpr int NT = kResThreads;
   static constexpr int HE = 3;   // halo entries a thread waits for at once
 
   const ResArgs &a;
   ResMap map;
-  double *win;             // LDS: RB + nh
-  double *own;             // LDS: x, then the shadow residual (RB each)
-  double *hs;              // LDS: the halo rows' vectors, nh each
   int *row;                // LDS: global row of each own row, or -1
   int *hrow;               // LDS: global row of each halo entry, or -1
   double *red;             // LDS: kMaxK * kMaxWaves
@@ -262,76 +267,40 @@ struct Resident {
   int *bad;                // LDS
   int nh, nb;
   unsigned ep = 0;
-  double av[RPT][NW], dm[RPT];
-  unsigned idx[RPT][2];
-  unsigned pub = 0;        // bit k: another block reads row k
+  unsigned pub = 0;        // bit k: another block reads the thread's row k
 
-  __device__ __forceinline__ Resident(const ResArgs &args) : a(args) {}
+  __device__ __forceinline__ ResNet(const ResArgs &args) : a(args) {}
 
-  __device__ __forceinline__ double *state(int q) const { return hs + (size_t)q * nh; }
-
-  // Loads the matrix rows.  False where a column is outside the window.
-  __device__ __forceinline__ bool load_rows() {
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < RPT; ++k) {
-      const int l = (int)threadIdx.x + k * NT;
-      const int i = map.own(l);
-      row[l] = i;
-      dm[k] = 1.0;
-      int s[4] = {l, l, l, l};
-#pragma unroll
-      for (int e = 0; e < NW; ++e) av[k][e] = 0.0;
-      if (i >= 0) {
-        if (nb > 1 && map.edge(l)) pub |= 1u << k;
-        dm[k] = a.A.ad[i];
-        if constexpr (F == F_CSRD) {
-          const int k1 = a.A.ia[i] - 1, cnt = a.A.ia[i + 1] - 1 - k1;
-          if (cnt > NW) ok = false;
-#pragma unroll
-          for (int e = 0; e < NW; ++e)
-            if (e < cnt) {
-              av[k][e] = a.A.av[k1 + e];
-              s[e] = map.slot(a.A.ja[k1 + e] - 1, RB);
-            }
-        } else {
-#pragma unroll
-          for (int e = 0; e < NW; ++e) {
-            av[k][e] = a.A.av[(size_t)NW * i + e];
-            // padding multiplies the row's own operand by its zero
-            if (av[k][e] != 0.0) s[e] = map.slot(a.A.ja[(size_t)NW * i + e] - 1, RB);
-          }
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (s[e] < 0) {
-          ok = false;
-          s[e] = l;
-        }
-      }
-      idx[k][0] = (unsigned)s[0] | ((unsigned)s[1] << 16);
-      idx[k][1] = (unsigned)s[2] | ((unsigned)s[3] << 16);
-    }
-    return ok;
+  // The words of the rows in one buffer: a pair per double, one per float.
+  template <class T>
+  __device__ __forceinline__ res_word *row_words(unsigned e, int j) const {
+    return a.rows + (size_t)(e & 1) * 2 * a.A.neq + (sizeof(T) / 4) * (size_t)j;
+  }
+  template <class T>
+  __device__ __forceinline__ void publish(int k, T v) const {
+    if (!(pub >> k & 1u)) return;
+    res_word *to = row_words<T>(ep + 1, row[threadIdx.x + k * NT]);
+    if constexpr (sizeof(T) == 8) res_put(to, v, ep + 1);
+    else res_store(to, ((res_word)__builtin_bit_cast(unsigned, v) << 32) | (ep + 1));
   }
 
-  // (A u)_k from the window; own = the row's own operand.  The reference's
-  // order of the products, as RowRegs / row_apply.
-  __device__ __forceinline__ double apply(int k, double own) const {
-    const double x0 = win[idx[k][0] & 0xffffu], x1 = win[idx[k][0] >> 16], x2 = win[idx[k][1] & 0xffffu];
-    const double t5 = dm[k] * own;
-    if constexpr (F == F_ELL3) {
-      return ((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + t5;
-    } else {
-      const double x3 = win[idx[k][1] >> 16];
-      if constexpr (F == F_CSRD) return (((t5 + av[k][0] * x0) + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3;
-      else return (((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3) + t5;
+  // The K sums of up to 16 members, 16 lanes to a value.
+  template <int K, int E>
+  __device__ __forceinline__ void group_sums(const res_word *from, int members, unsigned limit, double *tot) {
+    const int lane = (int)threadIdx.x & (kWave - 1);
+    double g[E];
+    const bool in = (lane & 15) < members;
+    if (!res_wait<E>(ep, g, limit, a.err, [&](int q) -> const res_word * {
+          const int e = lane + q * kWave;
+          return in && e < 16 * K ? from + 2 * (size_t)e : nullptr;
+        }))
+      *bad = 1;
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+      const double s = res_row_sum(in && lane + q * kWave < 16 * K ? g[q] : 0.0);
+#pragma unroll
+      for (int k = 4 * q; k < (K < 4 * q + 4 ? K : 4 * q + 4); ++k) tot[k] = res_lane(s, 16 * (k & 3) + 15);
     }
-  }
-
-  __device__ __forceinline__ void publish(int k, double v) const {
-    if (pub >> k & 1u) res_put(a.rows + 2 * ((size_t)((ep + 1) & 1) * a.A.neq + row[threadIdx.x + k * NT]), v, ep + 1);
   }
 
   // One exchange: the block's K sums to every block and theirs here, added in
@@ -339,8 +308,8 @@ struct Resident {
   // nh entries; null: none); then epi(totals) on thread 0.  publish() goes
   // before.  Some waves wait for the sums and the others for the halo.
   // False if a wait expired.
-  template <int K, class Epi>
-  __device__ __forceinline__ bool exchange(const double *v, double *hdst, Epi &&epi) {
+  template <int K, class T, class Epi>
+  __device__ __forceinline__ bool exchange(const double *v, T *hdst, Epi &&epi) {
     ++ep;
     const int t = (int)threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
 #pragma unroll
@@ -349,7 +318,8 @@ struct Resident {
       if (lane == kWave - 1) red[k * kMaxWaves + wid] = s;
     }
     lds_barrier();
-    static_assert(K <= 4, "16 lanes per value");
+    static_assert(K <= kResSums, "a lane adds at most two of the groups' sums");
+    constexpr int E = K > 4 ? 2 : 1;   // the fifth value goes with the first 16 lanes
     res_word *part = a.part + (size_t)(ep & 1) * (size_t)a.part_half;
     // a block may come to its first exchange long before the others
     const unsigned limit = ep == 1 ? kResSpin * (unsigned)a.gang : kResSpin;
@@ -368,7 +338,7 @@ struct Resident {
         own = q[0];
 #pragma unroll
         for (int w = 1; w < NT / kWave; ++w) own += q[w];
-        const int to = wide ? (map.c >> 4) * kWave + lane * 16 + (map.c & 15) : lane * kWave + map.c;
+        const int to = wide ? (map.c >> 4) * kResGroupSums + lane * 16 + (map.c & 15) : lane * kWave + map.c;
         if (nb > 1) res_put(part + 2 * (size_t)to, own, ep);
       }
       double tot[K];
@@ -384,40 +354,30 @@ struct Resident {
 #pragma unroll
         for (int k = 0; k < K; ++k) tot[k] = res_lane(res_wave_sum(lane < nb ? pv[k] : 0.0), kWave - 1);
       } else {
-        double g[1];
-        const bool mine = lane < 16 * K && (lane & 15) < (nb + 15) / 16;
-        const res_word *from = part + 2 * (size_t)(kResGroups * kWave + (map.c >> 4) * kWave + lane);
-        if (!res_wait<1>(ep, g, limit, a.err, [&](int) { return mine ? from : nullptr; })) *bad = 1;
-        const double s = res_row_sum(mine ? g[0] : 0.0);
-#pragma unroll
-        for (int k = 0; k < K; ++k) tot[k] = res_lane(s, 16 * k + 15);
+        group_sums<K, E>(part + 2 * (size_t)(kResGroups + (map.c >> 4)) * kResGroupSums, (nb + 15) / 16, limit, tot);
       }
       if (lane == 0) epi(tot);
     } else if (leads && wid == 1) {
-      double g[1];
       const int grp = map.c >> 4;
-      const bool mine = lane < 16 * K && (lane & 15) < nb - 16 * grp;
-      const res_word *from = part + 2 * (size_t)(grp * kWave + lane);
-      if (!res_wait<1>(ep, g, limit, a.err, [&](int) { return mine ? from : nullptr; })) *bad = 1;
-      const double s = res_row_sum(mine ? g[0] : 0.0);
-      double tot = 0.0;
+      double tot[K];
+      group_sums<K, E>(part + 2 * (size_t)grp * kResGroupSums, nb - 16 * grp, limit, tot);
+      // lane (value, group): that group's copy, all in one store (everyone waits
+      // for this wave: a store per value was 1.3 us slower at 256 blocks)
+      double mine = 0.0;
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const double sk = res_lane(s, 16 * k + 15);
-        if (lane >> 4 == k) tot = sk;
-      }
-      // lane (value, group): that group's copy
-      if (lane < 16 * K && (lane & 15) < (nb + 15) / 16)
-        res_put(part + 2 * (size_t)(kResGroups * kWave + (lane & 15) * kWave + (lane & 48) + grp), tot, ep);
+      for (int k = 0; k < (K < 4 ? K : 4); ++k)
+        if (lane >> 4 == k) mine = tot[k];
+      res_word *to = part + 2 * (size_t)((kResGroups + (lane & 15)) * kResGroupSums + grp);
+      if (lane < 16 * K && (lane & 15) < (nb + 15) / 16) res_put(to + 2 * (lane & 48), mine, ep);
+      if (K > 4 && lane < (nb + 15) / 16) res_put(to + 2 * 64, tot[K - 1], ep);
     } else if (nb > 1 && hdst && wid >= waiting) {
-      const res_word *rows = a.rows + (size_t)(ep & 1) * 2 * a.A.neq;
       const int ht = NT - waiting * kWave, h0 = t - waiting * kWave;
       auto from = [&](int h) -> const res_word * {
         const int j = h < nh ? hrow[h] : -1;
-        return j >= 0 ? rows + 2 * (size_t)j : nullptr;
+        return j >= 0 ? row_words<T>(ep, j) : nullptr;
       };
       for (int base = 0; base < nh; base += ht * HE) {
-        double hv[HE];
+        T hv[HE];
         const bool few = nh - base <= ht;
         const bool ok = few ? res_wait<1>(ep, hv, limit, a.err, [&](int) { return from(base + h0); })
                             : res_wait<HE>(ep, hv, limit, a.err, [&](int q) { return from(base + h0 + q * ht); });
@@ -439,6 +399,114 @@ struct Resident {
       return false;
     }
     return true;
+  }
+
+  // Block 0 writes the state, all of it but `next`, which is a solve's err
+  // word (cleared before the launch; one block alone never waits).
+  __device__ __forceinline__ void outcome(int how) {
+    if (map.c != 0) return;
+    if (threadIdx.x == 0) {
+      S->pad6 = how;
+      S->next = 0;
+    }
+    lds_barrier();
+    constexpr int skip = offsetof(KState, next) / sizeof(unsigned);
+    for (int q = (int)threadIdx.x; q < (int)(sizeof(KState) / sizeof(unsigned)); q += NT)
+      if (q != skip || nb == 1)
+        reinterpret_cast<unsigned *>(a.st)[q] = reinterpret_cast<const unsigned *>(S)[q];
+  }
+};
+
+// Row i's off-diagonal values and columns (0-based; -1: none there, and the
+// value 0, which then multiplies the row's own operand); i < 0: no row.
+// False if the row has more than fit.
+template <int F>
+__device__ __forceinline__ bool res_row(const Mat &A, int i, double *v, int *j) {
+  constexpr int NW = F == F_ELL3 ? 3 : 4;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) j[e] = -1;
+#pragma unroll
+  for (int e = 0; e < NW; ++e) v[e] = 0.0;
+  if (i < 0) return true;
+  if constexpr (F == F_CSRD) {
+    const int k1 = A.ia[i] - 1, cnt = A.ia[i + 1] - 1 - k1;
+#pragma unroll
+    for (int e = 0; e < NW; ++e)
+      if (e < cnt) {
+        v[e] = A.av[k1 + e];
+        j[e] = A.ja[k1 + e] - 1;
+      }
+    return cnt <= NW;
+  } else {
+#pragma unroll
+    for (int e = 0; e < NW; ++e) {
+      v[e] = A.av[(size_t)NW * i + e];
+      if (v[e] != 0.0) j[e] = A.ja[(size_t)NW * i + e] - 1;
+    }
+    return true;
+  }
+}
+// The window slots of those columns, two to a word, for local row l.
+__device__ __forceinline__ bool res_slots(const ResMap &map, int l, int base, const int *j, unsigned *idx) {
+  bool ok = true;
+  int s[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s[e] = j[e] < 0 ? l : map.slot(j[e], base);
+    if (s[e] < 0) {
+      ok = false;
+      s[e] = l;
+    }
+  }
+  idx[0] = (unsigned)s[0] | ((unsigned)s[1] << 16);
+  idx[1] = (unsigned)s[2] | ((unsigned)s[3] << 16);
+  return ok;
+}
+
+// The matrix rows of a block's threads in registers and the FP64 window.
+template <int F, int RPT>
+struct Resident : ResNet {
+  static constexpr int NW = F == F_ELL3 ? 3 : 4, RB = NT * RPT;
+
+  double *win;             // LDS: RB + nh
+  double *own;             // LDS: x, then the shadow residual (RB each)
+  double *hs;              // LDS: the halo rows' vectors, nh each
+  double av[RPT][NW], dm[RPT];
+  unsigned idx[RPT][2];
+
+  __device__ __forceinline__ Resident(const ResArgs &args) : ResNet(args) {}
+
+  __device__ __forceinline__ double *state(int q) const { return hs + (size_t)q * nh; }
+
+  // Loads the matrix rows.  False where a column is outside the window.
+  __device__ __forceinline__ bool load_rows() {
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int l = (int)threadIdx.x + k * NT;
+      const int i = map.own(l);
+      row[l] = i;
+      dm[k] = i >= 0 ? a.A.ad[i] : 1.0;
+      if (i >= 0 && nb > 1 && map.edge(l)) pub |= 1u << k;
+      int j[4];
+      ok = res_row<F>(a.A, i, av[k], j) && ok;
+      ok = res_slots(map, l, RB, j, idx[k]) && ok;
+    }
+    return ok;
+  }
+
+  // (A u)_k from the window; own = the row's own operand.  The reference's
+  // order of the products, as RowRegs / row_apply.
+  __device__ __forceinline__ double apply(int k, double own) const {
+    const double x0 = win[idx[k][0] & 0xffffu], x1 = win[idx[k][0] >> 16], x2 = win[idx[k][1] & 0xffffu];
+    const double t5 = dm[k] * own;
+    if constexpr (F == F_ELL3) {
+      return ((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + t5;
+    } else {
+      const double x3 = win[idx[k][1] >> 16];
+      if constexpr (F == F_CSRD) return (((t5 + av[k][0] * x0) + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3;
+      else return (((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3) + t5;
+    }
   }
 
   // r = b - A x0 on the block's rows, x0 read from memory.
@@ -488,7 +556,7 @@ struct Resident {
       v[1] += ri * ri;
     }
     KState *s = S;
-    if (!exchange<2>(v, nullptr, [s](const double *tot) {
+    if (!exchange<2, double>(v, nullptr, [s](const double *tot) {
           s->energy = tot[0];
           s->res2 = tot[1];
         }))
@@ -497,18 +565,6 @@ struct Resident {
     for (int k = 0; k < RPT; ++k)
       if (row[t + k * NT] >= 0) a.x[row[t + k * NT]] = x[k * NT];
     outcome(kResSolved);
-  }
-
-  // Block 0 writes the state, all of it but `next`, which is a solve's err
-  // word (cleared before the launch; one block alone never waits).
-  __device__ __forceinline__ void outcome(int how) {
-    if (map.c != 0) return;
-    if (threadIdx.x == 0) S->pad6 = how;
-    lds_barrier();
-    constexpr int skip = offsetof(KState, next) / sizeof(unsigned);
-    for (int q = (int)threadIdx.x; q < (int)(sizeof(KState) / sizeof(unsigned)); q += NT)
-      if (q != skip || nb == 1)
-        reinterpret_cast<unsigned *>(a.st)[q] = reinterpret_cast<const unsigned *>(S)[q];
   }
 
   __device__ __forceinline__ void pcg();
@@ -693,6 +749,206 @@ __device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
   finish();
 }
 
+// Mixed precision (fvc_mixed.h): the scaled FP32 rows and the four FP32
+// vectors {r~, q, p, y} in registers; x stays in memory, where only a block's
+// own threads read it, and the FP64 matrix is read again at the reliable
+// updates, whose window of x takes the place of the FP32 one.
+template <int F, int RPT>
+struct ResidentMixed : ResNet {
+  static constexpr int NW = F == F_ELL3 ? 3 : 4, RB = NT * RPT;
+
+  double *win;             // LDS: RB + nh, as floats between the updates
+  float *hs;               // LDS: the halo rows' r~, q, p, nh each
+  float av[RPT][NW], dsq[RPT];
+  unsigned idx[RPT][2];
+
+  __device__ __forceinline__ ResidentMixed(const ResArgs &args) : ResNet(args) {}
+
+  __device__ __forceinline__ bool load_rows() {
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int l = (int)threadIdx.x + k * NT, i = map.own(l);
+      row[l] = i;
+      if (i >= 0 && nb > 1 && map.edge(l)) pub |= 1u << k;
+      const double m = i >= 0 ? a.m[i] : 1.0;
+      const double si = 1.0 / sqrt(m);
+      dsq[k] = (float)sqrt(m);
+      double v[NW];
+      int j[4];
+      ok = res_row<F>(a.A, i, v, j) && ok;
+#pragma unroll
+      for (int e = 0; e < NW; ++e) {
+        av[k][e] = j[e] >= 0 ? (float)(v[e] * si * (1.0 / sqrt(a.m[j[e]]))) : 0.0f;
+      }
+      ok = res_slots(map, l, RB, j, idx[k]) && ok;
+    }
+    return ok;
+  }
+
+  // (S A S p)_k, unit diagonal (as RowRegs32 / row_apply32)
+  __device__ __forceinline__ float apply32(int k, float own) const {
+    const float *w = reinterpret_cast<const float *>(win);
+    const float x0 = w[idx[k][0] & 0xffffu], x1 = w[idx[k][0] >> 16], x2 = w[idx[k][1] & 0xffffu];
+    if constexpr (F == F_ELL3) {
+      return ((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + own;
+    } else {
+      const float x3 = w[idx[k][1] >> 16];
+      if constexpr (F == F_CSRD) return (((own + av[k][0] * x0) + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3;
+      else return (((av[k][0] * x0 + av[k][1] * x1) + av[k][2] * x2) + av[k][3] * x3) + own;
+    }
+  }
+  // (A x)_k in FP64: the row from memory, x from the window.
+  __device__ __forceinline__ double apply64(int k, int i, double own) const {
+    double v[NW];
+    int j[4];
+    res_row<F>(a.A, i, v, j);
+    const double x0 = win[idx[k][0] & 0xffffu], x1 = win[idx[k][0] >> 16], x2 = win[idx[k][1] & 0xffffu];
+    const double t5 = a.A.ad[i] * own;
+    if constexpr (F == F_ELL3) {
+      return ((v[0] * x0 + v[1] * x1) + v[2] * x2) + t5;
+    } else {
+      const double x3 = win[idx[k][1] >> 16];
+      if constexpr (F == F_CSRD) return (((t5 + v[0] * x0) + v[1] * x1) + v[2] * x2) + v[3] * x3;
+      else return (((v[0] * x0 + v[1] * x1) + v[2] * x2) + v[3] * x3) + t5;
+    }
+  }
+
+  // x of own and halo rows into the window
+  __device__ __forceinline__ bool window_x() {
+    const int t = (int)threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int i = row[t + k * NT];
+      const double xi = i >= 0 ? a.x[i] : 0.0;
+      win[t + k * NT] = xi;
+      publish(k, xi);
+    }
+    const double none[1] = {0.0};
+    return exchange<1>(none, win + RB, [](const double *) {});
+  }
+
+  __device__ __forceinline__ void pcg() {
+    const int t = (int)threadIdx.x;
+    MixedArgs e{};
+    e.tol = a.tol;
+    e.delta = a.delta;
+    e.maxit = a.maxit;
+    e.max_inner = a.max_inner;
+    KState *st = S;
+    float *w32 = reinterpret_cast<float *>(win);
+    float *hr = hs, *hq = hs + nh, *hp = hs + 2 * nh;
+    float r[RPT], q[RPT], p[RPT], y[RPT];
+    const bool ok = load_rows();
+    for (int h = t; h < nh; h += NT) hr[h] = hq[h] = hp[h] = 0.0f;
+    double v[4] = {0.0, 0.0, 0.0, ok ? 0.0 : 1.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int i = row[t + k * NT];
+      r[k] = q[k] = p[k] = y[k] = 0.0f;
+      double bi = 0.0, ri = 0.0;
+      if (i >= 0) {
+        // (x as given is whole in memory until the first exchange is over)
+        bi = a.b[i];
+        if (a.x0_zero) {
+          a.x[i] = 0.0;
+          ri = bi;
+        } else {
+          ri = bi - row_apply<F>(a.A, i, XVec{a.x});
+        }
+        r[k] = (float)(ri * (1.0 / sqrt(a.m[i])));
+      }
+      publish(k, r[k]);
+      v[0] += (double)r[k] * (double)r[k];
+      v[1] += ri * ri;
+      v[2] += bi * bi;
+    }
+    if (!exchange<4>(v, hr, [&](const double *tot) {
+          mixed_epi(e, MX_SETUP, st, tot);
+          if (tot[3] != 0.0) st->pend = 1;
+        }))
+      return;
+    if (S->pend) return outcome(kResDeclined);
+    while (!S->done) {
+      if (S->next == MX_A) {
+        const float al = S->step_i ? 0.0f : (float)S->alpha, be = S->ni ? 0.0f : (float)S->beta;
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+          y[k] = y[k] + al * p[k];
+          r[k] = r[k] - al * q[k];
+          p[k] = r[k] + be * p[k];
+          w32[t + k * NT] = p[k];
+        }
+        for (int h = t; h < nh; h += NT) {
+          const float rh = hr[h] - al * hq[h], ph = rh + be * hp[h];
+          hr[h] = rh;
+          hp[h] = ph;
+          w32[RB + h] = ph;
+        }
+        lds_barrier();
+        double v5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+          q[k] = apply32(k, p[k]);
+          publish(k, q[k]);
+          const double rd = r[k], qd = q[k];
+          v5[0] += (double)p[k] * qd;
+          v5[1] += rd * qd;
+          v5[2] += qd * qd;
+          v5[3] += rd * rd;
+          const double ru = rd * (double)dsq[k];
+          v5[4] += ru * ru;
+        }
+        if (!exchange<5>(v5, hq, [&](const double *tot) { mixed_epi(e, MX_A, st, tot); })) return;
+        continue;
+      }
+      // a reliable update: x += S (y + alpha p), r~ = S (b - A x) in FP64
+      const float al = (float)S->alpha;
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        const int i = row[t + k * NT];
+        const float yi = y[k] + al * p[k];
+        if (i >= 0) a.x[i] = a.x[i] + (1.0 / sqrt(a.m[i])) * (double)yi;
+        y[k] = 0.0f;
+        }
+      if (!window_x()) return;
+      double v3[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        const int i = row[t + k * NT];
+        if (i >= 0) {
+          const double bi = a.b[i], ri = bi - apply64(k, i, win[t + k * NT]);
+          r[k] = (float)(ri * (1.0 / sqrt(a.m[i])));
+          v3[1] += ri * ri;
+          v3[2] += bi * bi;
+        }
+        publish(k, r[k]);
+        v3[0] += (double)r[k] * (double)r[k];
+        }
+      if (!exchange<3>(v3, hr, [&](const double *tot) { mixed_epi(e, MX_R, st, tot); })) return;
+    }
+    if (S->status == S_NONFINITE) return outcome(kResDeclined);
+    if (!window_x()) return;
+    double v2[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int i = row[t + k * NT];
+      if (i >= 0) {
+        const double xi = win[t + k * NT], ax = apply64(k, i, xi), ri = a.b[i] - ax;
+        v2[0] += xi * ax;
+        v2[1] += ri * ri;
+      }
+    }
+    if (!exchange<2, double>(v2, nullptr, [st](const double *tot) {
+          st->energy = tot[0];
+          st->res2 = tot[1];
+        }))
+      return;
+    if (t == 0) S->mgs_j = map.p.H;   // whether every column is an int16 offset away
+    outcome(kResSolved);
+  }
+};
+
 // Sets a block up as part c of a system and solves it.  dyn: the block's
 // dynamic shared memory (res_lds_bytes).
 template <int F, int RPT, int Code>
@@ -704,22 +960,28 @@ __device__ __forceinline__ void resident_solve(const ResArgs &a, const ResPlan &
   for (int k = t; k < (int)(sizeof(KState) / sizeof(unsigned)); k += kResThreads)
     reinterpret_cast<unsigned *>(&S)[k] = 0u;
   if (t == 0) bad = 0;
-  Resident<F, RPT> w(a);
+  using Sys = std::conditional_t<Code == kResMixedPcg, ResidentMixed<F, RPT>, Resident<F, RPT>>;
+  Sys w(a);
   w.map.init(p, a.A.neq, c);
   w.nh = p.nb > 1 ? p.nh : 0;
   w.nb = p.nb;
   w.win = dyn;
-  w.own = dyn + kResThreads * RPT + w.nh;
-  w.hs = w.own + (size_t)res_own_vecs(Code) * kResThreads * RPT;
-  w.row = reinterpret_cast<int *>(w.hs + (size_t)res_halo_vecs(Code) * w.nh);
+  if constexpr (Code == kResMixedPcg) {
+    w.hs = reinterpret_cast<float *>(dyn + kResThreads * RPT + w.nh);
+    w.row = reinterpret_cast<int *>(w.hs + 3 * (size_t)w.nh);
+  } else {
+    w.own = dyn + kResThreads * RPT + w.nh;
+    w.hs = w.own + (size_t)res_own_vecs(Code) * kResThreads * RPT;
+    w.row = reinterpret_cast<int *>(w.hs + (size_t)res_halo_vecs(Code) * w.nh);
+  }
   w.hrow = w.row + kResThreads * RPT;
   w.red = red;
   w.S = &S;
   w.bad = &bad;
   for (int h = t; h < w.nh; h += kResThreads) w.hrow[h] = w.map.halo(h);
   __syncthreads();
-  if constexpr (Code == 1) w.pcg();
-  else w.bicgstab();
+  if constexpr (Code == kResBicgstab) w.bicgstab();
+  else w.pcg();
 }
 
 // Does block c take part in plan p?
@@ -766,9 +1028,23 @@ struct ResBatchArgs {
   ResPlan *plans;            // per system, cleared
   res_word *rows, *part;
   unsigned *err;
-  double tol;
-  int maxit, x0_zero, stop_rule, rmax, hmax;
+  double tol, delta;
+  int maxit, x0_zero, stop_rule, max_inner, rmax, hmax;
 };
+
+// An int / a struct of ints that is the same for the whole wavefront, in
+// scalar registers (the compiler cannot tell: the kernel also stores).
+__device__ __forceinline__ int res_uniform(const int *p) { return __builtin_amdgcn_readfirstlane(*p); }
+template <class T>
+__device__ __forceinline__ T res_uniform_ints(const T *p) {
+  static_assert(sizeof(T) % sizeof(int) == 0, "a struct of ints");
+  T v;
+  int w[sizeof(T) / sizeof(int)];
+#pragma unroll
+  for (size_t k = 0; k < sizeof(T) / sizeof(int); ++k) w[k] = res_uniform(reinterpret_cast<const int *>(p) + k);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
 
 constexpr int kResGang = 32;   // a team's first exchange may wait for its members' earlier systems
 
@@ -801,24 +1077,25 @@ __global__ __launch_bounds__(256) void resident_batch_prep_kernel(ResBatchArgs B
   resident_prep<F>(a);
 }
 
-template <int F, int RPT>
+template <int F, int RPT, int Code>
 __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArgs B) {
   extern __shared__ double dyn[];
   const int g = (int)gridDim.x, b0 = (int)blockIdx.x;
   const int b = (g & 7) == 0 ? (b0 & 7) * (g >> 3) + (b0 >> 3) : b0;
-  for (int k = B.block_ptr[b]; k < B.block_ptr[b + 1]; ++k) {
-    const int sys = B.block_list[k];
-    const SysDesc D = B.desc[sys];
+  const int k1 = res_uniform(B.block_ptr + b + 1);
+  for (int k = res_uniform(B.block_ptr + b); k < k1; ++k) {
+    const int sys = res_uniform(B.block_list + k);
+    const SysDesc D = res_uniform_ints(B.desc + sys);
     const int c = b - D.g_first;
     ResPlan p{};
     if (D.g_count > 1) {
-      p = B.plans[sys];
+      p = res_uniform_ints(B.plans + sys);
     } else {
       p.nb = 1;
       p.R = D.neq;
     }
     if (p.nb == 0 && c == 0 && threadIdx.x == 0) B.st[sys].pad6 = kResDeclined;
-    if (!resident_part<RPT, 1>(p, c)) continue;
+    if (!resident_part<RPT, Code>(p, c)) continue;
     ResArgs a{};
     resident_batch_mat<F>(B, D, a.A);
     a.st = B.st + sys;
@@ -826,7 +1103,7 @@ __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArg
     a.x = B.x + D.row_off;
     a.b = B.b + D.row_off;
     a.rows = B.rows + (size_t)4 * D.row_off;
-    a.part = B.part + B.part_off[sys];
+    a.part = B.part + res_uniform(B.part_off + sys);
     a.part_half = res_part_half(D.g_count);
     a.err = B.err;
     a.gang = kResGang;
@@ -834,7 +1111,9 @@ __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArg
     a.maxit = B.maxit;
     a.x0_zero = B.x0_zero;
     a.stop_rule = B.stop_rule;
-    resident_solve<F, RPT, 1>(a, p, c, dyn);
+    a.delta = B.delta;
+    a.max_inner = B.max_inner;
+    resident_solve<F, RPT, Code>(a, p, c, dyn);
     if (ld_relaxed(B.err) != 0u) return;   // (uniform enough: a block that goes on only waits, bounded)
     __syncthreads();                       // LDS is reused
   }

@@ -24,7 +24,8 @@ constexpr int kResGroups = 16;       // groups of 16 blocks whose sums are added
 // The words of one buffer for the partial sums of nb blocks: a pair per
 // (value, block) up to 64 blocks, beyond that one per (group, value, block of
 // the group) and one per (receiving group, value, group).
-constexpr int res_part_half(int nb) { return nb <= 64 ? 2 * 4 * 64 : 2 * 2 * kResGroups * 64; }
+constexpr int kResSums = 5, kResGroupSums = 16 * kResSums;
+constexpr int res_part_half(int nb) { return nb <= 64 ? 2 * kResSums * 64 : 2 * 2 * kResGroups * kResGroupSums; }
 constexpr int kResPartWords = 2 * res_part_half(kResMaxBlocks);
 
 // How rows are dealt to blocks, decided on the device by resident_prep_kernel
@@ -153,21 +154,32 @@ FVC_HD bool res_strips(int n, int H, int rmax, int bmax, int hmax, ResPlan &p) {
   return true;
 }
 
+// The solvers held on chip.
+constexpr int kResPcg = 1, kResBicgstab = 2, kResMixedPcg = 3;
+
 // The blocks' shared memory: the operand window (own rows, then halo
 // entries), x and the shadow residual (read once per iteration; the other
 // vectors are in registers, which these two would overflow at eight rows a
 // thread), the halo rows' vectors, and both kinds' global row numbers.
-constexpr int res_halo_vecs(int code) { return code == 1 ? 4 : 5; }
-constexpr int res_own_vecs(int code) { return code == 1 ? 1 : 2; }
+// Mixed precision: the window (doubles at the FP64 updates), three floats a
+// halo row; x stays in memory.
+constexpr int res_halo_vecs(int code) { return code == kResBicgstab ? 5 : 4; }
+constexpr int res_own_vecs(int code) { return code == kResBicgstab ? 2 : 1; }
+constexpr size_t res_own_bytes(int code) {
+  return code == kResMixedPcg ? sizeof(double) + sizeof(int) : (1 + res_own_vecs(code)) * sizeof(double) + sizeof(int);
+}
+constexpr size_t res_halo_bytes(int code) {
+  return code == kResMixedPcg ? sizeof(double) + 3 * sizeof(float) + sizeof(int)
+                              : (1 + res_halo_vecs(code)) * sizeof(double) + sizeof(int);
+}
 constexpr size_t res_lds_bytes(int code, int rpt, int nh) {
-  return (size_t)kResThreads * rpt * ((1 + res_own_vecs(code)) * sizeof(double) + sizeof(int)) +
-         (size_t)nh * ((1 + res_halo_vecs(code)) * sizeof(double) + sizeof(int));
+  return (size_t)kResThreads * rpt * res_own_bytes(code) + (size_t)nh * res_halo_bytes(code);
 }
 constexpr size_t kResLds = 156 * 1024;   // of a CU's 160 KB, less the reductions' static part
 // the halo entries that fit beside rpt rows per thread
 constexpr int res_max_halo(int code, int rpt) {
   const size_t left = kResLds - res_lds_bytes(code, rpt, 0);
-  const size_t nh = left / ((1 + res_halo_vecs(code)) * sizeof(double) + sizeof(int));
+  const size_t nh = left / res_halo_bytes(code);
   return nh < (size_t)kResMaxHalo ? (int)nh : kResMaxHalo;
 }
 

@@ -382,17 +382,18 @@ int drive_batches(DevState &d, hipStream_t s, int maxit, Iter &&iteration, State
 // The on-chip PCG / BiCGSTAB (fvc_resident.h).  Measured on MI355X against one
 // kernel per phase, whole solves to a true residual of 1e-10: PCG 4,096 rows
 // 3.93 -> 1.27 ms, 429,713 rows 77.8 -> 22.8; BiCGSTAB 12,707 rows 0.92 ->
-// 0.37, 1,048,576 rows 2.61 -> 0.77.
+// 0.37, 1,048,576 rows 2.61 -> 0.77.  Mixed PCG, us per FP32 iteration: 5,120
+// rows 8.2 -> 3.3, 160,860 12.2 -> 5.0, 1,048,576 18.1 -> 7.0.
 constexpr bool resident_format(int F) { return F == F_ELL4 || F == F_ELL3 || F == F_CSRD; }
 
-template <int F>
-const void *resident_fn(int code, int rpt) {
+template <int F, int Code>
+const void *resident_fn(int rpt) {
   if constexpr (resident_format(F)) {
     switch (rpt) {
-      case 1: return code == FVC_PCG ? (const void *)&resident_kernel<F, 1, 1> : (const void *)&resident_kernel<F, 1, 2>;
-      case 2: return code == FVC_PCG ? (const void *)&resident_kernel<F, 2, 1> : (const void *)&resident_kernel<F, 2, 2>;
-      case 4: return code == FVC_PCG ? (const void *)&resident_kernel<F, 4, 1> : (const void *)&resident_kernel<F, 4, 2>;
-      case 8: return code == FVC_PCG ? (const void *)&resident_kernel<F, 8, 1> : (const void *)&resident_kernel<F, 8, 2>;
+      case 1: return (const void *)&resident_kernel<F, 1, Code>;
+      case 2: return (const void *)&resident_kernel<F, 2, Code>;
+      case 4: return (const void *)&resident_kernel<F, 4, Code>;
+      case 8: return (const void *)&resident_kernel<F, 8, Code>;
     }
   }
   return nullptr;
@@ -402,7 +403,7 @@ const void *resident_fn(int code, int rpt) {
 // caller solves it one kernel per phase).  part: kResPartWords words; rows:
 // at least 4 neq words (vectors that the caller does not need yet).
 template <int F>
-int run_resident(DevState &d, const SolveIn &in, KState *st, unsigned *ctr, res_word *part, res_word *rows,
+int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned *ctr, res_word *part, res_word *rows,
                  fvc_stats *stats, hipStream_t s, bool *done) {
   *done = false;
   if constexpr (!resident_format(F)) {
@@ -414,9 +415,12 @@ int run_resident(DevState &d, const SolveIn &in, KState *st, unsigned *ctr, res_
     ResArgs a{};
     a.A = in.A; a.st = st; a.m = in.m; a.x = in.x; a.b = in.b;
     a.tol = in.tol; a.maxit = in.maxit; a.x0_zero = in.x0_zero; a.stop_rule = in.stop_rule;
-    const void *fn = resident_fn<F>(in.code, sh.rpt);
-    const int hmax = sh.blocks > 1 ? res_max_halo(in.code, sh.rpt) : 0;
-    const size_t lds = res_lds_bytes(in.code, sh.rpt, hmax);
+    a.delta = in.refresh_drop; a.max_inner = in.refresh_every;
+    const void *fn = kind == kResPcg        ? resident_fn<F, kResPcg>(sh.rpt)
+                     : kind == kResBicgstab ? resident_fn<F, kResBicgstab>(sh.rpt)
+                                            : resident_fn<F, kResMixedPcg>(sh.rpt);
+    const int hmax = sh.blocks > 1 ? res_max_halo(kind, sh.rpt) : 0;
+    const size_t lds = res_lds_bytes(kind, sh.rpt, hmax);
     HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int occ = 0;
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, kResThreads, lds));
@@ -447,7 +451,10 @@ int run_resident(DevState &d, const SolveIn &in, KState *st, unsigned *ctr, res_
     *done = true;
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, d.ev0, d.ev1));
-    fill_stats(stats, hs, in.code, true, ms, sh.blocks, kResThreads, 0);
+    int flags = 0;
+    if (kind == kResMixedPcg && F != F_CSRD && hs.mgs_j <= 32767) flags = FVC_FLAG_COL16;   // as 16-bit window slots
+    fill_stats(stats, hs, in.code, true, ms, sh.blocks, kResThreads, flags);
+    if (stats && kind == kResMixedPcg) stats->inner_iterations = hs.cycle;   // FP64 residual recomputations
     return status_of(hs);
   }
 }
@@ -570,7 +577,8 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   if (in.engine == FVC_ENGINE_AUTO && in.code != FVC_GMRES && fused && in.bs == 0 && in.G_req == 0 &&
       in.barrier == 0 && in.row_order == 0 && !in.lanex && res_part) {
     bool done = false;
-    rc = run_resident<F>(d, in, st, ctr, part, reinterpret_cast<res_word *>(vec[0]), stats, s, &done);
+    rc = run_resident<F>(d, in, in.code == FVC_PCG ? kResPcg : kResBicgstab, st, ctr, part,
+                         reinterpret_cast<res_word *>(vec[0]), stats, s, &done);
     if (rc || done) return rc;
   }
   const bool may_fall_back = persistent && in.engine == FVC_ENGINE_AUTO;
@@ -898,6 +906,10 @@ int run_mixed(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
                    align_up(n * sizeof(double)) + align_up(n * sizeof(float)) + 2 * align_up(n * sizeof(float4)) +
                    align_up(2 * sizeof(KState)) + align_up(2 * kMaxK * (size_t)G * sizeof(double)) +
                    align_up(std::max<size_t>(n16, 1) * sizeof(short)) + 4096;
+    // as in run_solve: the on-chip solver's words, and x as it was given
+    size_t res_part = align_up(kResPartWords * sizeof(res_word)), res_x = in.x0_zero ? 0 : align_up(n * sizeof(double));
+    if (d.noalloc && bytes + res_part + res_x > kScratchBytes) res_part = res_x = 0;
+    bytes += res_part + res_x;
     char *ws = nullptr;
     if ((rc = workspace(d, bytes, &ws))) return rc;
     Carve cv{ws, bytes};
@@ -906,6 +918,8 @@ int run_mixed(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
     int *wide = reinterpret_cast<int *>(ctr + kCtrWords + G);
     KState *st = cv.take<KState>(1);
     double *partials = cv.take<double>(kMaxK * (size_t)G);
+    res_word *part = cv.take<res_word>(res_part / sizeof(res_word));
+    double *xgiven = cv.take<double>(res_x / sizeof(double));
     Defer dfr{cv.take<KState>(2), cv.take<double>(2 * kMaxK * (size_t)G), 0};
     float *av32 = cv.take<float>(std::max<size_t>(nv, 1));
     short *jo = cv.take<short>(std::max<size_t>(n16, 1));
@@ -915,6 +929,17 @@ int run_mixed(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
     a.ps = align_up(n * sizeof(float4)) / sizeof(float4);
     a.rec = cv.take<float4>(2 * a.ps);
     if (!cv.fits()) return carve_overflow(cv);
+    // On chip where the launch is the library's choice (run_solve).  It works
+    // on x in place: x as given is kept for the case that it declines.
+    if (in.engine == FVC_ENGINE_AUTO && in.bs == 0 && in.G_req == 0 && in.barrier == 0 && in.row_order == 0 && res_part) {
+      bool done = false;
+      if (!in.x0_zero)
+        HIPCHK(hipMemcpyAsync(xgiven, in.x, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+      rc = run_resident<F>(d, in, kResMixedPcg, st, ctr, part, reinterpret_cast<res_word *>(a.rec), stats, s, &done);
+      if (rc || done) return rc;
+      if (!in.x0_zero)
+        HIPCHK(hipMemcpyAsync(in.x, xgiven, n * sizeof(double), hipMemcpyDeviceToDevice, s));
+    }
     a.A = in.A;
     a.A32.neq = neq;
     a.A32.w = in.A.w;
@@ -1631,7 +1656,7 @@ int dot_impl(const double *a, const double *b, int n, double *result, bool on_de
 
 // ------------------------------------------------------------- batches --
 
-// Systems lo .. hi - 1 of an FP64 batch on chip (fvc_resident.h): solves what
+// Systems lo .. hi - 1 of a batch on chip (fvc_resident.h): solves what
 // fits, in one launch, and adds to `todo` the systems it did not solve.
 // Measured on MI355X against the streaming kernels below: 48 systems of side
 // 32 .. 160 40.4 -> 4.6 ms; 256 systems of side 32 .. 512 (10.2M rows) 835 ms at
@@ -1649,8 +1674,13 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
   if constexpr (!resident_format(F)) {
     return leave();
   } else {
-    static const void *const fns[4] = {(const void *)&resident_batch_kernel<F, 1>, (const void *)&resident_batch_kernel<F, 2>,
-                                       (const void *)&resident_batch_kernel<F, 4>, (const void *)&resident_batch_kernel<F, 8>};
+    static const void *const fns[2][4] = {
+        {(const void *)&resident_batch_kernel<F, 1, kResPcg>, (const void *)&resident_batch_kernel<F, 2, kResPcg>,
+         (const void *)&resident_batch_kernel<F, 4, kResPcg>, (const void *)&resident_batch_kernel<F, 8, kResPcg>},
+        {(const void *)&resident_batch_kernel<F, 1, kResMixedPcg>, (const void *)&resident_batch_kernel<F, 2, kResMixedPcg>,
+         (const void *)&resident_batch_kernel<F, 4, kResMixedPcg>, (const void *)&resident_batch_kernel<F, 8, kResMixedPcg>}};
+    const bool mixed = o.precision == FVC_PREC_MIXED;
+    const int kind = mixed ? kResMixedPcg : kResPcg;
     std::vector<int> sizes(nsys);
     for (int i = 0; i < nsys; ++i) sizes[i] = row_off[lo + i + 1] - row_off[lo + i];
     const ResBatchPlan plan = plan_resident_batch(sizes, o.batch_work_exp10 > 0 ? o.batch_work_exp10 / 10.0 : 1.5, d.cus);
@@ -1658,9 +1688,9 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     // one block per CU: two (which one row a thread would allow) hold each
     // other up (48 systems of side 32 .. 160: 9.4 ms on 512 blocks of one row a
     // thread, 4.3 on 208 of four)
-    const void *fn = fns[plan.rpt == 1 ? 0 : plan.rpt == 2 ? 1 : plan.rpt == 4 ? 2 : 3];
-    const int hmax = res_max_halo(FVC_PCG, plan.rpt);
-    const size_t lds = res_lds_bytes(FVC_PCG, plan.rpt, hmax);
+    const void *fn = fns[mixed][plan.rpt == 1 ? 0 : plan.rpt == 2 ? 1 : plan.rpt == 4 ? 2 : 3];
+    const int hmax = res_max_halo(kind, plan.rpt);
+    const size_t lds = res_lds_bytes(kind, plan.rpt, hmax);
     HIPCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int occ = 0;
     HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, kResThreads, lds));
@@ -1690,9 +1720,11 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
                  at_ptr = put(plan.ptr.data(), plan.ptr.size()), at_list = put(plan.list.data(), plan.list.size());
     const size_t n = (size_t)row_off[hi];
     const size_t nclear = (size_t)nsys * (sizeof(ResPlan) / sizeof(unsigned)) + 1;
+    // mixed precision works on x in place: x as given is kept for what it declines
+    const size_t nkeep = mixed && o.x0_rule == FVC_X0_GIVEN ? n - (size_t)row_off[lo] : 0;
     const size_t bytes = align_up(up.size() * sizeof(int)) + align_up(nsys * sizeof(KState)) +
                          align_up(nclear * sizeof(unsigned)) + align_up(npart * sizeof(res_word)) +
-                         align_up(4 * n * sizeof(res_word)) + 4096;
+                         align_up(4 * n * sizeof(res_word)) + align_up(nkeep * sizeof(double)) + 4096;
     int rc = ensure_arena(d, bytes);
     if (rc) return rc;
     Carve cv{d.arena, bytes};
@@ -1701,7 +1733,9 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     unsigned *clear = cv.take<unsigned>(nclear);
     res_word *part = cv.take<res_word>(npart);
     res_word *rows = cv.take<res_word>(4 * n);
+    double *xkeep = cv.take<double>(nkeep);
     if (!cv.fits()) return carve_overflow(cv);
+    if (nkeep) HIPCHK(hipMemcpyAsync(xkeep, x + row_off[lo], nkeep * sizeof(double), hipMemcpyDeviceToDevice, s));
     HIPCHK(hipMemcpyAsync(dup, up.data(), up.size() * sizeof(int), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, clear, (int)nclear, st, nsys);
     ResBatchArgs B{};
@@ -1719,6 +1753,9 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     B.maxit = maxit;
     B.x0_zero = o.x0_rule == FVC_X0_GIVEN ? 0 : 1;
     B.stop_rule = o.stop_rule;
+    B.delta = o.refresh_drop_e3 > 0 ? o.refresh_drop_e3 * 1e-3 : kRefreshDrop;
+    B.max_inner = o.refresh_every > 0 ? o.refresh_every : kRefreshEvery;
+    if (B.delta >= 1.0) return fail(FVC_BAD_ARGUMENT, "refresh_drop_e3 %d must be below 1000", o.refresh_drop_e3);
     B.rmax = kResThreads * plan.rpt;
     B.hmax = hmax;
     if (!multi.empty())
@@ -1730,8 +1767,13 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     HIPCHK(hipMemcpyAsync(host_st.data() + lo, st, nsys * sizeof(KState), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(&err, B.err, sizeof err, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
-    for (int i = lo; i < hi; ++i)
-      if (err || host_st[i].pad6 != kResSolved) todo.push_back(i);
+    for (int i = lo; i < hi; ++i) {
+      if (!err && host_st[i].pad6 == kResSolved) continue;
+      todo.push_back(i);
+      if (nkeep)
+        HIPCHK(hipMemcpyAsync(x + row_off[i], xkeep + (row_off[i] - row_off[lo]), sizes[i - lo] * sizeof(double),
+                              hipMemcpyDeviceToDevice, s));
+    }
     return FVC_OK;
   }
 }
@@ -1770,7 +1812,7 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
   HIPCHK(hipEventRecord(d.ev0, s));
   // On chip where the launch is the library's choice; options that shape it
   // keep the kernels they were written for.
-  if (!mixed && o.engine == FVC_ENGINE_AUTO && o.recurrence == FVC_REC_FUSED && o.block_size == 0 &&
+  if (o.engine == FVC_ENGINE_AUTO && o.recurrence == FVC_REC_FUSED && o.block_size == 0 &&
       o.grid_blocks == 0 && o.barrier == 0 && o.batch_rows_per_wave == 0) {
     const int per = o.batch_launch_systems > 0 ? o.batch_launch_systems : nsys;
     for (int lo = 0; lo < nsys; lo += std::min(per, nsys - lo))
@@ -1797,7 +1839,11 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
     return FVC_OK;
   };
   const int ntodo = (int)todo.size();
-  if (ntodo == 0) return close(0);
+  if (ntodo == 0) {
+    bool near = mixed && F != F_CSRD;
+    for (const KState &q : host_st) near = near && q.mgs_j <= 32767;
+    return close(near ? FVC_FLAG_COL16 : 0);
+  }
   const size_t n = (size_t)total;
   const size_t nv = (size_t)val_off[nsys];   // stored off-diagonal values
   size_t bytes = align_up(((size_t)wave * kCtrWords + cap) * sizeof(unsigned)) + align_up((size_t)wave * sizeof(KState)) +
