@@ -55,7 +55,8 @@
 #define FVCI_RES_R(P, F, R)                                      \
   P __global__ void fvc::resident_kernel<F, R, 1>(fvc::ResArgs); \
   P __global__ void fvc::resident_kernel<F, R, 2>(fvc::ResArgs); \
-  P __global__ void fvc::resident_kernel<F, R, 3>(fvc::ResArgs);
+  P __global__ void fvc::resident_kernel<F, R, 3>(fvc::ResArgs); \
+  P __global__ void fvc::resident_kernel<F, R, 4>(fvc::ResArgs);
 #define FVCI_RES_RB(P, F, R)                                          \
   P __global__ void fvc::resident_batch_kernel<F, R, 1>(fvc::ResBatchArgs); \
   P __global__ void fvc::resident_batch_kernel<F, R, 3>(fvc::ResBatchArgs);

@@ -1123,6 +1123,65 @@ __device__ __forceinline__ void gmres_close_step(const GmresArgs &a, KState *st,
   }
 }
 
+// The scalar part of a cycle's start: t = ||g1||^2, ||b||^2 (first cycle),
+// ||b - A x||^2.
+__device__ __forceinline__ void gmres_start_epi(const GmresArgs &a, KState *st, bool first, const double *t) {
+  if (first) {
+    st->bnorm2 = t[1];
+    st->econv = a.tol * sqrt(t[1]);
+    st->conv = st->econv;
+    st->inner = 0;
+    st->status = S_MAXIT;
+    st->done = 0;
+  }
+  const double e1 = sqrt(t[0]);
+  if (a.stop_rule == 1) {
+    const double rt = sqrt(t[2]);
+    st->rnorm2 = t[2];
+    st->last = rt;
+    st->iter = st->cycle;
+    const bool stop = rt <= st->conv || !finite(rt) || !finite(e1) || st->cycle >= a.maxit;
+    if (rt <= st->conv) st->status = S_OK;
+    else if (!finite(rt) || !finite(e1)) st->status = S_NONFINITE;
+    if (stop) {
+      st->done = 1;
+      st->inner_done = 1;
+      return;
+    }
+    // this cycle's target for the preconditioned residual
+    st->econv = e1 * (st->conv / rt);
+  }
+  st->cycle = st->cycle + 1;
+  a.e[1] = e1;
+  a.nrm[1] = e1;
+  st->step_i = 1;
+  st->mgs_j = 1;
+  st->inner_done = 0;
+  st->ni = 0;
+  if (e1 == 0.0) {          // exact solution already: nothing to orthogonalise
+    st->status = S_OK;
+    st->done = 1;
+    st->inner_done = 1;
+    st->last = 0.0;
+    st->iter = st->cycle;
+  } else if (!finite(e1)) {
+    st->status = S_NONFINITE;
+    st->done = 1;
+    st->inner_done = 1;
+  }
+}
+// ... and of its end, after x was updated with nI columns.
+__device__ __forceinline__ void gmres_xupd_epi(const GmresArgs &a, KState *st, int nI) {
+  const double en = a.e[nI + 1];
+  st->last = fabs(en);
+  st->iter = st->cycle;
+  if (!finite(en)) { st->status = S_NONFINITE; st->done = 1; }
+  else if (a.stop_rule == 1) {}   // the next cycle's start tests the true residual
+  else if (fabs(en) <= st->econv) { st->status = S_OK; st->done = 1; }   // :402
+  else if (st->cycle >= a.maxit) { st->status = S_MAXIT; st->done = 1; }
+  st->inner_done = 0;
+}
+
 // Classical Gram-Schmidt with one re-orthogonalisation ("twice is enough",
 // Giraud, Langou, Rozloznik 2005): per Arnoldi step i two passes of dot
 // products against columns 1..i and one norm, instead of the i+1 sequential
@@ -1275,51 +1334,7 @@ __device__ __forceinline__ bool gmres_phase(const GmresArgs &a, int ph, double *
       v[0] += gi * gi;
       v[2] += ri * ri;
     }
-    return grid_sync<3>(a.g, v, lds, [&](const double *t) {
-      if (first) {
-        st->bnorm2 = t[1];
-        st->econv = a.tol * sqrt(t[1]);
-        st->conv = st->econv;
-        st->inner = 0;
-        st->status = S_MAXIT;
-        st->done = 0;
-      }
-      const double e1 = sqrt(t[0]);
-      if (a.stop_rule == 1) {
-        const double rt = sqrt(t[2]);
-        st->rnorm2 = t[2];
-        st->last = rt;
-        st->iter = st->cycle;
-        const bool stop = rt <= st->conv || !finite(rt) || !finite(e1) || st->cycle >= a.maxit;
-        if (rt <= st->conv) st->status = S_OK;
-        else if (!finite(rt) || !finite(e1)) st->status = S_NONFINITE;
-        if (stop) {
-          st->done = 1;
-          st->inner_done = 1;
-          return;
-        }
-        // this cycle's target for the preconditioned residual
-        st->econv = e1 * (st->conv / rt);
-      }
-      st->cycle = st->cycle + 1;
-      a.e[1] = e1;
-      a.nrm[1] = e1;
-      st->step_i = 1;
-      st->mgs_j = 1;
-      st->inner_done = 0;
-      st->ni = 0;
-      if (e1 == 0.0) {          // exact solution already: nothing to orthogonalise
-        st->status = S_OK;
-        st->done = 1;
-        st->inner_done = 1;
-        st->last = 0.0;
-        st->iter = st->cycle;
-      } else if (!finite(e1)) {
-        st->status = S_NONFINITE;
-        st->done = 1;
-        st->inner_done = 1;
-      }
-    });
+    return grid_sync<3>(a.g, v, lds, [&](const double *t) { gmres_start_epi(a, st, first, t); });
   }
   if (ph == GM_MV) {
     // g(i+1) = A g(i) / m; h(1,i) = g(i+1).g(1)
@@ -1383,16 +1398,7 @@ __device__ __forceinline__ bool gmres_phase(const GmresArgs &a, int ph, double *
       for (int j = 1; j <= nI; ++j) xr = xr + ysh[j] * a.gv[(size_t)(j - 1) * a.ld + r];
       a.x[r] = xr;
     }
-    return grid_sync<0>(a.g, v, lds, [&](const double *) {
-      const double en = a.e[nI + 1];
-      st->last = fabs(en);
-      st->iter = st->cycle;
-      if (!finite(en)) { st->status = S_NONFINITE; st->done = 1; }
-      else if (a.stop_rule == 1) {}   // the next cycle's start tests the true residual
-      else if (fabs(en) <= st->econv) { st->status = S_OK; st->done = 1; }   // :402
-      else if (st->cycle >= a.maxit) { st->status = S_MAXIT; st->done = 1; }
-      st->inner_done = 0;
-    });
+    return grid_sync<0>(a.g, v, lds, [&](const double *) { gmres_xupd_epi(a, st, nI); });
   }
   // GM_FINAL: energy x.b (src/Iterativos.f:412) and ||b - Ax||^2
   double v[2] = {0.0, 0.0};

@@ -1,5 +1,5 @@
-// fvc_resident.h -- PCG, BiCGSTAB and mixed PCG with the whole system held on
-// chip.
+// fvc_resident.h -- PCG, BiCGSTAB, mixed PCG and GMRES with the whole system
+// held on chip (of GMRES, all but the basis).
 //
 // One launch solves the system: every block loads its rows' matrix entries
 // once into registers and keeps its rows of every Krylov vector there too
@@ -250,6 +250,9 @@ struct ResArgs {
   double tol;
   double delta;            // mixed: residual drop that triggers an FP64 update
   int max_inner;           // mixed: FP32 iterations between updates, at most
+  double *gv;              // GMRES: basis columns 1 .. k, own rows only, ld apart
+  size_t ld;
+  int k;
   int maxit, x0_zero, stop_rule;
 };
 
@@ -528,12 +531,12 @@ struct Resident : ResNet {
     }
   }
 
-  // Energy x.Ax and ||b - Ax||^2 (src/Iterativos.f:82-83,204-205), then x and
-  // the state are written.
+  // Energy x.Ax (GMRES: x.b) and ||b - Ax||^2 (src/Iterativos.f:82-83,204-205,
+  // 412), then x and the state are written.
   // A breakdown or an overflow depends on the roundings on the way there, so
   // such a solve is declined, with x as it came: it is solved again in the
   // other engine's order of sums, whose outcome the caller gets.
-  __device__ __forceinline__ void finish() {
+  __device__ __forceinline__ void finish(bool energy_xb = false) {
     if (S->status == S_BREAKDOWN || S->status == S_NONFINITE) return outcome(kResDeclined);
     const int t = (int)threadIdx.x;
     const double *x = own + t;
@@ -552,7 +555,7 @@ struct Resident : ResNet {
       const int i = row[t + k * NT];
       const double bi = i >= 0 ? a.b[i] : 0.0;
       const double ri = bi - ax;
-      v[0] += xi * ax;
+      v[0] += xi * (energy_xb ? bi : ax);
       v[1] += ri * ri;
     }
     KState *s = S;
@@ -569,6 +572,7 @@ struct Resident : ResNet {
 
   __device__ __forceinline__ void pcg();
   __device__ __forceinline__ void bicgstab();
+  __device__ __forceinline__ void gmres();
 };
 
 // The fused PCG (cg1_*, fvc_krylov.h), one exchange per iteration.
@@ -747,6 +751,142 @@ __device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
     if (!exchange<4>(v4, ht, [&](const double *tot) { bicg2_epi(e, B2_Q, s_, tot); })) return;
   }
   finish();
+}
+
+// GMRES(k) with modified Gram-Schmidt in the reference's order (gmres_phase,
+// fvc_krylov.h), an exchange for each of the i + 1 reductions of Arnoldi step
+// i.  The vector being orthogonalised stays in registers; the basis columns,
+// k times too large for them, are in memory, where only their own block reads
+// them: the next column is on its way while the block waits for a sum, so
+// that a projection costs little more than its exchange.  The Hessenberg
+// matrix, the rotations and the back substitution are in every block's LDS.
+template <int F, int RPT>
+__device__ __forceinline__ void Resident<F, RPT>::gmres() {
+  __shared__ double hbuf[(kResGmresK + 1) * kResGmresK + 5 * (kResGmresK + 3)];
+  const int t = (int)threadIdx.x;
+  KState *st = S;
+  GmresArgs e{};
+  e.tol = a.tol;
+  e.k = a.k;
+  e.maxit = a.maxit;
+  e.stop_rule = a.stop_rule;
+  e.h = hbuf;
+  e.cs = hbuf + (kResGmresK + 1) * kResGmresK;
+  e.sn = e.cs + kResGmresK + 3;
+  e.e = e.sn + kResGmresK + 3;
+  e.y = e.e + kResGmresK + 3;
+  e.nrm = e.y + kResGmresK + 3;
+  double *x = own + t;
+  double w[RPT], gj[RPT], gn[RPT];
+  const double none[1] = {0.0};
+  const bool ok = load_rows();
+#pragma unroll
+  for (int k = 0; k < RPT; ++k) x[k * NT] = 0.0;
+  for (int h = t; h < nh; h += NT) win[RB + h] = 0.0;
+  const auto column = [&](int c, int i) -> double & { return a.gv[(size_t)(c - 1) * a.ld + i]; };
+  const auto load_column = [&](int c, double *g) {
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int i = row[t + k * NT];
+      g[k] = i >= 0 ? column(c, i) : 0.0;
+    }
+  };
+  for (bool first = true; !st->done; first = false) {
+    // g1 = (b - A x) / m
+    if (!first) {
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        win[t + k * NT] = x[k * NT];
+        publish(k, x[k * NT]);
+      }
+      if (!exchange<1>(none, win + RB, [](const double *) {})) return;
+    }
+    double v[4] = {0.0, 0.0, 0.0, ok ? 0.0 : 1.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int i = row[t + k * NT];
+      const double bi = i >= 0 ? a.b[i] : 0.0;
+      const double ri = first ? bi : bi - apply(k, x[k * NT]);
+      w[k] = ri / dm[k];
+      v[0] += w[k] * w[k];
+      if (first) v[1] += bi * bi;
+      v[2] += ri * ri;
+      publish(k, w[k]);
+    }
+    if (!exchange<4>(v, win + RB, [&](const double *tot) {
+          gmres_start_epi(e, st, first, tot);
+          if (tot[3] != 0.0) st->pend = 1;
+        }))
+      return;
+    if (st->pend) return outcome(kResDeclined);
+    if (st->done) break;
+    for (int i = 1; i <= a.k; ++i) {
+      // column i = w / ||w||, w = A g_i / m (the halo holds w of its rows)
+      const double ni = e.nrm[i];
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        const double g = w[k] / ni;
+        const int r = row[t + k * NT];
+        win[t + k * NT] = g;
+        if (r >= 0) column(i, r) = g;
+        if (i == 1) gj[k] = g;
+      }
+      for (int h = t; h < nh; h += NT) win[RB + h] = win[RB + h] / ni;
+      if (i > 1) load_column(1, gj);
+      lds_barrier();
+      double d[1] = {0.0};
+#pragma unroll
+      for (int k = 0; k < RPT; ++k) {
+        w[k] = apply(k, win[t + k * NT]) / dm[k];
+        d[0] += w[k] * gj[k];
+      }
+      if (i > 2) load_column(2, gn);
+      if (!exchange<1, double>(d, nullptr, [&](const double *tot) { e.h[(size_t)(i - 1) * (a.k + 1)] = tot[0]; })) return;
+      for (int j = 1; j <= i; ++j) {
+        const double hj = e.h[(size_t)(i - 1) * (a.k + 1) + (j - 1)];
+        d[0] = 0.0;
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+          w[k] = w[k] - hj * gj[k];
+          if (j == i) {
+            d[0] += w[k] * w[k];
+            publish(k, w[k]);
+          } else {
+            gj[k] = j + 1 == i ? win[t + k * NT] : gn[k];   // column i is still in the window
+            d[0] += w[k] * gj[k];
+          }
+        }
+        if (j + 2 < i) load_column(j + 2, gn);
+        if (!exchange<1>(d, j == i ? win + RB : nullptr, [&](const double *tot) {
+              double *hi = e.h + (size_t)(i - 1) * (a.k + 1);
+              if (j < i) {
+                hi[j] = tot[0];
+                return;
+              }
+              const double norm = sqrt(tot[0]);
+              hi[i] = norm;
+              e.nrm[i + 1] = norm;
+              gmres_close_step(e, st, i);
+            }))
+          return;
+      }
+      if (st->inner_done) break;
+    }
+    // x += sum_j y(j) g(j), in order
+    const int nI = st->ni;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int r = row[t + k * NT];
+      double xr = x[k * NT];
+      if (r >= 0)
+        for (int j = 1; j <= nI; ++j) xr = xr + e.y[j] * column(j, r);
+      x[k * NT] = xr;
+    }
+    lds_barrier();
+    if (t == 0) gmres_xupd_epi(e, st, nI);
+    lds_barrier();
+  }
+  finish(true);
 }
 
 // Mixed precision (fvc_mixed.h): the scaled FP32 rows and the four FP32
@@ -972,7 +1112,7 @@ __device__ __forceinline__ void resident_solve(const ResArgs &a, const ResPlan &
   } else {
     w.own = dyn + kResThreads * RPT + w.nh;
     w.hs = w.own + (size_t)res_own_vecs(Code) * kResThreads * RPT;
-    w.row = reinterpret_cast<int *>(w.hs + (size_t)res_halo_vecs(Code) * w.nh);
+    w.row = reinterpret_cast<int *>(w.hs + (Code == kResGmres ? 0 : (size_t)res_halo_vecs(Code) * w.nh));
   }
   w.hrow = w.row + kResThreads * RPT;
   w.red = red;
@@ -981,6 +1121,7 @@ __device__ __forceinline__ void resident_solve(const ResArgs &a, const ResPlan &
   for (int h = t; h < w.nh; h += kResThreads) w.hrow[h] = w.map.halo(h);
   __syncthreads();
   if constexpr (Code == kResBicgstab) w.bicgstab();
+  else if constexpr (Code == kResGmres) w.gmres();
   else w.pcg();
 }
 

@@ -155,22 +155,25 @@ FVC_HD bool res_strips(int n, int H, int rmax, int bmax, int hmax, ResPlan &p) {
 }
 
 // The solvers held on chip.
-constexpr int kResPcg = 1, kResBicgstab = 2, kResMixedPcg = 3;
+constexpr int kResPcg = 1, kResBicgstab = 2, kResMixedPcg = 3, kResGmres = 4;
 
 // The blocks' shared memory: the operand window (own rows, then halo
 // entries), x and the shadow residual (read once per iteration; the other
 // vectors are in registers, which these two would overflow at eight rows a
 // thread), the halo rows' vectors, and both kinds' global row numbers.
 // Mixed precision: the window (doubles at the FP64 updates), three floats a
-// halo row; x stays in memory.
+// halo row; x stays in memory.  GMRES: the window, x, and the Hessenberg
+// matrix of up to kResGmresK columns, static.
+constexpr int kResGmresK = 32;
 constexpr int res_halo_vecs(int code) { return code == kResBicgstab ? 5 : 4; }
 constexpr int res_own_vecs(int code) { return code == kResBicgstab ? 2 : 1; }
 constexpr size_t res_own_bytes(int code) {
   return code == kResMixedPcg ? sizeof(double) + sizeof(int) : (1 + res_own_vecs(code)) * sizeof(double) + sizeof(int);
 }
 constexpr size_t res_halo_bytes(int code) {
-  return code == kResMixedPcg ? sizeof(double) + 3 * sizeof(float) + sizeof(int)
-                              : (1 + res_halo_vecs(code)) * sizeof(double) + sizeof(int);
+  return code == kResGmres      ? sizeof(double) + sizeof(int)
+         : code == kResMixedPcg ? sizeof(double) + 3 * sizeof(float) + sizeof(int)
+                                : (1 + res_halo_vecs(code)) * sizeof(double) + sizeof(int);
 }
 constexpr size_t res_lds_bytes(int code, int rpt, int nh) {
   return (size_t)kResThreads * rpt * res_own_bytes(code) + (size_t)nh * res_halo_bytes(code);
@@ -178,7 +181,8 @@ constexpr size_t res_lds_bytes(int code, int rpt, int nh) {
 constexpr size_t kResLds = 156 * 1024;   // of a CU's 160 KB, less the reductions' static part
 // the halo entries that fit beside rpt rows per thread
 constexpr int res_max_halo(int code, int rpt) {
-  const size_t left = kResLds - res_lds_bytes(code, rpt, 0);
+  const size_t fixed = code == kResGmres ? ((kResGmresK + 1) * kResGmresK + 5 * (kResGmresK + 3)) * sizeof(double) : 0;
+  const size_t left = kResLds - fixed - res_lds_bytes(code, rpt, 0);
   const size_t nh = left / res_halo_bytes(code);
   return nh < (size_t)kResMaxHalo ? (int)nh : kResMaxHalo;
 }

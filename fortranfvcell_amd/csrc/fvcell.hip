@@ -379,11 +379,13 @@ int drive_batches(DevState &d, hipStream_t s, int maxit, Iter &&iteration, State
   return FVC_OK;
 }
 
-// The on-chip PCG / BiCGSTAB (fvc_resident.h).  Measured on MI355X against one
+// The on-chip solvers (fvc_resident.h).  Measured on MI355X against one
 // kernel per phase, whole solves to a true residual of 1e-10: PCG 4,096 rows
 // 3.93 -> 1.27 ms, 429,713 rows 77.8 -> 22.8; BiCGSTAB 12,707 rows 0.92 ->
 // 0.37, 1,048,576 rows 2.61 -> 0.77.  Mixed PCG, us per FP32 iteration: 5,120
-// rows 8.2 -> 3.3, 160,860 12.2 -> 5.0, 1,048,576 18.1 -> 7.0.
+// rows 8.2 -> 3.3, 160,860 12.2 -> 5.0, 1,048,576 18.1 -> 7.0.  GMRES(30) with
+// modified Gram-Schmidt, whole solves: 4,096 rows 9.7 -> 2.2 ms, 160,860 17.9 ->
+// 4.7, 1,048,576 24.8 -> 6.8.
 constexpr bool resident_format(int F) { return F == F_ELL4 || F == F_ELL3 || F == F_CSRD; }
 
 template <int F, int Code>
@@ -401,10 +403,11 @@ const void *resident_fn(int rpt) {
 
 // Solves on chip if the system fits; *done says whether it did (else the
 // caller solves it one kernel per phase).  part: kResPartWords words; rows:
-// at least 4 neq words (vectors that the caller does not need yet).
+// at least 4 neq words (vectors that the caller does not need yet).  GMRES:
+// gv, the basis columns, ld apart.
 template <int F>
 int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned *ctr, res_word *part, res_word *rows,
-                 fvc_stats *stats, hipStream_t s, bool *done) {
+                 fvc_stats *stats, hipStream_t s, bool *done, double *gv = nullptr, size_t ld = 0) {
   *done = false;
   if constexpr (!resident_format(F)) {
     return FVC_OK;
@@ -416,8 +419,10 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
     a.A = in.A; a.st = st; a.m = in.m; a.x = in.x; a.b = in.b;
     a.tol = in.tol; a.maxit = in.maxit; a.x0_zero = in.x0_zero; a.stop_rule = in.stop_rule;
     a.delta = in.refresh_drop; a.max_inner = in.refresh_every;
+    a.gv = gv; a.ld = ld; a.k = in.gmres_k;
     const void *fn = kind == kResPcg        ? resident_fn<F, kResPcg>(sh.rpt)
                      : kind == kResBicgstab ? resident_fn<F, kResBicgstab>(sh.rpt)
+                     : kind == kResGmres    ? resident_fn<F, kResGmres>(sh.rpt)
                                             : resident_fn<F, kResMixedPcg>(sh.rpt);
     const int hmax = sh.blocks > 1 ? res_max_halo(kind, sh.rpt) : 0;
     const size_t lds = res_lds_bytes(kind, sh.rpt, hmax);
@@ -554,8 +559,12 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   // the on-chip solver's words for partial sums, where the fixed workspace
   // has room for them (its limit stays that of the engines below)
   size_t res_part = align_up(kResPartWords * sizeof(res_word));
-  if (d.noalloc && bytes + res_part > kScratchBytes) res_part = 0;
-  bytes += res_part;
+  // (GMRES with modified Gram-Schmidt: also the words of the rows, since the
+  // basis takes the vectors)
+  const bool res_gmres = in.code == FVC_GMRES && !cgs && !lag && k <= kResGmresK;
+  size_t res_rows = res_gmres ? align_up(4 * n * sizeof(res_word)) : 0;
+  if (d.noalloc && bytes + res_part + res_rows > kScratchBytes) res_part = res_rows = 0;
+  bytes += res_part + res_rows;
   char *ws = nullptr;
   if ((rc = workspace(d, bytes, &ws))) return rc;
   Carve cv{ws, bytes};
@@ -563,6 +572,7 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   KState *st = cv.take<KState>(1);
   double *partials = cv.take<double>(npart);
   res_word *part = cv.take<res_word>(res_part / sizeof(res_word));
+  res_word *grows = cv.take<res_word>(res_rows / sizeof(res_word));
   // deferred reductions (kernel-per-phase engine of the fused methods)
   Defer dfr{cv.take<KState>(2), cv.take<double>(2 * kMaxK * (size_t)G), 0};
   double *vec[kMaxGmresK + 1];
@@ -574,11 +584,12 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   if (!cv.fits()) return carve_overflow(cv);
   // On chip where the launch is the library's choice; options that shape it
   // keep the engines they were written for.
-  if (in.engine == FVC_ENGINE_AUTO && in.code != FVC_GMRES && fused && in.bs == 0 && in.G_req == 0 &&
+  if (in.engine == FVC_ENGINE_AUTO && (res_gmres || in.code != FVC_GMRES) && fused && in.bs == 0 && in.G_req == 0 &&
       in.barrier == 0 && in.row_order == 0 && !in.lanex && res_part) {
     bool done = false;
-    rc = run_resident<F>(d, in, in.code == FVC_PCG ? kResPcg : kResBicgstab, st, ctr, part,
-                         reinterpret_cast<res_word *>(vec[0]), stats, s, &done);
+    const int kind = res_gmres ? kResGmres : in.code == FVC_PCG ? kResPcg : kResBicgstab;
+    rc = run_resident<F>(d, in, kind, st, ctr, part, res_gmres ? grows : reinterpret_cast<res_word *>(vec[0]), stats, s,
+                         &done, vec[0], nvec > 1 ? (size_t)(vec[1] - vec[0]) : n);
     if (rc || done) return rc;
   }
   const bool may_fall_back = persistent && in.engine == FVC_ENGINE_AUTO;

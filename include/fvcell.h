@@ -73,12 +73,13 @@ extern "C" {
                                    cycles                                                    */
 
 /* Engines. */
-#define FVC_ENGINE_AUTO 0        /* PCG and BiCGSTAB (fused, FP64, ELLPACK of width 3 or 4
-                                    or CSRD rows of at most four off-diagonals, none of
-                                    the options that shape a launch set): on chip in one
+#define FVC_ENGINE_AUTO 0        /* PCG (FP64 and mixed), BiCGSTAB (FP64) and GMRES (FP64,
+                                    FVC_ORTH_MGS, k <= 32) on ELLPACK of width 3 or 4 or
+                                    CSRD rows of at most four off-diagonals, with none of
+                                    the options that shape a launch set: on chip in one
                                     launch where the system fits (up to 1,048,576 rows on
-                                    256 CUs; stats.engine then says PERSISTENT), else
-                                    KERNELS.  GMRES: PERSISTENT                          */
+                                    256 CUs; stats.engine then says PERSISTENT).  Else
+                                    KERNELS, GMRES PERSISTENT                            */
 #define FVC_ENGINE_KERNELS 1     /* one kernel per phase; fused recurrences sum the block
                                     partials at the next launch, the others in the last
                                     block of the launch                                 */

@@ -215,3 +215,38 @@ def test_resident_mixed_declines(fvc):
     assert st["engine"] == fvc.ENGINE_KERNELS and st["status"] == 0
     x2, st2 = fvc.solve(f, fvc.PCG, x0=x, tol=1e-10, precision=fvc.PREC_MIXED, x0_rule=fvc.X0_GIVEN)
     assert st2["iterations"] == 0 and np.array_equal(x2, x)
+
+
+@pytest.mark.parametrize("kind,nx,ny", SHAPES[2:])
+@pytest.mark.parametrize("k", [1, 2, 3, 15, 32])
+def test_resident_gmres_matches_kernels(fvc, kind, nx, ny, k):
+    """Modified Gram-Schmidt on chip against one kernel per phase: the same
+    steps, and after one cycle x to 1e-11 (sums in another order, of
+    vectors of norm one, over k projections); the restart lengths around the
+    prefetch of columns, and the longest that the chip takes."""
+    m = _mesh(kind, nx, ny)
+    s = P.advdiff_system(m, dt=0.005, under_relax=0.8)
+    for lay in (P.to_ell, P.to_csrd):
+        f = lay(s)
+        for opt in (dict(maxit=1, stop_rule=fvc.STOP_REFERENCE), dict(maxit=400, stop_rule=fvc.STOP_RELRES)):
+            if opt["maxit"] > 1 and (k < 15 or m.neq > 60000):
+                continue
+            print(f"resident gmres({k}) {kind} {nx}x{ny} neq={m.neq} {lay.__name__} {opt}", flush=True)
+            kw = dict(tol=1e-10, gmres_k=k, **opt)
+            xa, sa = fvc.solve(f, fvc.GMRES, **kw)
+            xk, sk = fvc.solve(f, fvc.GMRES, engine=fvc.ENGINE_KERNELS, **kw)
+            assert (sa["status"], sa["iterations"], sa["inner_iterations"]) == \
+                (sk["status"], sk["iterations"], sk["inner_iterations"]), (sa, sk)
+            assert _rel(xa, xk) <= (1e-11 if opt["maxit"] == 1 else 1e-8)
+            assert abs(sa["energy"] - sk["energy"]) <= 1e-8 * abs(sk["energy"])
+            if opt["maxit"] > 1:
+                assert sa["true_relres"] <= 1e-10
+
+
+def test_resident_gmres_exact_start(fvc):
+    """A zero right-hand side: the exact solution at once, in either engine."""
+    for n in (20, 70):
+        f = P.to_ell(P.config_advdiff(n, peclet_max=10.0))
+        x, st = fvc.solve(f, fvc.GMRES, b=np.zeros(n * n), tol=1e-10, gmres_k=10)
+        xk, sk = fvc.solve(f, fvc.GMRES, b=np.zeros(n * n), tol=1e-10, gmres_k=10, engine=fvc.ENGINE_KERNELS)
+        assert (st["status"], st["iterations"]) == (sk["status"], sk["iterations"]) and not x.any() and not xk.any()
