@@ -456,6 +456,37 @@ __device__ void cg1_rows(const Cg1Args &a, int ph, const KState *S, double *v,
   }
 }
 
+// What CG1_ITER's scalar part reads of the state: an engine whose block waits
+// for the totals loads it meanwhile.
+struct Cg1Scalars {
+  double d, alpha, conv;
+  int iter;
+};
+__device__ __forceinline__ Cg1Scalars cg1_scalars(const KState *st) {
+  return {st->d, st->alpha, st->conv, st->iter};
+}
+// Every block waits for this one thread, so the quotients and the root that do
+// not depend on each other are written without a branch between them and run
+// side by side.
+__device__ __forceinline__ void cg1_iter_epi(const Cg1Args &a, const Cg1Scalars &c, KState *st, const double *t) {
+  const int j = c.iter + 1;
+  const double gamma = t[0];
+  const double beta = gamma / c.d;
+  const double den = t[1] - beta * (gamma / c.alpha);
+  const double alpha = gamma / den;
+  const double last = sqrt(a.stop_rule == 1 ? t[2] : fabs(gamma));
+  st->alpha = alpha;
+  st->beta = beta;
+  st->d = gamma;
+  st->rnorm2 = t[2];
+  st->iter = j;
+  st->last = last;
+  const bool conv = a.stop_rule == 1 ? last <= c.conv : last < c.conv;   // src/Iterativos.f:73
+  const bool lost = !finite(gamma) | !finite(beta), zero = den == 0.0, over = !finite(alpha);
+  st->status = conv ? S_OK : lost ? S_NONFINITE : zero ? S_BREAKDOWN : over ? S_NONFINITE : S_MAXIT;
+  st->done = (conv | lost | zero | over | (j >= a.maxit)) ? 1 : 0;
+}
+
 __device__ inline void cg1_epi(const Cg1Args &a, int ph, KState *st, const double *t) {
   if (ph == CG1_SETUP) {
     st->d = t[0];
@@ -481,29 +512,7 @@ __device__ inline void cg1_epi(const Cg1Args &a, int ph, KState *st, const doubl
     if (t[0] == 0.0) { st->status = S_BREAKDOWN; st->done = 1; }
     else if (!finite(st->alpha)) { st->status = S_NONFINITE; st->done = 1; }
   } else if (ph == CG1_ITER) {
-    const int j = st->iter + 1;
-    const double gamma = t[0];
-    const double beta = gamma / st->d;
-    const double den = t[1] - beta * gamma / st->alpha;
-    const double alpha = gamma / den;
-    st->beta = beta;
-    st->alpha = alpha;
-    st->d = gamma;
-    st->rnorm2 = t[2];
-    st->iter = j;
-    bool conv;
-    if (a.stop_rule == 1) {
-      st->last = sqrt(t[2]);
-      conv = st->last <= st->conv;
-    } else {
-      st->last = sqrt(fabs(gamma));
-      conv = st->last < st->conv;   // src/Iterativos.f:73
-    }
-    if (conv) { st->status = S_OK; st->done = 1; }
-    else if (!finite(gamma) || !finite(beta)) { st->status = S_NONFINITE; st->done = 1; }
-    else if (den == 0.0) { st->status = S_BREAKDOWN; st->done = 1; }
-    else if (!finite(alpha)) { st->status = S_NONFINITE; st->done = 1; }
-    else if (j >= a.maxit) { st->status = S_MAXIT; st->done = 1; }
+    cg1_iter_epi(a, cg1_scalars(st), st, t);
   } else {
     st->energy = t[0];
     st->res2 = t[1];
@@ -937,6 +946,45 @@ __device__ void bicg2_rows(const Bicg2Args &a, int ph, const KState *S, double *
   else sweep(LaneX<false>{});
 }
 
+// The scalar parts of P and Q (see cg1_iter_epi).
+struct Bicg2Scalars {
+  double d, rr0, alpha, conv;
+  int iter;
+};
+__device__ __forceinline__ Bicg2Scalars bicg2_scalars(const KState *st) {
+  return {st->d, st->rr0, st->alpha, st->conv, st->iter};
+}
+__device__ __forceinline__ void bicg2_p_epi(const Bicg2Args &a, const Bicg2Scalars &c, KState *st, const double *t) {
+  const int j = c.iter + 1;
+  const double alpha = c.rr0 / t[0];
+  // the stop test of iteration j-1 (src/Iterativos.f:188-190)
+  const double beta1 = t[1] / c.d;
+  const double last = sqrt(a.stop_rule == 1 ? t[2] : fabs(beta1));
+  const bool tests = j > 1;
+  const bool conv = tests & (a.stop_rule == 1 ? last <= c.conv : last < c.conv);
+  const bool lost = tests & !finite(beta1), full = tests & (j - 1 >= a.maxit);
+  const bool zero = t[0] == 0.0, over = !finite(alpha);
+  if (tests) {
+    st->rnorm2 = t[2];
+    st->last = last;
+  }
+  st->alpha = alpha;
+  st->status = conv ? S_OK : lost ? S_NONFINITE : full ? S_MAXIT : zero ? S_BREAKDOWN : over ? S_NONFINITE : S_MAXIT;
+  st->done = (conv | lost | full | zero | over) ? 1 : 0;
+}
+__device__ __forceinline__ void bicg2_q_epi(const Bicg2Scalars &c, KState *st, const double *t) {
+  const double w = t[0] / t[1];
+  const double rho = t[2] - w * t[3];
+  const double beta = (rho / c.rr0) * (c.alpha / w);
+  st->omega = w;
+  st->beta = beta;
+  st->rr0 = rho;
+  st->iter = c.iter + 1;
+  const bool zero = (t[1] == 0.0) | (w == 0.0), over = !finite(w) | !finite(beta);
+  st->status = zero ? S_BREAKDOWN : over ? S_NONFINITE : S_MAXIT;
+  st->done = (zero | over) ? 1 : 0;
+}
+
 __device__ inline void bicg2_epi(const Bicg2Args &a, int ph, KState *st, const double *t) {
   if (ph == B2_SETUP) {
     st->d = t[0];
@@ -958,37 +1006,9 @@ __device__ inline void bicg2_epi(const Bicg2Args &a, int ph, KState *st, const d
     if (!finite(t[0])) { st->status = S_NONFINITE; st->done = 1; }
     if (a.maxit <= 0 && !st->done) st->done = 1;
   } else if (ph == B2_P) {
-    const int j = st->iter + 1;
-    if (j > 1) {
-      // the stop test of iteration j-1 (src/Iterativos.f:188-190)
-      const double beta1 = t[1] / st->d;
-      st->rnorm2 = t[2];
-      bool conv;
-      if (a.stop_rule == 1) {
-        st->last = sqrt(t[2]);
-        conv = st->last <= st->conv;
-      } else {
-        st->last = sqrt(fabs(beta1));
-        conv = st->last < st->conv;
-      }
-      if (conv) { st->status = S_OK; st->done = 1; return; }
-      if (!finite(beta1)) { st->status = S_NONFINITE; st->done = 1; return; }
-      if (j - 1 >= a.maxit) { st->status = S_MAXIT; st->done = 1; return; }
-    }
-    const double alpha = st->rr0 / t[0];
-    st->alpha = alpha;
-    if (t[0] == 0.0) { st->status = S_BREAKDOWN; st->done = 1; }
-    else if (!finite(alpha)) { st->status = S_NONFINITE; st->done = 1; }
+    bicg2_p_epi(a, bicg2_scalars(st), st, t);
   } else if (ph == B2_Q) {
-    const double w = t[0] / t[1];
-    const double rho = t[2] - w * t[3];
-    const double beta = (rho / st->rr0) * (st->alpha / w);
-    st->omega = w;
-    st->beta = beta;
-    st->rr0 = rho;
-    st->iter = st->iter + 1;
-    if (t[1] == 0.0 || w == 0.0) { st->status = S_BREAKDOWN; st->done = 1; }
-    else if (!finite(w) || !finite(beta)) { st->status = S_NONFINITE; st->done = 1; }
+    bicg2_q_epi(bicg2_scalars(st), st, t);
   } else {
     st->energy = t[0];
     st->res2 = t[1];

@@ -335,6 +335,38 @@ __device__ __forceinline__ void mixed_rows(const MixedArgs &a, int ph, const KSt
   }
 }
 
+// The scalar part of an FP32 iteration, what it reads of the state loaded (and
+// the roots of it taken) beforehand (see cg1_iter_epi).
+struct MixedScalars {
+  double limit, floor;   // the estimate and the recursive residual that end the inner solve
+  int iter, inner;
+};
+__device__ __forceinline__ MixedScalars mixed_scalars(const MixedArgs &a, const KState *st) {
+  return {st->conv * st->tscale, a.delta * sqrt(st->rr0), st->iter, st->inner};
+}
+__device__ __forceinline__ void mixed_a_epi(const MixedArgs &a, const MixedScalars &c, KState *st, const double *t) {
+  const double sig = t[0], tau = t[1], th = t[2], rho = t[3];
+  const int j = c.iter + 1, inner = c.inner + 1;
+  const double alpha = rho / sig;
+  const double rho1 = rho - 2.0 * alpha * tau + alpha * alpha * th;
+  const double beta = rho1 / rho;
+  const double est = sqrt(t[4]);
+  const bool ok = (sig != 0.0) & (rho != 0.0) & finite(alpha) & finite(beta);
+  st->iter = j;
+  st->inner = inner;
+  st->last = est;
+  st->d = rho;
+  st->alpha = ok ? alpha : 0.0;
+  st->beta = ok ? beta : 0.0;
+  st->step_i = 0;
+  st->ni = 0;
+  const bool tolhit = (inner > 1) & (est <= c.limit);
+  const bool drop = sqrt(fmax(rho1, 0.0)) < c.floor;
+  st->inner_done = tolhit ? 1 : 0;
+  const bool upd = !ok | tolhit | drop | (inner >= a.max_inner) | (j >= a.maxit);
+  st->next = upd ? MX_X : MX_A;
+}
+
 __device__ __forceinline__ void mixed_epi(const MixedArgs &a, int ph, KState *st, const double *t) {
   if (ph == MX_SETUP || ph == MX_R) {
     const double tr = sqrt(t[1]);
@@ -367,26 +399,7 @@ __device__ __forceinline__ void mixed_epi(const MixedArgs &a, int ph, KState *st
     else if (!finite(t[0]) || !finite(t[1])) { st->status = S_NONFINITE; st->done = 1; }
     else if (st->iter >= a.maxit) { st->status = S_MAXIT; st->done = 1; }
   } else if (ph == MX_A) {
-    const double sig = t[0], tau = t[1], th = t[2], rho = t[3];
-    const int j = st->iter + 1;
-    st->iter = j;
-    st->inner = st->inner + 1;
-    const double alpha = rho / sig;
-    const double rho1 = rho - 2.0 * alpha * tau + alpha * alpha * th;
-    const double beta = rho1 / rho;
-    const double est = sqrt(t[4]);
-    const bool ok = sig != 0.0 && rho != 0.0 && finite(alpha) && finite(beta);
-    st->last = est;
-    st->d = rho;
-    st->alpha = ok ? alpha : 0.0;
-    st->beta = ok ? beta : 0.0;
-    st->step_i = 0;
-    st->ni = 0;
-    const bool tolhit = st->inner > 1 && est <= st->conv * st->tscale;
-    const bool drop = sqrt(fmax(rho1, 0.0)) < a.delta * sqrt(st->rr0);
-    st->inner_done = tolhit ? 1 : 0;
-    const bool upd = !ok || tolhit || drop || st->inner >= a.max_inner || j >= a.maxit;
-    st->next = upd ? MX_X : MX_A;
+    mixed_a_epi(a, mixed_scalars(a, st), st, t);
   } else if (ph == MX_X) {
     st->next = MX_R;
   } else {

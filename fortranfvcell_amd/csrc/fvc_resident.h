@@ -22,10 +22,13 @@
 // ahead of any other (it needs every block's partial sums), so a word is
 // never overwritten before it was read.
 //
-// Measured on MI355X (us per exchange, 512 threads a block, three sums):
-// 3.3 at 8 blocks with 64 halo rows each side, 3.7 at 64 blocks, 4.3 at 256
-// with 64..256 halo rows a side, 8.0 at 256 with 1,024; a launch per phase
-// costs 9 us at 4,096 rows and 26-30 us at a million.  The halo volume is
+// Measured on MI355X (us per PCG iteration, one exchange each): 1.1 in one
+// block of 400 rows, 2.1 at 5,120 rows (10 blocks), 2.4 at 32,300 (40), 3.1 at
+// 160,860 (168), 4.9 at 1,048,576 (256); a launch per phase costs 9 us at 4,096
+// rows and 26-30 us at a million.  An iteration of one block is a chain of
+// latencies (LDS, barriers, quotients), one of many adds the flight of its words,
+// twice beyond 64 blocks; with 1,024 halo rows a side instead of 256 the flight
+// was twice as long.  The halo volume is
 // what makes the difference at 256 blocks, so rows are dealt in tiles of the
 // mesh where the columns show one (ResPlan), else in contiguous strips.
 #pragma once
@@ -161,38 +164,64 @@ __device__ __forceinline__ res_word res_load(const res_word *p) {
 __device__ __forceinline__ void res_store(res_word *p, res_word v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// A double as two words: the exchange's number in the low half, half of the
-// double in the high one.
-__device__ __forceinline__ void res_put(res_word *p, double v, unsigned ep) {
+// A double as two words, `apart` from each other: the exchange's number in the
+// low half, half of the double in the high one.  Sums keep their low halves
+// together and their high halves together, so that a wave's load of either is
+// of whole lines (half as many lines to a look: 4 % of a PCG iteration at 160
+// blocks and above); a row's two words are neighbours, for a tile's columns are
+// published row by row.
+__device__ __forceinline__ void res_put(res_word *p, size_t apart, double v, unsigned ep) {
   const res_word u = __builtin_bit_cast(res_word, v);
   res_store(p, (u << 32) | ep);
-  res_store(p + 1, (u & 0xffffffff00000000ull) | ep);
+  res_store(p + apart, (u & 0xffffffff00000000ull) | ep);
 }
 __device__ __forceinline__ double res_get(res_word lo, res_word hi) {
   return __builtin_bit_cast(double, (hi & 0xffffffff00000000ull) | (lo >> 32));
 }
 
-// The sum over a wavefront, in its last lane: row shifts and row broadcasts
-// in the ALU's data path (DPP) instead of the shuffles' trips through LDS,
-// which an iteration would wait for twice.
-template <int Ctrl, int RowMask>
+// Sums over a wavefront in the ALU's data path (row shifts by DPP, swaps of
+// halves and of rows) instead of the shuffles' trips through LDS.  Two waves
+// share a SIMD, so the sums of every wave at once are bound by instructions: K
+// values one by one take 6 K steps of three, while a swap halves the lanes of
+// two values at the price of one, and up to four values are one after two
+// swaps: 7 steps instead of 18 or 24.
+template <int Ctrl>
 __device__ __forceinline__ double res_dpp_add(double v) {
   const res_word u = __builtin_bit_cast(res_word, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, Ctrl, RowMask, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), Ctrl, RowMask, 0xF, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, Ctrl, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), Ctrl, 0xF, 0xF, true);
   return v + __builtin_bit_cast(double, ((res_word)(unsigned)hi << 32) | (unsigned)lo);
 }
 __device__ __forceinline__ double res_row_sum(double v) {   // of each 16 lanes, in the last
-  v = res_dpp_add<0x111, 0xF>(v);   // row_shr:1
-  v = res_dpp_add<0x112, 0xF>(v);   // row_shr:2
-  v = res_dpp_add<0x114, 0xF>(v);   // row_shr:4
-  return res_dpp_add<0x118, 0xF>(v);   // row_shr:8
+  v = res_dpp_add<0x111>(v);   // row_shr:1
+  v = res_dpp_add<0x112>(v);   // row_shr:2
+  v = res_dpp_add<0x114>(v);   // row_shr:4
+  return res_dpp_add<0x118>(v);   // row_shr:8
 }
-__device__ __forceinline__ double res_wave_sum(double v) {
-  v = res_row_sum(v);
-  v = res_dpp_add<0x142, 0xA>(v);   // row_bcast:15 into rows 1 and 3
-  v = res_dpp_add<0x143, 0xC>(v);   // row_bcast:31 into rows 2 and 3
-  return v;
+// a's halves (rows) added in the lower half (even rows), b's in the other
+template <bool Halves>
+__device__ __forceinline__ double res_fold(double a, double b) {
+  const res_word u = __builtin_bit_cast(res_word, a), w = __builtin_bit_cast(res_word, b);
+  const auto swap = [](unsigned x, unsigned y) {
+    if constexpr (Halves) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  };
+  const auto lo = swap((unsigned)u, (unsigned)w), hi = swap((unsigned)(u >> 32), (unsigned)(w >> 32));
+  return __builtin_bit_cast(double, ((res_word)hi[0] << 32) | lo[0]) +
+         __builtin_bit_cast(double, ((res_word)hi[1] << 32) | lo[1]);
+}
+// The sums of K <= 4 values: value k in the last lane of row res_sum_row<K>(k).
+template <int K>
+__device__ __forceinline__ constexpr int res_sum_row(int k) { return K == 1 ? 3 - k : ((k & 1) << 1) | (k >> 1); }
+template <int K>
+__device__ __forceinline__ double res_wave_sums(const double *v) {
+  if constexpr (K == 1) {
+    const double r = res_dpp_add<0x142>(res_row_sum(v[0]));   // row_bcast:15: two rows in the last lane of row 3, and of row 1,
+    return res_dpp_add<0x143>(r);                             // which row_bcast:31 takes there
+  }
+  const double a = res_fold<true>(v[0], K > 1 ? v[K > 1 ? 1 : 0] : 0.0);
+  const double b = K > 2 ? res_fold<true>(v[K > 2 ? 2 : 0], K > 3 ? v[K > 3 ? 3 : 0] : 0.0) : 0.0;
+  return res_row_sum(res_fold<false>(a, b));
 }
 __device__ __forceinline__ double res_lane(double v, int lane) {
   const res_word u = __builtin_bit_cast(res_word, v);
@@ -201,12 +230,24 @@ __device__ __forceinline__ double res_lane(double v, int lane) {
   return __builtin_bit_cast(double, ((res_word)hi << 32) | lo);
 }
 
-// Waits for up to E doubles (or floats, a word each), at(q) being the address of the q-th or null;
-// all loads of a poll are issued together.  False if the wait expired, after
-// `limit` polls or when another wait did (*err).
-template <int E, class T, class At>
-__device__ __forceinline__ bool res_wait(unsigned ep, T *v, unsigned limit, const unsigned *err, At &&at) {
+// How long a wave sleeps, in units of 64 cycles, before it looks for the first
+// time: a look takes about as long as a word takes to arrive, so one that comes
+// too early costs a second one and slows the words of others.  The sums of a
+// flat exchange or of a group and the halo's rows are one word's flight away,
+// the group totals two.  PCG, us per iteration, without any and with these:
+// 32,300 rows (40 blocks) 2.73 / 2.41, 160,860 (168) 3.44 / 3.07, 429,713 (224)
+// 4.21 / 3.69, 1,048,576 (256) 5.39 / 4.97; four units more or less at any of
+// them changes that by up to 3 %.
+constexpr int kResNapSums = 10, kResNapGroup = 8, kResNapRows = 14, kResNapTotals = 46;
+
+// Waits for up to E doubles (or floats, a word each), at(q) being the address
+// of the q-th's low half or null, the other half `apart` words on; all loads of
+// a poll are issued together.  False if the wait expired, after `limit` polls
+// or when another wait did (*err).
+template <int Nap, int E, class T, class At>
+__device__ __forceinline__ bool res_wait(unsigned ep, T *v, size_t apart, unsigned limit, const unsigned *err, At &&at) {
   res_word lo[E], hi[E];
+  __builtin_amdgcn_s_sleep(Nap);
   for (unsigned spins = 0;;) {
 #pragma unroll
     for (int q = 0; q < E; ++q) {
@@ -214,7 +255,7 @@ __device__ __forceinline__ bool res_wait(unsigned ep, T *v, unsigned limit, cons
       lo[q] = hi[q] = ep;
       if (p) {
         lo[q] = res_load(p);
-        if constexpr (sizeof(T) == 8) hi[q] = res_load(p + 1);
+        if constexpr (sizeof(T) == 8) hi[q] = res_load(p + apart);
       }
     }
     bool ok = true;
@@ -271,6 +312,8 @@ struct ResNet {
   int nh, nb;
   unsigned ep = 0;
   unsigned pub = 0;        // bit k: another block reads the thread's row k
+  double sc[3];            // alpha, beta, omega of the last exchange that read them
+  int done = 0;
 
   __device__ __forceinline__ ResNet(const ResArgs &args) : a(args) {}
 
@@ -283,19 +326,19 @@ struct ResNet {
   __device__ __forceinline__ void publish(int k, T v) const {
     if (!(pub >> k & 1u)) return;
     res_word *to = row_words<T>(ep + 1, row[threadIdx.x + k * NT]);
-    if constexpr (sizeof(T) == 8) res_put(to, v, ep + 1);
+    if constexpr (sizeof(T) == 8) res_put(to, 1, v, ep + 1);
     else res_store(to, ((res_word)__builtin_bit_cast(unsigned, v) << 32) | (ep + 1));
   }
 
   // The K sums of up to 16 members, 16 lanes to a value.
-  template <int K, int E>
+  template <int Nap, int K, int E>
   __device__ __forceinline__ void group_sums(const res_word *from, int members, unsigned limit, double *tot) {
     const int lane = (int)threadIdx.x & (kWave - 1);
     double g[E];
     const bool in = (lane & 15) < members;
-    if (!res_wait<E>(ep, g, limit, a.err, [&](int q) -> const res_word * {
+    if (!res_wait<Nap, E>(ep, g, kResGroupSums, limit, a.err, [&](int q) -> const res_word * {
           const int e = lane + q * kWave;
-          return in && e < 16 * K ? from + 2 * (size_t)e : nullptr;
+          return in && e < 16 * K ? from + e : nullptr;
         }))
       *bad = 1;
 #pragma unroll
@@ -308,17 +351,23 @@ struct ResNet {
 
   // One exchange: the block's K sums to every block and theirs here, added in
   // the order of the blocks; the published rows of the halo into hdst (LDS,
-  // nh entries; null: none); then epi(totals) on thread 0.  publish() goes
-  // before.  Some waves wait for the sums and the others for the halo.
-  // False if a wait expired.
-  template <int K, class T, class Epi>
-  __device__ __forceinline__ bool exchange(const double *v, T *hdst, Epi &&epi) {
+  // nh entries; null: none); then epi()(totals) on thread 0, epi() itself
+  // while the totals are on their way.  publish() goes before; work() is what
+  // no other block waits for and is done meanwhile.  The first N scalars of
+  // the new state are read on the way out (sc, done).  Some waves wait for the
+  // sums and the others for the halo.  False if a wait expired.
+  template <int K, int N, class T, class Epi, class Work>
+  __device__ __forceinline__ bool exchange(const double *v, T *hdst, Epi &&epi, Work &&work) {
     ++ep;
     const int t = (int)threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      const double s = res_wave_sum(v[k]);
-      if (lane == kWave - 1) red[k * kMaxWaves + wid] = s;
+    {
+      const double s = res_wave_sums<(K < 4 ? K : 4)>(v);
+      const int k = res_sum_row<(K < 4 ? K : 4)>(lane >> 4);
+      if ((lane & 15) == 15 && k < K) red[k * kMaxWaves + wid] = s;
+      if constexpr (K > 4) {
+        const double s4 = res_wave_sums<1>(v + 4);
+        if (lane == kWave - 1) red[4 * kMaxWaves + wid] = s4;
+      }
     }
     lds_barrier();
     static_assert(K <= kResSums, "a lane adds at most two of the groups' sums");
@@ -341,39 +390,49 @@ struct ResNet {
         own = q[0];
 #pragma unroll
         for (int w = 1; w < NT / kWave; ++w) own += q[w];
-        const int to = wide ? (map.c >> 4) * kResGroupSums + lane * 16 + (map.c & 15) : lane * kWave + map.c;
-        if (nb > 1) res_put(part + 2 * (size_t)to, own, ep);
+        const int to = wide ? (map.c >> 4) * 2 * kResGroupSums + lane * 16 + (map.c & 15) : lane * 2 * kWave + map.c;
+        if (nb > 1) res_put(part + to, wide ? kResGroupSums : kWave, own, ep);
       }
+      auto close = epi();
+      work();
       double tot[K];
       if (nb == 1) {
 #pragma unroll
         for (int k = 0; k < K; ++k) tot[k] = res_lane(own, k);
       } else if (!wide) {
         double pv[K];
-        if (!res_wait<K>(ep, pv, limit, a.err, [&](int q) -> const res_word * {
-              return lane < nb ? part + 2 * ((size_t)q * kWave + lane) : nullptr;
+        if (!res_wait<kResNapSums, K>(ep, pv, kWave, limit, a.err, [&](int q) -> const res_word * {
+              return lane < nb ? part + (q * 2 * kWave + lane) : nullptr;
             }))
           *bad = 1;
 #pragma unroll
-        for (int k = 0; k < K; ++k) tot[k] = res_lane(res_wave_sum(lane < nb ? pv[k] : 0.0), kWave - 1);
+        for (int k = 0; k < K; ++k) pv[k] = lane < nb ? pv[k] : 0.0;
+        const double s = res_wave_sums<(K < 4 ? K : 4)>(pv);
+#pragma unroll
+        for (int k = 0; k < (K < 4 ? K : 4); ++k) tot[k] = res_lane(s, 16 * res_sum_row<(K < 4 ? K : 4)>(k) + 15);
+        if constexpr (K > 4) tot[4] = res_lane(res_wave_sums<1>(pv + 4), kWave - 1);
       } else {
-        group_sums<K, E>(part + 2 * (size_t)(kResGroups + (map.c >> 4)) * kResGroupSums, (nb + 15) / 16, limit, tot);
+        group_sums<kResNapTotals, K, E>(part + 2 * (size_t)(kResGroups + (map.c >> 4)) * kResGroupSums, (nb + 15) / 16, limit, tot);
       }
-      if (lane == 0) epi(tot);
+      if (lane == 0) close(tot);
     } else if (leads && wid == 1) {
+      work();
       const int grp = map.c >> 4;
       double tot[K];
-      group_sums<K, E>(part + 2 * (size_t)grp * kResGroupSums, nb - 16 * grp, limit, tot);
+      group_sums<kResNapGroup, K, E>(part + 2 * (size_t)grp * kResGroupSums, nb - 16 * grp, limit, tot);
       // lane (value, group): that group's copy, all in one store (everyone waits
       // for this wave: a store per value was 1.3 us slower at 256 blocks)
       double mine = 0.0;
 #pragma unroll
       for (int k = 0; k < (K < 4 ? K : 4); ++k)
         if (lane >> 4 == k) mine = tot[k];
-      res_word *to = part + 2 * (size_t)((kResGroups + (lane & 15)) * kResGroupSums + grp);
-      if (lane < 16 * K && (lane & 15) < (nb + 15) / 16) res_put(to + 2 * (lane & 48), mine, ep);
-      if (K > 4 && lane < (nb + 15) / 16) res_put(to + 2 * 64, tot[K - 1], ep);
-    } else if (nb > 1 && hdst && wid >= waiting) {
+      res_word *to = part + 2 * (size_t)((kResGroups + (lane & 15)) * kResGroupSums) + grp;
+      if (lane < 16 * K && (lane & 15) < (nb + 15) / 16) res_put(to + (lane & 48), kResGroupSums, mine, ep);
+      if (K > 4 && lane < (nb + 15) / 16) res_put(to + 64, kResGroupSums, tot[K - 1], ep);
+    } else {
+      work();
+    }
+    if (nb > 1 && hdst && wid >= waiting) {
       const int ht = NT - waiting * kWave, h0 = t - waiting * kWave;
       auto from = [&](int h) -> const res_word * {
         const int j = h < nh ? hrow[h] : -1;
@@ -382,8 +441,8 @@ struct ResNet {
       for (int base = 0; base < nh; base += ht * HE) {
         T hv[HE];
         const bool few = nh - base <= ht;
-        const bool ok = few ? res_wait<1>(ep, hv, limit, a.err, [&](int) { return from(base + h0); })
-                            : res_wait<HE>(ep, hv, limit, a.err, [&](int q) { return from(base + h0 + q * ht); });
+        const bool ok = few ? res_wait<kResNapRows, 1>(ep, hv, 1, limit, a.err, [&](int) { return from(base + h0); })
+                            : res_wait<kResNapRows, HE>(ep, hv, 1, limit, a.err, [&](int q) { return from(base + h0 + q * ht); });
         if (!ok) {
           *bad = 1;
           break;
@@ -396,12 +455,22 @@ struct ResNet {
       }
     }
     lds_barrier();
-    if (nb == 1) return true;
-    if (*bad) {
-      if (t == 0) st_relaxed(a.err, 1u);
-      return false;
+    // all at once: each read is a trip to LDS
+    int lost = nb > 1 ? *bad : 0;
+    if constexpr (N > 0) {
+      done = S->done;
+      sc[0] = S->alpha;
+      sc[1] = N > 1 ? S->beta : 0.0;
+      sc[2] = N > 2 ? S->omega : 0.0;
+      asm volatile("" : "+v"(lost), "+v"(done), "+v"(sc[0]), "+v"(sc[1]), "+v"(sc[2]));
     }
-    return true;
+    if (!lost) return true;
+    if (t == 0) st_relaxed(a.err, 1u);
+    return false;
+  }
+  template <int K, int N = 0, class T, class Epi>
+  __device__ __forceinline__ bool exchange(const double *v, T *hdst, Epi &&epi) {
+    return exchange<K, N>(v, hdst, epi, [] {});
   }
 
   // Block 0 writes the state, all of it but `next`, which is a solve's err
@@ -547,7 +616,7 @@ struct Resident : ResNet {
     }
     double none[1] = {0.0};
     // the halo's x must be here before the product: an exchange of its own
-    if (!exchange<1>(none, win + RB, [](const double *) {})) return;
+    if (!exchange<1>(none, win + RB, [] { return [](const double *) {}; })) return;
     double v[2] = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
@@ -559,9 +628,11 @@ struct Resident : ResNet {
       v[1] += ri * ri;
     }
     KState *s = S;
-    if (!exchange<2, double>(v, nullptr, [s](const double *tot) {
-          s->energy = tot[0];
-          s->res2 = tot[1];
+    if (!exchange<2, 0, double>(v, nullptr, [s] {
+          return [s](const double *tot) {
+            s->energy = tot[0];
+            s->res2 = tot[1];
+          };
         }))
       return;
 #pragma unroll
@@ -604,22 +675,23 @@ __device__ __forceinline__ void Resident<F, RPT>::pcg() {
     v[1] += w[k] * w[k];
     v[2] += r[k] * r[k];
   }
-  if (!exchange<4>(v, hr, [&](const double *tot) {
-        cg1_epi(e, CG1_SETUP, s_, tot);
-        if (tot[3] != 0.0) s_->pend = 1;
+  if (!exchange<4, 1>(v, hr, [&] {
+        return [&](const double *tot) {
+          cg1_epi(e, CG1_SETUP, s_, tot);
+          if (tot[3] != 0.0) s_->pend = 1;
+        };
       }))
     return;
   if (S->pend) return outcome(kResDeclined);   // a block's columns do not fit its window
   // round 0 is W0 (w = A u), the following ones CG1_ITER
-  for (int it = 0; !S->done; ++it) {
+  for (int it = 0; !done; ++it) {
+    const double al = sc[0], be = sc[1];
     if (it > 0) {
-      const double al = S->alpha, be = S->beta;
 #pragma unroll
       for (int k = 0; k < RPT; ++k) {
         const double u = win[t + k * NT];   // r / m, of the previous iteration
         p[k] = it == 1 ? u : u + be * p[k];
         s[k] = it == 1 ? w[k] : w[k] + be * s[k];
-        x[k * NT] = x[k * NT] + al * p[k];
         r[k] = r[k] - al * s[k];
       }
       for (int h = t; h < nh; h += NT) {
@@ -628,28 +700,38 @@ __device__ __forceinline__ void Resident<F, RPT>::pcg() {
         hr[h] = hr[h] - al * sj;
       }
     }
-    double u[RPT];
+    double u[RPT], v3[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
       u[k] = r[k] / dm[k];
       win[t + k * NT] = u[k];
+      v3[0] += r[k] * u[k];
+      v3[2] += r[k] * r[k];
     }
     for (int h = t; h < nh; h += NT) win[RB + h] = hr[h] / hm[h];
     lds_barrier();
-    double v3[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
       w[k] = apply(k, u[k]);
       publish(k, w[k]);
-      v3[0] += r[k] * u[k];
       v3[1] += w[k] * u[k];
-      v3[2] += r[k] * r[k];
     }
-    if (!exchange<3>(v3, hw, [&](const double *tot) {
-          if (it == 0) cg1_epi(e, CG1_W0, s_, tot + 1);
-          else cg1_epi(e, CG1_ITER, s_, tot);
-        }))
-      return;
+    const bool go = exchange<3, 2>(
+        v3, hw,
+        [&] {
+          const Cg1Scalars c = cg1_scalars(s_);
+          return [&, c](const double *tot) {
+            if (it == 0) cg1_epi(e, CG1_W0, s_, tot + 1);
+            else cg1_iter_epi(e, c, s_, tot);
+          };
+        },
+        [&] {
+          if (it > 0) {
+#pragma unroll
+            for (int k = 0; k < RPT; ++k) x[k * NT] = x[k * NT] + al * p[k];
+          }
+        });
+    if (!go) return;
   }
   finish();
 }
@@ -686,23 +768,25 @@ __device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
     v0[2] += q_[k] * q_[k];
     q_[k] = 0.0;
   }
-  if (!exchange<4>(v0, hp, [&](const double *tot) {
-        bicg2_epi(e, B2_SETUP, s_, tot);
-        if (tot[3] != 0.0) s_->pend = 1;
+  if (!exchange<4, 1>(v0, hp, [&] {
+        return [&](const double *tot) {
+          bicg2_epi(e, B2_SETUP, s_, tot);
+          if (tot[3] != 0.0) s_->pend = 1;
+        };
       }))
     return;
   if (S->pend) return outcome(kResDeclined);
   for (int h = t; h < nh; h += NT) hsb[h] = hp[h];
-  for (int it = 1; !S->done; ++it) {
+  for (int it = 1; !done; ++it) {
     // P: completes iteration it - 1, p, v = A (p/m)
     double v3[3] = {0.0, 0.0, 0.0};
     if (it > 1) {
-      const double al = S->alpha, be = S->beta, om = S->omega;
+      const double be = sc[1], om = sc[2];
 #pragma unroll
       for (int k = 0; k < RPT; ++k) {
-        const double z2 = s[k] / dm[k];
+        const double z2 = win[t + k * NT];   // s / m, of Q
         const double bi = s[k] - om * q_[k];
-        x[k * NT] = (x[k * NT] + al * (p[k] / dm[k])) + om * z2;
+        x[k * NT] = x[k * NT] + om * z2;
         s[k] = bi;
         p[k] = bi + be * (p[k] - om * v[k]);
         v3[1] += bi * z2;
@@ -724,31 +808,41 @@ __device__ __forceinline__ void Resident<F, RPT>::bicgstab() {
       publish(k, v[k]);
       v3[0] += v[k] * rh[k * NT];
     }
-    if (!exchange<3>(v3, hv, [&](const double *tot) { bicg2_epi(e, B2_P, s_, tot); })) return;
-    if (S->done) break;
+    if (!exchange<3, 1>(v3, hv, [&] {
+          const Bicg2Scalars c = bicg2_scalars(s_);
+          return [&, c](const double *tot) { bicg2_p_epi(e, c, s_, tot); };
+        }))
+      return;
+    if (done) break;
     // Q: s = b - alpha v, t = A (s/m)
-    const double al = S->alpha;
+    const double al = sc[0];
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
       s[k] = s[k] - al * v[k];
+      x[k * NT] = x[k * NT] + al * win[t + k * NT];   // p / m, of P
       win[t + k * NT] = s[k] / dm[k];
     }
     for (int h = t; h < nh; h += NT) {
       hsb[h] = hsb[h] - al * hv[h];
       win[RB + h] = hsb[h] / hm[h];
     }
-    lds_barrier();
     double v4[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) v4[2] += rh[k * NT] * s[k];
+    lds_barrier();
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
       q_[k] = apply(k, win[t + k * NT]);
       publish(k, q_[k]);
       v4[0] += q_[k] * s[k];
       v4[1] += q_[k] * q_[k];
-      v4[2] += rh[k * NT] * s[k];
       v4[3] += rh[k * NT] * q_[k];
     }
-    if (!exchange<4>(v4, ht, [&](const double *tot) { bicg2_epi(e, B2_Q, s_, tot); })) return;
+    if (!exchange<4, 3>(v4, ht, [&] {
+          const Bicg2Scalars c = bicg2_scalars(s_);
+          return [&, c](const double *tot) { bicg2_q_epi(c, s_, tot); };
+        }))
+      return;
   }
   finish();
 }
@@ -799,7 +893,7 @@ __device__ __forceinline__ void Resident<F, RPT>::gmres() {
         win[t + k * NT] = x[k * NT];
         publish(k, x[k * NT]);
       }
-      if (!exchange<1>(none, win + RB, [](const double *) {})) return;
+      if (!exchange<1>(none, win + RB, [] { return [](const double *) {}; })) return;
     }
     double v[4] = {0.0, 0.0, 0.0, ok ? 0.0 : 1.0};
 #pragma unroll
@@ -813,9 +907,11 @@ __device__ __forceinline__ void Resident<F, RPT>::gmres() {
       v[2] += ri * ri;
       publish(k, w[k]);
     }
-    if (!exchange<4>(v, win + RB, [&](const double *tot) {
-          gmres_start_epi(e, st, first, tot);
-          if (tot[3] != 0.0) st->pend = 1;
+    if (!exchange<4>(v, win + RB, [&] {
+          return [&](const double *tot) {
+            gmres_start_epi(e, st, first, tot);
+            if (tot[3] != 0.0) st->pend = 1;
+          };
         }))
       return;
     if (st->pend) return outcome(kResDeclined);
@@ -841,9 +937,15 @@ __device__ __forceinline__ void Resident<F, RPT>::gmres() {
         d[0] += w[k] * gj[k];
       }
       if (i > 2) load_column(2, gn);
-      if (!exchange<1, double>(d, nullptr, [&](const double *tot) { e.h[(size_t)(i - 1) * (a.k + 1)] = tot[0]; })) return;
+      if (!exchange<1, 1, double>(d, nullptr, [&] {
+            return [&](const double *tot) {
+              e.h[(size_t)(i - 1) * (a.k + 1)] = tot[0];
+              st->alpha = tot[0];
+            };
+          }))
+        return;
       for (int j = 1; j <= i; ++j) {
-        const double hj = e.h[(size_t)(i - 1) * (a.k + 1) + (j - 1)];
+        const double hj = sc[0];
         d[0] = 0.0;
 #pragma unroll
         for (int k = 0; k < RPT; ++k) {
@@ -857,16 +959,19 @@ __device__ __forceinline__ void Resident<F, RPT>::gmres() {
           }
         }
         if (j + 2 < i) load_column(j + 2, gn);
-        if (!exchange<1>(d, j == i ? win + RB : nullptr, [&](const double *tot) {
-              double *hi = e.h + (size_t)(i - 1) * (a.k + 1);
-              if (j < i) {
-                hi[j] = tot[0];
-                return;
-              }
-              const double norm = sqrt(tot[0]);
-              hi[i] = norm;
-              e.nrm[i + 1] = norm;
-              gmres_close_step(e, st, i);
+        if (!exchange<1, 1>(d, j == i ? win + RB : nullptr, [&] {
+              return [&](const double *tot) {
+                double *hi = e.h + (size_t)(i - 1) * (a.k + 1);
+                if (j < i) {
+                  hi[j] = tot[0];
+                  st->alpha = tot[0];
+                  return;
+                }
+                const double norm = sqrt(tot[0]);
+                hi[i] = norm;
+                e.nrm[i + 1] = norm;
+                gmres_close_step(e, st, i);
+              };
             }))
           return;
       }
@@ -965,7 +1070,7 @@ struct ResidentMixed : ResNet {
       publish(k, xi);
     }
     const double none[1] = {0.0};
-    return exchange<1>(none, win + RB, [](const double *) {});
+    return exchange<1>(none, win + RB, [] { return [](const double *) {}; });
   }
 
   __device__ __forceinline__ void pcg() {
@@ -1003,9 +1108,11 @@ struct ResidentMixed : ResNet {
       v[1] += ri * ri;
       v[2] += bi * bi;
     }
-    if (!exchange<4>(v, hr, [&](const double *tot) {
-          mixed_epi(e, MX_SETUP, st, tot);
-          if (tot[3] != 0.0) st->pend = 1;
+    if (!exchange<4>(v, hr, [&] {
+          return [&](const double *tot) {
+            mixed_epi(e, MX_SETUP, st, tot);
+            if (tot[3] != 0.0) st->pend = 1;
+          };
         }))
       return;
     if (S->pend) return outcome(kResDeclined);
@@ -1039,7 +1146,11 @@ struct ResidentMixed : ResNet {
           const double ru = rd * (double)dsq[k];
           v5[4] += ru * ru;
         }
-        if (!exchange<5>(v5, hq, [&](const double *tot) { mixed_epi(e, MX_A, st, tot); })) return;
+        if (!exchange<5>(v5, hq, [&] {
+              const MixedScalars c = mixed_scalars(e, st);
+              return [&, c](const double *tot) { mixed_a_epi(e, c, st, tot); };
+            }))
+          return;
         continue;
       }
       // a reliable update: x += S (y + alpha p), r~ = S (b - A x) in FP64
@@ -1065,7 +1176,7 @@ struct ResidentMixed : ResNet {
         publish(k, r[k]);
         v3[0] += (double)r[k] * (double)r[k];
         }
-      if (!exchange<3>(v3, hr, [&](const double *tot) { mixed_epi(e, MX_R, st, tot); })) return;
+      if (!exchange<3>(v3, hr, [&] { return [&](const double *tot) { mixed_epi(e, MX_R, st, tot); }; })) return;
     }
     if (S->status == S_NONFINITE) return outcome(kResDeclined);
     if (!window_x()) return;
@@ -1079,9 +1190,11 @@ struct ResidentMixed : ResNet {
         v2[1] += ri * ri;
       }
     }
-    if (!exchange<2, double>(v2, nullptr, [st](const double *tot) {
-          st->energy = tot[0];
-          st->res2 = tot[1];
+    if (!exchange<2, 0, double>(v2, nullptr, [st] {
+          return [st](const double *tot) {
+            st->energy = tot[0];
+            st->res2 = tot[1];
+          };
         }))
       return;
     if (t == 0) S->mgs_j = map.p.H;   // whether every column is an int16 offset away
