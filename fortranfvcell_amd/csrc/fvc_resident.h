@@ -133,19 +133,19 @@ __device__ __forceinline__ void resident_prep(const ResPrepArgs &a) {
     if (worst[s] > 0) atomicMax(&s_hx[s], worst[s]);
   __syncthreads();
   // thread t tries t / 2 + 1 columns of tiles over the row lengths H and
-  // H + 1 in turn; the fewest halo entries win
+  // H + 1 in turn; the least cost wins
   auto tiles = [&](int q, ResPlan &p) {
     return res_tiles(n, H + (q & 1), max(s_hx[q & 1], 1), (q >> 1) + 1, a.rmax, a.bmax, a.hmax, p);
   };
   for (int q = threadIdx.x; q < 2 * min(a.bmax, kResMaxBlocks); q += blockDim.x) {
     ResPlan p{};
-    if (tiles(q, p)) atomicMin(&s_best, (p.nh << 10) | q);
+    if (tiles(q, p)) atomicMin(&s_best, (res_cost(p) << 10) | q);
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
   ResPlan p{};
   const bool strips = res_strips(n, H, a.rmax, a.bmax, a.hmax, p);
-  if (s_best < INT_MAX && !(strips && 2 * H <= (s_best >> 10))) tiles(s_best & 1023, p);
+  if (s_best < INT_MAX && !(strips && res_cost(p) <= (s_best >> 10))) tiles(s_best & 1023, p);
   p.H = H;
   p.ticket = (int)gridDim.x;
   *a.plan = p;

@@ -143,6 +143,12 @@ FVC_HD bool res_tiles(int n, int S, int hx, int ntx, int rmax, int bmax, int hma
   return p.nh <= hmax;
 }
 
+// Which of two plans is taken: the one of at most kResOneStep blocks, then the
+// one of fewer halo entries (253 x 257 rows: 2.6 us per PCG iteration in 64
+// strips of 514 halo entries, 3.1 in 72 tiles of 134).
+constexpr int kResOneStep = 64;   // blocks up to which the sums are added in one step
+FVC_HD int res_cost(const ResPlan &p) { return (p.nb > kResOneStep ? 2 * kResMaxHalo : 0) + p.nh; }
+
 // Strips of rmax rows for columns up to H rows away.
 FVC_HD bool res_strips(int n, int H, int rmax, int bmax, int hmax, ResPlan &p) {
   const int nb = (int)(((long)n + rmax - 1) / rmax);
@@ -190,20 +196,29 @@ constexpr int res_max_halo(int code, int rpt) {
 // Rows per thread and blocks at most for neq rows on `cus` compute units;
 // rpt 0: the system does not fit the chip.  Measured on MI355X (us per
 // iteration, PCG / BiCGSTAB):
-//   * one block needs no exchange: 2,025 rows 1.9 / 4.0 against 2.6 / 5.1 on
-//     8 blocks; 4,095 rows 2.8 / 5.9 against 2.6 / 5.2, so one block up to
+//   * one block needs no exchange: 2,025 rows 1.7 / 3.1 against 2.2 / 4.2 on
+//     8 blocks; 4,096 rows 2.5 / 5.4 against 2.1 / 4.2, so one block up to
 //     2,048 rows;
-//   * up to 64 blocks the sums need one step instead of two: 32,300 rows 3.2
-//     on 40 blocks of 1,024 against 3.7 on 80 of 512, but 65,536 rows 3.6
-//     either on 80 of 1,024 or 40 of 2,048, so two rows a thread at most for
-//     that;
-//   * beyond, the fewest rows per thread: 262,144 rows 4.6 at 2, 4.8 at 4,
-//     5.5 at 8 -- as long as a twentieth of the rows stays free for tiles that
-//     the mesh's edge cuts (524,176 rows 8.1 in strips at 4, 5.6 in tiles at 8).
+//   * then one row a thread while 52 blocks hold them (64 with the sixth more
+//     that tiles need): 12,707 rows 2.1 / 4.2 against 2.3 / 4.7 at two, but
+//     32,300 rows 2.4 / 5.0 either way, and GMRES on 26,895 rows 2.59 ms a solve
+//     on 64 blocks against 2.50 on 32;
+//   * up to 64 blocks the sums need one step instead of two: 59,713 rows 2.5 /
+//     5.2 on 64 blocks of 1,024 against 3.1 / 6.1 on 72, 65,160 rows 2.6 / 5.4
+//     against 3.1 / 6.1 on 80 (GMRES 3.73 -> 2.83 ms a solve, mixed PCG 8.4 ->
+//     7.5), so two rows a thread as long as 64 blocks hold them.  Four rows a
+//     thread on 64 blocks still serve PCG, but not BiCGSTAB, whose arithmetic
+//     for them outweighs the step: 81,200 rows 2.8 / 6.1 against 3.1 / 6.0 at
+//     two, 127,800 rows 2.9 / 6.5 against 3.1 / 6.1.  More blocks than 64 are
+//     launched for plans that need them; res_cost prefers the others;
+//   * beyond, the fewest rows per thread: 160,860 rows 3.1 / 6.1 at 2, 3.5 / 7.0
+//     at 4, 3.9 / 8.5 at 8 -- as long as a twentieth of the rows stays free for
+//     tiles that the mesh's edge cuts (524,176 rows in strips at 4 took half as
+//     long again as in tiles at 8).
 struct ResShape {
   int rpt, blocks;
 };
-inline ResShape resident_shape(int neq, int cus) {
+inline ResShape resident_shape(int neq, int cus, int kind = kResPcg) {
   const long n = neq, most = (cus < kResMaxBlocks ? cus : kResMaxBlocks) & ~7;
   for (int rpt = 1; rpt <= 4; rpt *= 2)
     if (n <= (long)kResThreads * rpt) return {rpt, 1};
@@ -213,8 +228,10 @@ inline ResShape resident_shape(int neq, int cus) {
     const long want = (nb + nb / 6 + 8) & ~7L;
     return (int)(want < most ? want : most);
   };
-  for (int rpt = 1; rpt <= 2; rpt *= 2)
-    if (n <= (long)kResThreads * rpt * (most < 52 ? most : 52) && blocks(rpt) <= 64) return {rpt, blocks(rpt)};
+  for (int rpt = 1; rpt <= (kind == kResPcg ? 4 : 2); rpt *= 2) {
+    const long few = rpt == 1 ? 52 : kResOneStep;
+    if (n <= (long)kResThreads * rpt * (most < few ? most : few)) return {rpt, blocks(rpt)};
+  }
   for (int rpt = 2; rpt <= 8; rpt *= 2) {
     const long room = (long)kResThreads * rpt * most;
     if (n <= (rpt < 8 ? room - room / 20 : room)) return {rpt, blocks(rpt)};
@@ -234,9 +251,9 @@ struct ResBatchPlan {
   double load = 0.0;                   // the most loaded block, us per unit of iterations
 };
 
-// us per PCG iteration at 1, 2, 4, 8 rows a thread, one block and a team
-// (MI355X, resident_shape's measurements)
-constexpr double kResIterAlone[4] = {1.3, 1.5, 1.9, 2.75}, kResIterTeam[4] = {2.8, 2.95, 3.4, 4.4};
+// us per PCG iteration at 1, 2, 4, 8 rows a thread, one full block and a team
+// (MI355X)
+constexpr double kResIterAlone[4] = {1.3, 1.3, 1.7, 2.5}, kResIterTeam[4] = {2.1, 2.3, 2.7, 3.8};
 
 // blocks: co-resident ones.  A system's iterations are taken as
 // neq^(expo - 1) (PCG on these meshes: expo 1.5), its time as iterations

@@ -413,7 +413,7 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
     return FVC_OK;
   } else {
     const int neq = in.A.neq;
-    const ResShape sh = resident_shape(neq, d.cus);
+    const ResShape sh = resident_shape(neq, d.cus, kind);
     if (sh.rpt == 0) return FVC_OK;
     ResArgs a{};
     a.A = in.A; a.st = st; a.m = in.m; a.x = in.x; a.b = in.b;

@@ -250,3 +250,23 @@ def test_resident_gmres_exact_start(fvc):
         x, st = fvc.solve(f, fvc.GMRES, b=np.zeros(n * n), tol=1e-10, gmres_k=10)
         xk, sk = fvc.solve(f, fvc.GMRES, b=np.zeros(n * n), tol=1e-10, gmres_k=10, engine=fvc.ENGINE_KERNELS)
         assert (st["status"], st["iterations"]) == (sk["status"], sk["iterations"]) and not x.any() and not xk.any()
+
+
+@pytest.mark.parametrize("kind,nx,ny", [("quad", 208, 128), ("quad", 213, 125), ("quad", 253, 257), ("quad", 256, 256),
+                                        ("quad", 64, 1024), ("quad", 6001, 10), ("quad", 257, 256), ("tri", 181, 0),
+                                        ("quad", 512, 256), ("quad", 361, 363), ("quad", 171, 767)])
+def test_resident_at_the_edges_of_64_blocks(fvc, kind, nx, ny):
+    """Plans of at most 64 blocks are preferred: one, two and (PCG) four rows
+    a thread at the last rows that 52 and 64 blocks hold and just beyond, in
+    tiles and in strips.  After two iterations only the order of the sums differs (1e-12, as above)."""
+    m = _mesh(kind, nx, ny)
+    sp = P.pressure_system(m, k=P.lognormal_k(3, m.neq), pin="penalty")
+    sm = P.advdiff_system(m, dt=0.005, under_relax=0.8)
+    for code, s in ((fvc.PCG, sp), (fvc.BICGSTAB, sm)):
+        f = P.to_ell(s)
+        print(f"64 blocks {kind} {nx}x{ny} neq={m.neq} code={code}", flush=True)
+        kw = dict(tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_ZERO, maxit=2)
+        xa, sa = fvc.solve(f, code, **kw)
+        xk, sk = fvc.solve(f, code, engine=fvc.ENGINE_KERNELS, **kw)
+        assert sa["engine"] == fvc.ENGINE_PERSISTENT and sa["iterations"] == sk["iterations"] == 2
+        assert _rel(xa, xk) <= 1e-12
