@@ -42,6 +42,14 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
+ON_CHIP_THREADS = 512   # threads per block on chip (GMRES with modified Gram-Schmidt streams with 1,024)
+
+
+def rates(nbytes: float, seconds: float, streamed: bool) -> dict:
+    """Rate of the bytes that a schedule streams from memory.  A solve held on
+    chip does not move them (its matrix is read once): it has no such rate."""
+    gbs = nbytes / seconds / 1e9 if streamed else None
+    return {"GBs_algorithmic": gbs, "frac": gbs / HBM_PEAK_GBS if streamed else None, "on_chip": not streamed}
 
 
 def log(*a):
@@ -372,17 +380,18 @@ def gmres_only(n: int, steps: int) -> None:
         out[name] = {"cycles": st["iterations"], "arnoldi_steps": st["inner_iterations"],
                      "ms_per_solve": float(np.mean(ts)) * 1e3, "true_relres": st["true_relres"],
                      "status": st["status"],
-                     "GBs_algorithmic": (gb / float(np.mean(ts)) / 1e9) if "precision" not in kw else None}
+                     "GBs_algorithmic": None if "precision" in kw or (name == "mgs" and st["block_size"] == ON_CHIP_THREADS)
+                     else gb / float(np.mean(ts)) / 1e9}
     print(json.dumps({"workload": f"GMRES(30), {n}x{n} momentum system, true relative residual 1e-10",
                       "neq": s.neq, "steps": steps, **out}), flush=True)
 
 
 def batch_only(steps: int) -> None:
     """Only the 256-system batch (pressure systems, sides log-uniform in
-    [32, 512], each to true relative residual 1e-10), FP64 and mixed, at the
-    options the autotuner picks on MI355X (1,024 threads, work exponent 1.5;
-    FP64 64 systems per launch, mixed 86), `steps` batched solves each: the
-    batch kernels, for a profile."""
+    [32, 512], each to true relative residual 1e-10), FP64 and mixed, on chip
+    (the library's own choice) and streamed at the fastest launches (1,024
+    threads, work exponent 1.5; FP64 64 systems per launch, mixed 86), `steps`
+    batched solves each: the batch kernels, for a profile."""
     import fortranfvcell_amd as F
     from fortranfvcell_amd import problems as P
     F.init(0)
@@ -390,9 +399,11 @@ def batch_only(steps: int) -> None:
     sizes = [(int(f["neq"]), int(f["nad"])) for f in fmts]
     db = F.DeviceBatch(F.concat_ell(fmts))
     out = {}
-    for name, prec, per in (("fp64", F.PREC_FP64, 64), ("mixed", F.PREC_MIXED, 86)):
-        kw = dict(tol=1e-10, precision=prec, stop_rule=F.STOP_RELRES, block_size=1024, batch_work_exp10=15,
-                  batch_launch_systems=per)
+    for name, prec, per in (("fp64", F.PREC_FP64, 0), ("mixed", F.PREC_MIXED, 0),
+                            ("fp64_streamed", F.PREC_FP64, 64), ("mixed_streamed", F.PREC_MIXED, 86)):
+        kw = dict(tol=1e-10, precision=prec, stop_rule=F.STOP_RELRES)
+        if per:
+            kw.update(block_size=1024, batch_work_exp10=15, batch_launch_systems=per)
         ts = []
         for _ in range(steps):
             sts = db.solve(**kw)
@@ -404,8 +415,7 @@ def batch_only(steps: int) -> None:
                      + q["inner_iterations"] * (spmv_bytes(ne, nz) + 40 * ne) for q, (ne, nz) in zip(sts, sizes))
         t = float(np.mean(ts))
         out[name] = {"ms": t * 1e3, "solves_per_s": len(sts) / t, "algorithmic_bytes": nb,
-                     "GBs_algorithmic": nb / t / 1e9, "frac": nb / t / 1e9 / HBM_PEAK_GBS,
-                     "max_iterations": max(q["iterations"] for q in sts),
+                     **rates(nb, t, per > 0), "max_iterations": max(q["iterations"] for q in sts),
                      "all_converged": all(q["status"] == 0 for q in sts)}
     print(json.dumps({"workload": "256 pressure systems, sides log-uniform in [32, 512], true relative residual 1e-10",
                       "rows": int(sum(ne for ne, _ in sizes)), "steps": steps, **out}), flush=True)
@@ -516,10 +526,16 @@ def main():
     x = ds.x.get()
     relres = float(np.linalg.norm(s.b - P.scipy_csr(s) @ x) / np.linalg.norm(s.b))
     its = st["iterations"]
-    solve_bytes = bicgstab_solve_bytes(neq, nnz, its)
-    launches = 2 * its + 4   # SETUP, P/Q per iteration, the closing P and Q, FINAL (+ a no-row flush)
     kt = float(np.mean(kern))
-    achieved = solve_bytes / kt / 1e9
+    # the same solve by the engine that streams the system from memory (what
+    # systems beyond the chip take), for the roofline
+    skw = dict(opts, engine=F.ENGINE_KERNELS)
+    ds.solve(F.BICGSTAB, tol=tol, **skw)
+    sts = [ds.solve(F.BICGSTAB, tol=tol, **skw) for _ in range(args.steps)]
+    kst = float(np.mean([q["seconds"] for q in sts]))
+    solve_bytes = bicgstab_solve_bytes(neq, nnz, sts[0]["iterations"])
+    launches = 2 * sts[0]["iterations"] + 4   # SETUP, P/Q per iteration, the closing P and Q, FINAL (+ a no-row flush)
+    achieved = solve_bytes / kst / 1e9
     log(f"BiCGSTAB: {its} it, {kt * 1e3:.3f} ms/solve kernel, wall {wall / args.steps * 1e3:.3f} ms, relres {relres:.2e}")
 
     result = {
@@ -545,8 +561,12 @@ def main():
                    "iterations": its, "true_relres": relres, "engine": st["engine"],
                    "grid_blocks": st["grid_blocks"], "block_size": st["block_size"],
                    "device": info["name"]},
-        # the dominant kernel is bicg2_kernel<0> (ELLPACK width 4): one launch
-        # per phase.  achieved = algorithmic bytes per launch / event time per
+        # the steps above hold the system on chip where it fits: one launch a
+        # solve, the matrix read once
+        "on_chip": st["engine"] == F.ENGINE_PERSISTENT,
+        "us_per_iteration": kt / its * 1e6,
+        # the streaming engine's dominant kernel is bicg2_kernel<0> (ELLPACK
+        # width 4): one launch per phase, timed apart from the steps.  achieved = algorithmic bytes per launch / event time per
         # launch on the solve's stream, i.e. bytes per solve / time per solve
         # (launch gaps and the host's done-checks included, so a lower bound
         # of the kernel-only rate rocprofv3 reports)
@@ -556,8 +576,8 @@ def main():
                      "kernel": "fvc::bicg2_kernel<0> (two-phase BiCGSTAB, one launch per phase)",
                      "launches_per_solve": launches,
                      "algorithmic_bytes_per_launch": solve_bytes / launches,
-                     "us_per_launch": kt / launches * 1e6,
-                     "solve_ms": kt * 1e3},
+                     "us_per_launch": kst / launches * 1e6,
+                     "solve_ms": kst * 1e3},
     }
 
     if not args.no_extra:
@@ -592,9 +612,8 @@ def main():
             gm[oname] = {"cycles": st_g["iterations"], "arnoldi_steps": st_g["inner_iterations"],
                          "ms_per_solve": st_g["seconds"] * 1e3, "solves_per_s": 1.0 / st_g["seconds"],
                          "true_relres": st_g["true_relres"], "status": st_g["status"],
-                         "GBs_algorithmic": gb / st_g["seconds"] / 1e9,
-                         "frac": gb / st_g["seconds"] / 1e9 / HBM_PEAK_GBS, "block_size": st_g["block_size"],
-                         "grid_blocks": st_g["grid_blocks"]}
+                         "block_size": st_g["block_size"], "grid_blocks": st_g["grid_blocks"],
+                         **rates(gb, st_g["seconds"], oname != "mgs" or st_g["block_size"] != ON_CHIP_THREADS)}
         extra["gmres30"] = gm
         log("gmres30", gm)
         # the reference's defaults: underU = 1 (src/Main.f:219), no transient
@@ -614,7 +633,7 @@ def main():
                         f"{ns}x{ns} cells",
             "bicgstab": {"iterations": st_sb["iterations"], "ms_per_solve": st_sb["seconds"] * 1e3,
                          "true_relres": st_sb["true_relres"], "status": st_sb["status"],
-                         "GBs_algorithmic": sbb / st_sb["seconds"] / 1e9},
+                         **rates(sbb, st_sb["seconds"], st_sb["engine"] == F.ENGINE_KERNELS)},
             "gmres30_cgs2_lag": {"cycles": st_sg["iterations"], "arnoldi_steps": st_sg["inner_iterations"],
                              "ms_per_solve": st_sg["seconds"] * 1e3, "true_relres": st_sg["true_relres"],
                              "status": st_sg["status"]},
@@ -630,7 +649,7 @@ def main():
         pb = st_p["iterations"] * pcg_iter_bytes(sp.neq, ellp["nad"]) + 2 * spmv_bytes(sp.neq, ellp["nad"])
         extra["pcg_pressure"] = {"iterations": st_p["iterations"], "ms_per_solve": st_p["seconds"] * 1e3,
                                  "solves_per_s": 1.0 / st_p["seconds"], "true_relres": st_p["true_relres"],
-                                 "GBs_algorithmic": pb / st_p["seconds"] / 1e9,
+                                 **rates(pb, st_p["seconds"], st_p["engine"] == F.ENGINE_KERNELS),
                                  "us_per_iteration": st_p["seconds"] / st_p["iterations"] * 1e6}
         log("pcg", extra["pcg_pressure"])
         # mixed precision (FP32 inner PCG, FP64 residuals and refinement) against
@@ -731,8 +750,8 @@ def main():
                           "layout": tb["layout"],
                           "trials_ms": {f"{q['layout']} {q['options']}": round(q["seconds"] * 1e3, 2)
                                         for q in tb["trials"]},
-                          "algorithmic_bytes": nb, "GBs_algorithmic": nb / t / 1e9,
-                          "frac": nb / t / 1e9 / HBM_PEAK_GBS}
+                          "algorithmic_bytes": nb, **rates(nb, t, tuned.get("block_size", 0) != 0 or
+                                                               tuned.get("batch_rows_per_wave", 0) != 0)}
         single = 0.0
         for f in fmts:
             d1 = F.DeviceSystem(f)
