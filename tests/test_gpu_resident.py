@@ -270,3 +270,21 @@ def test_resident_at_the_edges_of_64_blocks(fvc, kind, nx, ny):
         xk, sk = fvc.solve(f, code, engine=fvc.ENGINE_KERNELS, **kw)
         assert sa["engine"] == fvc.ENGINE_PERSISTENT and sa["iterations"] == sk["iterations"] == 2
         assert _rel(xa, xk) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [108, 301, 392])
+def test_resident_finds_the_row_length(fvc, n):
+    """Triangles split from quads, 2 n cells to a row, at sizes where rows
+    spread evenly over the system miss every place where 2 n - 1 wraps: tiles
+    of that length would hold columns outside their window."""
+    m = _mesh("tri", n, 0)
+    s = P.advdiff_system(m, dt=0.005, under_relax=0.8)
+    kw = dict(tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_ZERO, maxit=2)
+    for lay in (P.to_ell, P.to_csrd):
+        f = lay(s)
+        for code in (fvc.PCG, fvc.BICGSTAB):
+            print(f"row length tri {n} {lay.__name__} code={code}", flush=True)
+            xa, sa = fvc.solve(f, code, **kw)
+            xk, sk = fvc.solve(f, code, engine=fvc.ENGINE_KERNELS, **kw)
+            assert sa["engine"] == fvc.ENGINE_PERSISTENT and sa["iterations"] == sk["iterations"] == 2
+            assert _rel(xa, xk) <= 1e-12
