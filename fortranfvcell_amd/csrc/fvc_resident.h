@@ -59,6 +59,7 @@ struct ResPrepArgs {
   res_word *part, *rows;   // cleared here: nparts and 4 neq words
   int nparts;
   int rmax, bmax, hmax;    // rows per block, blocks and halo entries at most
+  int one_step;            // prefer plans of at most kResOneStep blocks
 };
 
 // The columns of row i that count: off-diagonal entries other than
@@ -153,13 +154,13 @@ __device__ __forceinline__ void resident_prep(const ResPrepArgs &a) {
   };
   for (int q = threadIdx.x; q < 2 * min(a.bmax, kResMaxBlocks); q += blockDim.x) {
     ResPlan p{};
-    if (tiles(q, p)) atomicMin(&s_best, (res_cost(p) << 10) | q);
+    if (tiles(q, p)) atomicMin(&s_best, (res_cost(p, a.one_step) << 10) | q);
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
   ResPlan p{};
   const bool strips = res_strips(n, H, a.rmax, a.bmax, a.hmax, p);
-  if (s_best < INT_MAX && !(strips && res_cost(p) <= (s_best >> 10))) tiles(s_best & 1023, p);
+  if (s_best < INT_MAX && !(strips && res_cost(p, a.one_step) <= (s_best >> 10))) tiles(s_best & 1023, p);
   p.H = H;
   p.ticket = (int)gridDim.x;
   *a.plan = p;

@@ -143,11 +143,13 @@ FVC_HD bool res_tiles(int n, int S, int hx, int ntx, int rmax, int bmax, int hma
   return p.nh <= hmax;
 }
 
-// Which of two plans is taken: the one of at most kResOneStep blocks, then the
-// one of fewer halo entries (253 x 257 rows: 2.6 us per PCG iteration in 64
+// Which of two plans is taken: where one_step is asked for, the one of at most
+// kResOneStep blocks, then the one of fewer halo entries (253 x 257 rows: 2.6 us per PCG iteration in 64
 // strips of 514 halo entries, 3.1 in 72 tiles of 134).
 constexpr int kResOneStep = 64;   // blocks up to which the sums are added in one step
-FVC_HD int res_cost(const ResPlan &p) { return (p.nb > kResOneStep ? 2 * kResMaxHalo : 0) + p.nh; }
+FVC_HD int res_cost(const ResPlan &p, bool one_step) {
+  return (one_step && p.nb > kResOneStep ? 2 * kResMaxHalo : 0) + p.nh;
+}
 
 // Strips of rmax rows for columns up to H rows away.
 FVC_HD bool res_strips(int n, int H, int rmax, int bmax, int hmax, ResPlan &p) {
@@ -206,11 +208,14 @@ constexpr int res_max_halo(int code, int rpt) {
 //   * up to 64 blocks the sums need one step instead of two: 59,713 rows 2.5 /
 //     5.2 on 64 blocks of 1,024 against 3.1 / 6.1 on 72, 65,160 rows 2.6 / 5.4
 //     against 3.1 / 6.1 on 80 (GMRES 3.73 -> 2.83 ms a solve, mixed PCG 8.4 ->
-//     7.5), so two rows a thread as long as 64 blocks hold them.  Four rows a
-//     thread on 64 blocks still serve PCG, but not BiCGSTAB, whose arithmetic
-//     for them outweighs the step: 81,200 rows 2.8 / 6.1 against 3.1 / 6.0 at
-//     two, 127,800 rows 2.9 / 6.5 against 3.1 / 6.1.  More blocks than 64 are
-//     launched for plans that need them; res_cost prefers the others;
+//     7.5), so two rows a thread as long as 64 blocks hold them, and for PCG
+//     four: 81,200 rows 2.8 against 3.1 at two, 127,800 rows 2.9 against 3.1
+//     (BiCGSTAB 6.1 against 6.0, 6.5 against 6.1).  More blocks than 64 are
+//     launched for plans that need them; res_cost prefers the others.
+//     BiCGSTAB, which gains less, stays with the plan of least halo from 53,248
+//     rows on: its count of iterations follows the order of the sums (65,536
+//     rows of a steady transport system: 5,143 iterations with it, 5,445 on 64
+//     blocks, the reference's 5,096);
 //   * beyond, the fewest rows per thread: 160,860 rows 3.1 / 6.1 at 2, 3.5 / 7.0
 //     at 4, 3.9 / 8.5 at 8 -- as long as a twentieth of the rows stays free for
 //     tiles that the mesh's edge cuts (524,176 rows in strips at 4 took half as
@@ -229,7 +234,7 @@ inline ResShape resident_shape(int neq, int cus, int kind = kResPcg) {
     return (int)(want < most ? want : most);
   };
   for (int rpt = 1; rpt <= (kind == kResPcg ? 4 : 2); rpt *= 2) {
-    const long few = rpt == 1 ? 52 : kResOneStep;
+    const long few = rpt == 1 || kind == kResBicgstab ? 52 : kResOneStep;
     if (n <= (long)kResThreads * rpt * (most < few ? most : few)) return {rpt, blocks(rpt)};
   }
   for (int rpt = 2; rpt <= 8; rpt *= 2) {

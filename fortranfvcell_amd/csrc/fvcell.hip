@@ -442,7 +442,8 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
       a.err = reinterpret_cast<unsigned *>(&st->next);
       a.gang = 1;
       hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, (int)kCtrWords, st, 1);
-      ResPrepArgs pa{in.A, plan, part, rows, kResPartWords, kResThreads * sh.rpt, sh.blocks, hmax};
+      ResPrepArgs pa{in.A, plan, part, rows, kResPartWords, kResThreads * sh.rpt, sh.blocks, hmax,
+                     kind != kResBicgstab};
       hipLaunchKernelGGL(resident_prep_kernel<F>, dim3(std::min((neq + 255) / 256, 4 * d.cus)), dim3(256), 0, s, pa);
     }
     HIPCHK(hipGetLastError());
