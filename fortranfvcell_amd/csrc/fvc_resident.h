@@ -303,6 +303,7 @@ struct ResArgs {
   unsigned *err;           // set when a wait expired; the waits of others end too
   int part_half;
   int gang;                // how many times longer the first exchange may take
+  unsigned strict;         // from this exchange on a wait ends after one look (tests)
   double tol;
   double delta;            // mixed: residual drop that triggers an FP64 update
   int max_inner;           // mixed: FP32 iterations between updates, at most
@@ -389,7 +390,7 @@ struct ResNet {
     constexpr int E = K > 4 ? 2 : 1;   // the fifth value goes with the first 16 lanes
     res_word *part = a.part + (size_t)(ep & 1) * (size_t)a.part_half;
     // a block may come to its first exchange long before the others
-    const unsigned limit = ep == 1 ? kResSpin * (unsigned)a.gang : kResSpin;
+    const unsigned limit = ep >= a.strict ? 0u : ep == 1 ? kResSpin * (unsigned)a.gang : kResSpin;
     // Up to 64 blocks a lane per block adds all sums.  Beyond, so many
     // readers of so many words hold each other up (256 blocks: 7 us), and
     // the sums go in two steps: the first block of 16 adds its group's and
@@ -1297,6 +1298,7 @@ struct ResBatchArgs {
   ResPlan *plans;            // per system, cleared
   res_word *rows, *part;
   unsigned *err;
+  unsigned strict;           // as ResArgs'
   double tol, delta;
   int maxit, x0_zero, stop_rule, max_inner, rmax, hmax;
 };
@@ -1349,6 +1351,7 @@ __global__ __launch_bounds__(256) void resident_batch_prep_kernel(ResBatchArgs B
 template <int F, int RPT, int Code>
 __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArgs B) {
   extern __shared__ double dyn[];
+  __shared__ unsigned stop;
   const int g = (int)gridDim.x, b0 = (int)blockIdx.x;
   const int b = (g & 7) == 0 ? (b0 & 7) * (g >> 3) + (b0 >> 3) : b0;
   const int k1 = res_uniform(B.block_ptr + b + 1);
@@ -1376,6 +1379,7 @@ __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArg
     a.part_half = res_part_half(D.g_count);
     a.err = B.err;
     a.gang = kResGang;
+    a.strict = B.strict;
     a.tol = B.tol;
     a.maxit = B.maxit;
     a.x0_zero = B.x0_zero;
@@ -1383,8 +1387,13 @@ __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArg
     a.delta = B.delta;
     a.max_inner = B.max_inner;
     resident_solve<F, RPT, Code>(a, p, c, dyn);
-    if (ld_relaxed(B.err) != 0u) return;   // (uniform enough: a block that goes on only waits, bounded)
-    __syncthreads();                       // LDS is reused
+    // Once a wait expired, every block leaves, all of its waves or none: the
+    // word is set while others look at it, and a block whose wave 0 alone had
+    // left would go on to its next system with nobody to run the scalar part, a
+    // loop without an end where one block holds that system and waits for no one.
+    if (threadIdx.x == 0) stop = ld_relaxed(B.err);
+    __syncthreads();   // (also: LDS is reused)
+    if (stop != 0u) return;
   }
 }
 

@@ -119,6 +119,9 @@ struct DevState {
   const double *mat_m = nullptr;
   bool mat_valid = false;
   bool keep_next = false;
+  // the exchange from which the next call's waits on chip end after one look
+  // (fvc_test_expire; ~0u: none)
+  unsigned strict_next = ~0u;
   // fvc_solve_dev_noalloc: the device address of `scratch` on this device, and
   // whether the call in progress must take its workspace from there
   char *scratch_dev = nullptr;
@@ -283,6 +286,7 @@ struct SolveIn {
   int orth;               // GMRES: FVC_ORTH_*
   int refresh_every;      // mixed: FP32 iterations between FP64 residual recomputations, at most
   double refresh_drop;    // mixed: residual drop that triggers one
+  unsigned strict;        // on chip: ResArgs::strict
 };
 
 // Persistent launches are ordinary launches whose grid fits the device at
@@ -420,6 +424,7 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
     a.tol = in.tol; a.maxit = in.maxit; a.x0_zero = in.x0_zero; a.stop_rule = in.stop_rule;
     a.delta = in.refresh_drop; a.max_inner = in.refresh_every;
     a.gv = gv; a.ld = ld; a.k = in.gmres_k;
+    a.strict = in.strict;
     const void *fn = kind == kResPcg        ? resident_fn<F, kResPcg>(sh.rpt)
                      : kind == kResBicgstab ? resident_fn<F, kResBicgstab>(sh.rpt)
                      : kind == kResGmres    ? resident_fn<F, kResGmres>(sh.rpt)
@@ -1542,6 +1547,8 @@ int solve_impl(int code, int matriz, int unsym, int neq, int nad, const double *
     db = tb;
   }
   SolveIn in{};
+  in.strict = d->strict_next;
+  d->strict_next = ~0u;
   in.code = code;
   in.F = md.F;
   in.A = md.m;
@@ -1676,7 +1683,7 @@ int dot_impl(const double *a, const double *b, int n, double *result, bool on_de
 template <int F>
 int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_off, const std::vector<int> &val_off, int w,
                        const double *ad, const double *av, const int *ia, const int *ja, double *x, const double *b,
-                       double tol, int maxit, const fvc_options &o, std::vector<KState> &host_st,
+                       double tol, int maxit, const fvc_options &o, unsigned strict, std::vector<KState> &host_st,
                        std::vector<int> &todo, hipStream_t s) {
   const int nsys = hi - lo;
   const auto leave = [&] {
@@ -1761,6 +1768,7 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     B.plans = reinterpret_cast<ResPlan *>(clear + 1);
     B.rows = rows;
     B.part = part;
+    B.strict = strict;
     B.tol = tol;
     B.maxit = maxit;
     B.x0_zero = o.x0_rule == FVC_X0_GIVEN ? 0 : 1;
@@ -1821,6 +1829,8 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
   const int min_rows = o.batch_rows_per_wave > 0 ? o.batch_rows_per_wave * (bs / 64) : 64;
   std::vector<KState> host_st(nsys);
   std::vector<int> todo;   // the systems the launches below solve
+  const unsigned strict = d.strict_next;
+  d.strict_next = ~0u;
   HIPCHK(hipEventRecord(d.ev0, s));
   // On chip where the launch is the library's choice; options that shape it
   // keep the kernels they were written for.
@@ -1829,7 +1839,7 @@ int run_batch(DevState &d, int nsys, const std::vector<int> &row_off, const std:
     const int per = o.batch_launch_systems > 0 ? o.batch_launch_systems : nsys;
     for (int lo = 0; lo < nsys; lo += std::min(per, nsys - lo))
       if ((rc = run_resident_batch<F>(d, lo, lo + std::min(per, nsys - lo), row_off, val_off, w, ad, av, ia, ja, x, b, tol,
-                                      maxit, o, host_st, todo, s)))
+                                      maxit, o, strict, host_st, todo, s)))
         return rc;
   } else {
     for (int i = 0; i < nsys; ++i) todo.push_back(i);
@@ -2090,6 +2100,18 @@ int fvc_keep_matrix(int32_t keep) {
   if (rc) return rc;
   std::lock_guard<std::mutex> lk(d->mu);
   d->keep_next = keep != 0;
+  return FVC_OK;
+}
+
+// Not part of the ABI, for the tests of what follows an expired wait: on the
+// current device, the next solve or batch ends each of its on-chip waits from
+// the exchange-th on (1: from the first) after one look.
+int fvc_test_expire(int32_t exchange) {
+  DevState *d = nullptr;
+  const int rc = current_device(&d);
+  if (rc) return rc;
+  std::lock_guard<std::mutex> lk(d->mu);
+  d->strict_next = exchange > 0 ? (unsigned)exchange : ~0u;
   return FVC_OK;
 }
 
