@@ -60,6 +60,8 @@ struct ResPrepArgs {
   int nparts;
   int rmax, bmax, hmax;    // rows per block, blocks and halo entries at most
   int one_step;            // prefer plans of at most kResOneStep blocks
+  const double *x;         // copied to keep (neq), the start vector of a solve that
+  double *keep;            // must be done again; null: not asked for
 };
 
 // The columns of row i that count: off-diagonal entries other than
@@ -90,6 +92,8 @@ __device__ __forceinline__ void resident_prep(const ResPrepArgs &a) {
   const int first = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   for (size_t k = first; k < (size_t)4 * n; k += (size_t)step) a.rows[k] = 0ull;
   for (int k = first; k < a.nparts; k += step) a.part[k] = 0ull;
+  if (a.keep)
+    for (long i = first; i < n; i += step) a.keep[i] = a.x[i];
   int h = 0;
   for (long i = first; i < n; i += step) {
     res_columns<F>(a.A, (int)i, [&](int j) { h = max(h, abs(j - (int)i)); });

@@ -407,11 +407,15 @@ const void *resident_fn(int rpt) {
 
 // Solves on chip if the system fits; *done says whether it did (else the
 // caller solves it one kernel per phase).  part: kResPartWords words; rows:
-// at least 4 neq words (vectors that the caller does not need yet).  GMRES:
-// gv, the basis columns, ld apart.
+// at least 4 neq words (vectors that the caller does not need yet).  keep: neq
+// doubles for x as given, which is put back if a wait expired, since blocks
+// write x when their own last exchange is over (null: x is not a start vector,
+// or the caller keeps it).  The copy is the plan's kernel's, which goes through
+// memory anyway.  GMRES: gv, the basis columns, ld apart.
 template <int F>
 int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned *ctr, res_word *part, res_word *rows,
-                 fvc_stats *stats, hipStream_t s, bool *done, double *gv = nullptr, size_t ld = 0) {
+                 fvc_stats *stats, hipStream_t s, bool *done, double *keep = nullptr, double *gv = nullptr,
+                 size_t ld = 0) {
   *done = false;
   if constexpr (!resident_format(F)) {
     return FVC_OK;
@@ -448,7 +452,7 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
       a.gang = 1;
       hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, (int)kCtrWords, st, 1);
       ResPrepArgs pa{in.A, plan, part, rows, kResPartWords, kResThreads * sh.rpt, sh.blocks, hmax,
-                     kind != kResBicgstab};
+                     kind != kResBicgstab, in.x, keep};
       hipLaunchKernelGGL(resident_prep_kernel<F>, dim3(std::min((neq + 255) / 256, 4 * d.cus)), dim3(256), 0, s, pa);
     }
     HIPCHK(hipGetLastError());
@@ -458,7 +462,9 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
     const int rc = read_state(d, st, s);
     if (rc) return rc;
     const KState &hs = *d.host_st;
-    if (hs.pad6 != kResSolved || hs.next != 0) return FVC_OK;   // does not fit, or a wait expired
+    const bool expired = sh.blocks > 1 && (hs.next != 0 || (hs.pad6 != kResSolved && hs.pad6 != kResDeclined));
+    if (expired && keep) HIPCHK(hipMemcpyAsync(in.x, keep, (size_t)neq * sizeof(double), hipMemcpyDeviceToDevice, s));
+    if (expired || hs.pad6 != kResSolved) return FVC_OK;
     *done = true;
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, d.ev0, d.ev1));
@@ -595,7 +601,7 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
     bool done = false;
     const int kind = res_gmres ? kResGmres : in.code == FVC_PCG ? kResPcg : kResBicgstab;
     rc = run_resident<F>(d, in, kind, st, ctr, part, res_gmres ? grows : reinterpret_cast<res_word *>(vec[0]), stats, s,
-                         &done, vec[0], nvec > 1 ? (size_t)(vec[1] - vec[0]) : n);
+                         &done, in.x0_zero ? nullptr : xbackup, vec[0], nvec > 1 ? (size_t)(vec[1] - vec[0]) : n);
     if (rc || done) return rc;
   }
   const bool may_fall_back = persistent && in.engine == FVC_ENGINE_AUTO;
@@ -1739,8 +1745,10 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
                  at_ptr = put(plan.ptr.data(), plan.ptr.size()), at_list = put(plan.list.data(), plan.list.size());
     const size_t n = (size_t)row_off[hi];
     const size_t nclear = (size_t)nsys * (sizeof(ResPlan) / sizeof(unsigned)) + 1;
-    // mixed precision works on x in place: x as given is kept for what it declines
-    const size_t nkeep = mixed && o.x0_rule == FVC_X0_GIVEN ? n - (size_t)row_off[lo] : 0;
+    // x as given is kept for the systems that are solved again: mixed precision
+    // works on x in place, and an expired wait sends all of them, those whose x
+    // is written too
+    const size_t nkeep = o.x0_rule == FVC_X0_GIVEN ? n - (size_t)row_off[lo] : 0;
     const size_t bytes = align_up(up.size() * sizeof(int)) + align_up(nsys * sizeof(KState)) +
                          align_up(nclear * sizeof(unsigned)) + align_up(npart * sizeof(res_word)) +
                          align_up(4 * n * sizeof(res_word)) + align_up(nkeep * sizeof(double)) + 4096;

@@ -41,3 +41,53 @@ def test_batch_leaves_whole(fvc, uneven, precision):
             assert sts[i]["status"] == ss[i]["status"] == 0, (i, sts[i])
             assert np.linalg.norm(s.b - mats[s.neq] @ xi) <= 1.01e-10 * np.linalg.norm(s.b), i
             assert np.linalg.norm(xi - yi) <= 1e-8 * np.linalg.norm(yi), i
+
+
+@pytest.mark.parametrize("code", [1, 2], ids=["pcg", "bicgstab"])
+@pytest.mark.parametrize("nx,ny", [(70, 61), (231, 230), (499, 498)])
+def test_solve_restarts_from_x0(fvc, nx, ny, code):
+    """The other engine starts from the caller's x0 also where some blocks had
+    written their x already (a wait of the last exchange): the same bits as that
+    engine alone.  Where every word was there at the first look the solve ends on
+    chip: the order of the sums only, over three iterations (1e-12)."""
+    m = P.quad_mesh(nx, ny, jitter=0.1, seed=nx)
+    s = P.pressure_system(m, k=P.lognormal_k(3, m.neq), pin="penalty") if code == 1 else \
+        P.advdiff_system(m, dt=0.005, under_relax=0.8)
+    f = P.to_ell(s)
+    x0 = np.random.default_rng(nx).normal(size=m.neq)
+    kw = dict(x0=x0, tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_GIVEN, maxit=3)
+    xk, sk = fvc.solve(f, code, engine=fvc.ENGINE_KERNELS, **kw)
+    fell = 0
+    for exchange in range(1, 12):
+        print(f"{nx}x{ny} code={code} expires from exchange {exchange} on", flush=True)
+        for _ in range(4):
+            _expire(exchange)
+            xa, sa = fvc.solve(f, code, **kw)
+            assert (sa["status"], sa["iterations"]) == (sk["status"], sk["iterations"]) == (1, 3)
+            if sa["engine"] == fvc.ENGINE_KERNELS:
+                fell += 1
+                assert np.array_equal(xa, xk)
+            else:
+                assert np.linalg.norm(xa - xk) <= 1e-12 * np.linalg.norm(xk)
+    assert fell > 0
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+def test_batch_restarts_from_x0(fvc, uneven, precision):
+    """As above: an expired wait sends every system of the batch to the other
+    kernels, those whose x was written too.  After three iterations the order of
+    the sums only (FP64 1e-12; FP32 vectors may round the other way, 1e-6)."""
+    batch = fvc.concat_ell([P.to_ell(s) for s in uneven])
+    ro = batch["row_offsets"]
+    x0 = np.random.default_rng(1).normal(size=int(ro[-1]))
+    x0[batch["ad"] > 1e50] = 0.0   # the pinned rows hold it
+    kw = dict(x0=x0, tol=1e-10, stop_rule=fvc.STOP_RELRES, x0_rule=fvc.X0_GIVEN, precision=precision, maxit=3)
+    xs, ss = fvc.solve_batch(batch, block_size=512, **kw)
+    for exchange in range(1, 10):
+        print(f"batch expires from exchange {exchange} on, precision {precision}", flush=True)
+        _expire(exchange)
+        x, sts = fvc.solve_batch(batch, **kw)
+        for i in range(len(uneven)):
+            xi, yi = x[ro[i]:ro[i + 1]], xs[ro[i]:ro[i + 1]]
+            assert (sts[i]["status"], sts[i]["iterations"]) == (ss[i]["status"], ss[i]["iterations"]) == (1, 3), i
+            assert np.linalg.norm(xi - yi) <= (1e-12 if precision == 0 else 1e-6) * np.linalg.norm(yi), i
