@@ -276,6 +276,7 @@ int choose_blocks(int neq, int cus, int occ_blocks, int requested) {
 struct SolveIn {
   int code, F;
   Mat A;
+  long nval;              // stored off-diagonal values (CSR: all values)
   const double *m;
   double *x;
   const double *b;
@@ -405,7 +406,23 @@ const void *resident_fn(int rpt) {
   return nullptr;
 }
 
-// Solves on chip if the system fits; *done says whether it did (else the
+// Is the on-chip solver tried?  Decided before any workspace is reserved for
+// it.  It is where the launch is the library's choice (options that shape it
+// keep the engines they were written for), the format is one whose rows fit the
+// registers (CSRD: if no more than four off-diagonals a row are stored on
+// average) and the rows fit the chip.  Whether the columns fit a plan, the
+// device decides.
+template <int F>
+bool resident_wanted(const DevState &d, const SolveIn &in, int kind) {
+  if (!resident_format(F) || in.engine != FVC_ENGINE_AUTO || in.bs != 0 || in.G_req != 0 || in.barrier != 0 ||
+      in.row_order != 0)
+    return false;
+  if (kind != kResMixedPcg && (in.recurrence != FVC_REC_FUSED || in.lanex)) return false;
+  if (F == F_CSRD && in.nval > 4L * in.A.neq) return false;
+  return resident_shape(in.A.neq, d.cus, kind).rpt != 0;
+}
+
+// Solves on chip (resident_wanted) if the columns fit; *done says whether they did (else the
 // caller solves it one kernel per phase).  part: kResPartWords words; rows:
 // at least 4 neq words (vectors that the caller does not need yet).  keep: neq
 // doubles for x as given, which is put back if a wait expired, since blocks
@@ -422,7 +439,6 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
   } else {
     const int neq = in.A.neq;
     const ResShape sh = resident_shape(neq, d.cus, kind);
-    if (sh.rpt == 0) return FVC_OK;
     ResArgs a{};
     a.A = in.A; a.st = st; a.m = in.m; a.x = in.x; a.b = in.b;
     a.tol = in.tol; a.maxit = in.maxit; a.x0_zero = in.x0_zero; a.stop_rule = in.stop_rule;
@@ -569,12 +585,14 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
                  align_up(2 * sizeof(KState)) + align_up(2 * kMaxK * (size_t)G * sizeof(double)) +
                  align_up(lag_small * sizeof(double)) + align_up(lag_parts * sizeof(double)) + 4096;
   // the on-chip solver's words for partial sums, where the fixed workspace
-  // has room for them (its limit stays that of the engines below)
-  size_t res_part = align_up(kResPartWords * sizeof(res_word));
-  // (GMRES with modified Gram-Schmidt: also the words of the rows, since the
-  // basis takes the vectors)
+  // has room for them (its limit stays that of the engines below); GMRES with
+  // modified Gram-Schmidt: also the words of the rows, since the basis takes
+  // the vectors
   const bool res_gmres = in.code == FVC_GMRES && !cgs && !lag && k <= kResGmresK;
-  size_t res_rows = res_gmres ? align_up(4 * n * sizeof(res_word)) : 0;
+  const int kind = res_gmres ? kResGmres : in.code == FVC_PCG ? kResPcg : kResBicgstab;
+  const bool on_chip = (res_gmres || in.code != FVC_GMRES) && resident_wanted<F>(d, in, kind);
+  size_t res_part = on_chip ? align_up(kResPartWords * sizeof(res_word)) : 0;
+  size_t res_rows = on_chip && res_gmres ? align_up(4 * n * sizeof(res_word)) : 0;
   if (d.noalloc && bytes + res_part + res_rows > kScratchBytes) res_part = res_rows = 0;
   bytes += res_part + res_rows;
   char *ws = nullptr;
@@ -594,12 +612,8 @@ int run_solve(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
   double *lagsmall = cv.take<double>(lag_small);
   double *lagpart = cv.take<double>(lag_parts);
   if (!cv.fits()) return carve_overflow(cv);
-  // On chip where the launch is the library's choice; options that shape it
-  // keep the engines they were written for.
-  if (in.engine == FVC_ENGINE_AUTO && (res_gmres || in.code != FVC_GMRES) && fused && in.bs == 0 && in.G_req == 0 &&
-      in.barrier == 0 && in.row_order == 0 && !in.lanex && res_part) {
+  if (res_part) {
     bool done = false;
-    const int kind = res_gmres ? kResGmres : in.code == FVC_PCG ? kResPcg : kResBicgstab;
     rc = run_resident<F>(d, in, kind, st, ctr, part, res_gmres ? grows : reinterpret_cast<res_word *>(vec[0]), stats, s,
                          &done, in.x0_zero ? nullptr : xbackup, vec[0], nvec > 1 ? (size_t)(vec[1] - vec[0]) : n);
     if (rc || done) return rc;
@@ -930,7 +944,9 @@ int run_mixed(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
                    align_up(2 * sizeof(KState)) + align_up(2 * kMaxK * (size_t)G * sizeof(double)) +
                    align_up(std::max<size_t>(n16, 1) * sizeof(short)) + 4096;
     // as in run_solve: the on-chip solver's words, and x as it was given
-    size_t res_part = align_up(kResPartWords * sizeof(res_word)), res_x = in.x0_zero ? 0 : align_up(n * sizeof(double));
+    const bool on_chip = resident_wanted<F>(d, in, kResMixedPcg);
+    size_t res_part = on_chip ? align_up(kResPartWords * sizeof(res_word)) : 0;
+    size_t res_x = on_chip && !in.x0_zero ? align_up(n * sizeof(double)) : 0;
     if (d.noalloc && bytes + res_part + res_x > kScratchBytes) res_part = res_x = 0;
     bytes += res_part + res_x;
     char *ws = nullptr;
@@ -952,9 +968,9 @@ int run_mixed(DevState &d, const SolveIn &in, fvc_stats *stats, hipStream_t s) {
     a.ps = align_up(n * sizeof(float4)) / sizeof(float4);
     a.rec = cv.take<float4>(2 * a.ps);
     if (!cv.fits()) return carve_overflow(cv);
-    // On chip where the launch is the library's choice (run_solve).  It works
-    // on x in place: x as given is kept for the case that it declines.
-    if (in.engine == FVC_ENGINE_AUTO && in.bs == 0 && in.G_req == 0 && in.barrier == 0 && in.row_order == 0 && res_part) {
+    // The on-chip solver works on x in place: x as given is kept for the case
+    // that it declines.
+    if (res_part) {
       bool done = false;
       if (!in.x0_zero)
         HIPCHK(hipMemcpyAsync(xgiven, in.x, n * sizeof(double), hipMemcpyDeviceToDevice, s));
@@ -1558,6 +1574,7 @@ int solve_impl(int code, int matriz, int unsym, int neq, int nad, const double *
   in.code = code;
   in.F = md.F;
   in.A = md.m;
+  in.nval = md.nval;
   in.m = m;
   in.x = dx;
   in.b = db;
@@ -1743,15 +1760,15 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     }
     const size_t at_part = put(part_off.data(), part_off.size()), at_multi = put(multi.data(), multi.size()),
                  at_ptr = put(plan.ptr.data(), plan.ptr.size()), at_list = put(plan.list.data(), plan.list.size());
-    const size_t n = (size_t)row_off[hi];
+    const size_t nrows = multi.empty() ? 0 : 4 * (size_t)row_off[hi];   // words of the systems of several blocks
     const size_t nclear = (size_t)nsys * (sizeof(ResPlan) / sizeof(unsigned)) + 1;
     // x as given is kept for the systems that are solved again: mixed precision
     // works on x in place, and an expired wait sends all of them, those whose x
     // is written too
-    const size_t nkeep = o.x0_rule == FVC_X0_GIVEN ? n - (size_t)row_off[lo] : 0;
+    const size_t nkeep = o.x0_rule == FVC_X0_GIVEN ? (size_t)(row_off[hi] - row_off[lo]) : 0;
     const size_t bytes = align_up(up.size() * sizeof(int)) + align_up(nsys * sizeof(KState)) +
                          align_up(nclear * sizeof(unsigned)) + align_up(npart * sizeof(res_word)) +
-                         align_up(4 * n * sizeof(res_word)) + align_up(nkeep * sizeof(double)) + 4096;
+                         align_up(nrows * sizeof(res_word)) + align_up(nkeep * sizeof(double)) + 4096;
     int rc = ensure_arena(d, bytes);
     if (rc) return rc;
     Carve cv{d.arena, bytes};
@@ -1759,7 +1776,7 @@ int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_
     KState *st = cv.take<KState>(nsys);
     unsigned *clear = cv.take<unsigned>(nclear);
     res_word *part = cv.take<res_word>(npart);
-    res_word *rows = cv.take<res_word>(4 * n);
+    res_word *rows = cv.take<res_word>(nrows);
     double *xkeep = cv.take<double>(nkeep);
     if (!cv.fits()) return carve_overflow(cv);
     if (nkeep) HIPCHK(hipMemcpyAsync(xkeep, x + row_off[lo], nkeep * sizeof(double), hipMemcpyDeviceToDevice, s));
