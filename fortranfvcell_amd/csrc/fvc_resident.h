@@ -43,7 +43,13 @@
 
 namespace fvc {
 
-constexpr unsigned kResSpin = 1u << 20;   // polls of a bounded wait (about two seconds)
+// Polls of a bounded wait: about 0.4 s.  The first exchange of a solve is also
+// where its blocks wait until all of them have a CU, and some may not get one
+// for as long as another stream's kernel runs; the engine that streams needs no
+// such thing, so that wait is given up after about 3 ms, what that engine takes
+// for BiCGSTAB on 1,048,576 rows.  Beside a kernel of one wave that runs 0.8 s, such a
+// solve takes 6.4 ms (394 with the full wait), 3.2 if it streams at once.
+constexpr unsigned kResSpin = 1u << 20, kResFirst = 1u << 13;
 
 typedef unsigned long long res_word;
 
@@ -306,7 +312,7 @@ struct ResArgs {
   res_word *part;          // two buffers of part_half words
   unsigned *err;           // set when a wait expired; the waits of others end too
   int part_half;
-  int gang;                // how many times longer the first exchange may take
+  unsigned first;          // polls that the first exchange may take
   unsigned strict;         // from this exchange on a wait ends after one look (tests)
   double tol;
   double delta;            // mixed: residual drop that triggers an FP64 update
@@ -393,8 +399,7 @@ struct ResNet {
     static_assert(K <= kResSums, "a lane adds at most two of the groups' sums");
     constexpr int E = K > 4 ? 2 : 1;   // the fifth value goes with the first 16 lanes
     res_word *part = a.part + (size_t)(ep & 1) * (size_t)a.part_half;
-    // a block may come to its first exchange long before the others
-    const unsigned limit = ep >= a.strict ? 0u : ep == 1 ? kResSpin * (unsigned)a.gang : kResSpin;
+    const unsigned limit = ep >= a.strict ? 0u : ep == 1 ? a.first : kResSpin;
     // Up to 64 blocks a lane per block adds all sums.  Beyond, so many
     // readers of so many words hold each other up (256 blocks: 7 us), and
     // the sums go in two steps: the first block of 16 adds its group's and
@@ -1321,7 +1326,8 @@ __device__ __forceinline__ T res_uniform_ints(const T *p) {
   return v;
 }
 
-constexpr int kResGang = 32;   // a team's first exchange may wait for its members' earlier systems
+// A team's first exchange waits for its members' earlier systems (up to 12 s).
+constexpr unsigned kResFirstTeam = 32 * kResSpin;
 
 template <int F>
 __device__ __forceinline__ void resident_batch_mat(const ResBatchArgs &B, const SysDesc &D, Mat &A) {
@@ -1382,7 +1388,7 @@ __global__ __launch_bounds__(kResThreads) void resident_batch_kernel(ResBatchArg
     a.part = B.part + res_uniform(B.part_off + sys);
     a.part_half = res_part_half(D.g_count);
     a.err = B.err;
-    a.gang = kResGang;
+    a.first = kResFirstTeam;
     a.strict = B.strict;
     a.tol = B.tol;
     a.maxit = B.maxit;

@@ -465,7 +465,7 @@ int run_resident(DevState &d, const SolveIn &in, int kind, KState *st, unsigned 
       a.part = part;
       a.part_half = kResPartWords / 2;
       a.err = reinterpret_cast<unsigned *>(&st->next);
-      a.gang = 1;
+      a.first = kResFirst;
       hipLaunchKernelGGL(reset_kernel, dim3(1), dim3(256), 0, s, ctr, (int)kCtrWords, st, 1);
       ResPrepArgs pa{in.A, plan, part, rows, kResPartWords, kResThreads * sh.rpt, sh.blocks, hmax,
                      kind != kResBicgstab, in.x, keep};

@@ -2,12 +2,18 @@
 launch ends, and the other engines solve the system from what the caller gave.
 The expiry is forced by the host, which has every wait from a given exchange on
 end after one look (fvc_test_expire); every block still leaves by itself."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from fortranfvcell_amd import _lib, problems as P
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _expire(exchange):
@@ -91,3 +97,50 @@ def test_batch_restarts_from_x0(fvc, uneven, precision):
             xi, yi = x[ro[i]:ro[i + 1]], xs[ro[i]:ro[i + 1]]
             assert (sts[i]["status"], sts[i]["iterations"]) == (ss[i]["status"], ss[i]["iterations"]) == (1, 3), i
             assert np.linalg.norm(xi - yi) <= (1e-12 if precision == 0 else 1e-6) * np.linalg.norm(yi), i
+
+
+
+# (a process of its own: torch's HIP runtime has to be loaded first)
+BESIDE = r"""
+import sys, time
+import torch
+import numpy as np
+import fortranfvcell_amd as F
+from fortranfvcell_amd import problems as P
+code = int(sys.argv[1])
+F.init(0)
+s = P.config_advdiff(1024)
+ds = F.DeviceSystem(P.to_ell(s))
+kw = dict(tol=1e-10, stop_rule=F.STOP_RELRES, x0_rule=F.X0_ZERO)
+assert ds.solve(code, **kw)["engine"] == F.ENGINE_PERSISTENT
+torch.cuda._sleep(1000)
+torch.cuda.synchronize()
+t = time.perf_counter()
+torch.cuda._sleep(10_000_000)
+torch.cuda.synchronize()
+cycles = int(0.8 * 1e7 / (time.perf_counter() - t))
+side = torch.cuda.Stream()
+with torch.cuda.stream(side):
+    torch.cuda._sleep(cycles)
+time.sleep(0.01)
+t = time.perf_counter()
+st = ds.solve(code, **kw)
+t = time.perf_counter() - t
+asleep = not side.query()
+side.synchronize()
+r = np.linalg.norm(s.b - P.scipy_csr(s) @ ds.x.get()) / np.linalg.norm(s.b)
+print("result", t, int(asleep), st["status"], st["engine"], r)
+"""
+
+
+@pytest.mark.parametrize("code", [2, 3], ids=["bicgstab", "gmres"])
+def test_solve_beside_a_long_kernel(code):
+    """A wave of another stream, asleep for 0.8 s, keeps one of the 256 blocks off
+    the chip (blocks of eight rows a thread take all of a CU's registers): the
+    solve does not wait for it but goes to an engine that needs no CU to itself,
+    which takes 3 ms (BiCGSTAB) and 25 ms (GMRES) alone."""
+    r = subprocess.run([sys.executable, "-c", BESIDE, str(code)], cwd=ROOT, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    t, asleep, status, engine, relres = (float(v) for v in r.stdout.split("result")[1].split())
+    print(f"code {code}: {t * 1e3:.1f} ms, engine {engine:.0f}, other stream still busy {asleep:.0f}", flush=True)
+    assert asleep == 1 and t < 0.2 and status == 0 and relres <= 1.01e-10
