@@ -77,9 +77,13 @@ extern "C" {
                                     FVC_ORTH_MGS, k <= 32) on ELLPACK of width 3 or 4 or
                                     CSRD rows of at most four off-diagonals, with none of
                                     the options that shape a launch set: on chip in one
-                                    launch where the system fits (up to 1,048,576 rows on
-                                    256 CUs; stats.engine then says PERSISTENT).  Else
-                                    KERNELS, GMRES PERSISTENT                            */
+                                    launch where the system fits (stats.engine then says
+                                    PERSISTENT).  On 256 CUs that is up to 1,020,000 rows
+                                    of a mesh numbered row by row, 1,048,576 where it
+                                    tiles exactly; of another numbering, as long as the
+                                    bandwidth fits (squares in reverse Cuthill-McKee
+                                    order: BiCGSTAB up to 498,000 rows, PCG 783,000).
+                                    Else KERNELS, GMRES PERSISTENT                       */
 #define FVC_ENGINE_KERNELS 1     /* one kernel per phase; fused recurrences sum the block
                                     partials at the next launch, the others in the last
                                     block of the launch                                 */
@@ -225,7 +229,9 @@ int fvc_solve_dev(int32_t code, int32_t matriz, int32_t unsym, int32_t neq, int3
 /* fvc_solve_dev with no allocation.  No counterpart in the reference: for
  * callers that cannot allocate device memory (code under graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  Same arguments, stopping
- * rules, results and status codes as fvc_solve_dev, for ELLPACK storage
+ * rules, results and status codes as fvc_solve_dev (to the bit, unless the
+ * workspace holds the streaming engine but not the on-chip solver's words
+ * beside it: 80 KB, GMRES 32 bytes a row more), for ELLPACK storage
  * (matriz 4; other formats return FVC_UNSUPPORTED).  The solver's scratch
  * (vectors, partial sums, counters, state) comes from one fixed workspace of
  * FVC_NOALLOC_WORKSPACE_BYTES per device, which the library holds until the
