@@ -144,8 +144,8 @@ FVC_HD bool res_tiles(int n, int S, int hx, int ntx, int rmax, int bmax, int hma
 }
 
 // Which of two plans is taken: where one_step is asked for, the one of at most
-// kResOneStep blocks, then the one of fewer halo entries (253 x 257 rows: 2.6 us per PCG iteration in 64
-// strips of 514 halo entries, 3.1 in 72 tiles of 134).
+// kResOneStep blocks, then the one of fewer halo entries (253 x 257 rows: 2.6 us
+// per PCG iteration in 64 strips of 514 halo entries, 3.1 in 72 tiles of 134).
 constexpr int kResOneStep = 64;   // blocks up to which the sums are added in one step
 FVC_HD int res_cost(const ResPlan &p, bool one_step) {
   return (one_step && p.nb > kResOneStep ? 2 * kResMaxHalo : 0) + p.nh;
@@ -212,10 +212,12 @@ constexpr int res_max_halo(int code, int rpt) {
 //     four: 81,200 rows 2.8 against 3.1 at two, 127,800 rows 2.9 against 3.1
 //     (BiCGSTAB 6.1 against 6.0, 6.5 against 6.1).  More blocks than 64 are
 //     launched for plans that need them; res_cost prefers the others.
-//     BiCGSTAB, which gains less, stays with the plan of least halo from 53,248
-//     rows on: its count of iterations follows the order of the sums (65,536
-//     rows of a steady transport system: 5,143 iterations with it, 5,445 on 64
-//     blocks, the reference's 5,096);
+//     BiCGSTAB stays with the plan of least halo from 53,248 rows on, at a price
+//     (59,713 rows 0.33 ms a solve against 0.29 on 64 blocks).  Its count of
+//     iterations moves with the order of the sums, and on the one system where
+//     it is held to the reference's, 65,536 rows of steady transport, 5,096
+//     iterations within 3 %, it is 5,143 with this plan and 5,445 on 64 blocks.
+//     One system does not show that either plan needs fewer in general;
 //   * beyond, the fewest rows per thread: 160,860 rows 3.1 / 6.1 at 2, 3.5 / 7.0
 //     at 4, 3.9 / 8.5 at 8 -- as long as a twentieth of the rows stays free for
 //     tiles that the mesh's edge cuts (524,176 rows in strips at 4 took half as

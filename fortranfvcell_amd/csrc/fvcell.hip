@@ -386,11 +386,11 @@ int drive_batches(DevState &d, hipStream_t s, int maxit, Iter &&iteration, State
 
 // The on-chip solvers (fvc_resident.h).  Measured on MI355X against one
 // kernel per phase, whole solves to a true residual of 1e-10: PCG 4,096 rows
-// 3.93 -> 1.27 ms, 429,713 rows 77.8 -> 22.8; BiCGSTAB 12,707 rows 0.92 ->
-// 0.37, 1,048,576 rows 2.61 -> 0.77.  Mixed PCG, us per FP32 iteration: 5,120
-// rows 8.2 -> 3.3, 160,860 12.2 -> 5.0, 1,048,576 18.1 -> 7.0.  GMRES(30) with
-// modified Gram-Schmidt, whole solves: 4,096 rows 9.7 -> 2.2 ms, 160,860 17.9 ->
-// 4.7, 1,048,576 24.8 -> 6.8.
+// 3.93 -> 0.99 ms, 429,713 rows 77.8 -> 16.3; BiCGSTAB 12,707 rows 0.92 ->
+// 0.24, 1,048,576 rows 2.61 -> 0.70.  Mixed PCG, us per FP32 iteration (a solve's time over them): 5,120
+// rows 8.2 -> 2.7, 160,860 12.2 -> 3.5, 1,048,576 18.1 -> 5.2.  GMRES(30) with
+// modified Gram-Schmidt, whole solves: 4,096 rows 9.7 -> 2.1 ms, 160,860 17.9 ->
+// 3.8, 1,048,576 24.8 -> 5.6.
 constexpr bool resident_format(int F) { return F == F_ELL4 || F == F_ELL3 || F == F_CSRD; }
 
 template <int F, int Code>
@@ -1701,8 +1701,9 @@ int dot_impl(const double *a, const double *b, int n, double *result, bool on_de
 // Systems lo .. hi - 1 of a batch on chip (fvc_resident.h): solves what
 // fits, in one launch, and adds to `todo` the systems it did not solve.
 // Measured on MI355X against the streaming kernels below: 48 systems of side
-// 32 .. 160 40.4 -> 4.6 ms; 256 systems of side 32 .. 512 (10.2M rows) 835 ms at
-// the tuned launches -> 115.
+// 32 .. 160 40.4 -> 3.5 ms; 256 systems of side 32 .. 512 (10.2M rows) 835 ms at
+// the tuned launches -> 118; 10,000 systems of side 6 .. 12 39 -> 21 (half of it
+// the host's plan).
 template <int F>
 int run_resident_batch(DevState &d, int lo, int hi, const std::vector<int> &row_off, const std::vector<int> &val_off, int w,
                        const double *ad, const double *av, const int *ia, const int *ja, double *x, const double *b,
