@@ -6,12 +6,11 @@
 // (256 CUs hold 128 MB of registers; a row of a 4-neighbour system with its
 // six vectors takes about 100 bytes), so that an iteration reads neither the
 // matrix nor a vector from memory.  (At eight rows a thread the 256 registers of
-// a lane do not hold everything: 16 to 204 bytes of scratch a lane, 44 to 164 in
-// batches, width 3 least.  With the exchanges' words BiCGSTAB moves 15 MB an
-// iteration past L2 at 1,048,576 rows, streamed 243; PCG on 160,000 rows, two a
-// thread and no scratch, 1.8 MB, streamed 22.)
-// What an iteration waits for is the exchange between blocks, once per
-// grid reduction:
+// a lane do not hold everything: up to 204 bytes of scratch a lane, BiCGSTAB at
+// width 4.  With the exchanges' words it moves 15 MB an iteration past L2 at
+// 1,048,576 rows, streamed 243; PCG on 160,000 rows, two a thread and no scratch,
+// 1.8 MB, streamed 22.)  What an iteration waits for is the exchange between
+// blocks, once per grid reduction:
 //   * the SpMV reads its operand from an LDS window of the block's own rows
 //     and of the halo rows its columns reach.  A halo row's operand is not
 //     sent: its r, s, p ... follow the same recurrences as the owner's, on

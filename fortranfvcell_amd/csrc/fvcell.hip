@@ -387,10 +387,10 @@ int drive_batches(DevState &d, hipStream_t s, int maxit, Iter &&iteration, State
 // The on-chip solvers (fvc_resident.h).  Measured on MI355X against one
 // kernel per phase, whole solves to a true residual of 1e-10: PCG 4,096 rows
 // 3.93 -> 0.99 ms, 429,713 rows 77.8 -> 16.3; BiCGSTAB 12,707 rows 0.92 ->
-// 0.24, 1,048,576 rows 2.61 -> 0.70.  Mixed PCG, us per FP32 iteration (a solve's time over them): 5,120
-// rows 8.2 -> 2.7, 160,860 12.2 -> 3.5, 1,048,576 18.1 -> 5.2.  GMRES(30) with
-// modified Gram-Schmidt, whole solves: 4,096 rows 9.7 -> 2.1 ms, 160,860 17.9 ->
-// 3.8, 1,048,576 24.8 -> 5.6.
+// 0.24, 1,048,576 rows 2.61 -> 0.70.  Mixed PCG, us per FP32 iteration (a solve's
+// time over them): 5,120 rows 8.2 -> 2.7, 160,860 12.2 -> 3.5, 1,048,576 18.1 ->
+// 5.2.  GMRES(30) with modified Gram-Schmidt, whole solves: 4,096 rows 9.7 -> 2.1
+// ms, 160,860 17.9 -> 3.8, 1,048,576 24.8 -> 5.6.
 constexpr bool resident_format(int F) { return F == F_ELL4 || F == F_ELL3 || F == F_CSRD; }
 
 template <int F, int Code>
